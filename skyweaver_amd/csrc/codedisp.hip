@@ -433,6 +433,47 @@ __device__ __forceinline__ void load_column(const CdParams& p, int f, int col, l
     }
 }
 
+// The raw samples (re | im << 8) of one unit of the register kernels: value
+// i = c R1 + n1 is sample b + 512 n1 + t of column col0 + c, b the segment's
+// first sample relative to the gulp start (negative: history).  The uniform
+// tests are made once for the unit's columns, so its 32 loads are in flight
+// together, and nothing here uses a loaded value, so they stay in flight
+// until the caller unpacks them.  (Tested and merged two to a register per
+// column, each column's loads were waited for where they were issued: 16
+// round trips per unit at N = 1024, none behind the transforms; 256 channels
+// x 128 columns x 65536 samples took 8.47 ms, now 4.88; N = 16384 at 64
+// channels 1.71, now 1.57.)
+template <int R1>
+__device__ __forceinline__ void load_unit(const CdParams& p, int f, int col0, long b, int t, uint32_t (&raw)[32])
+{
+    constexpr int C = 32 / R1;
+    const size_t cc = (size_t)f * p.PA + col0;
+    const uint16_t* cur = reinterpret_cast<const uint16_t*>(p.cur) + cc * p.T;
+    if(b >= 0 && b + 512 * R1 <= p.T) {  // inside this gulp
+#pragma unroll
+        for(int c = 0; c < C; ++c) {
+            const uint16_t* x = cur + (size_t)c * p.T + b;
+#pragma unroll
+            for(int n1 = 0; n1 < R1; ++n1) raw[c * R1 + n1] = x[512 * n1 + t];
+        }
+    } else {
+        // sample tau < 0: the previous gulp's tail or the history buffer.
+        // tau < T always: a gulp's segments are those whose input ends
+        // inside it (sw_codedisp_run), so no load here needs a test.
+        const int ll = p.prev ? p.T : p.Oh;
+        const uint16_t* lo = reinterpret_cast<const uint16_t*>(p.prev ? p.prev : p.hist) + cc * ll + ll;
+        const int b32 = (int)b;
+#pragma unroll
+        for(int c = 0; c < C; ++c)
+#pragma unroll
+            for(int n1 = 0; n1 < R1; ++n1) {
+                const int tau = b32 + 512 * n1 + t;
+                const uint16_t* x = tau < 0 ? lo + (size_t)c * ll : cur + (size_t)c * p.T;
+                raw[c * R1 + n1] = x[tau];
+            }
+    }
+}
+
 // Quantise y / N and write the kept positions [O/2, N - O/2) of a segment
 // into the output ring (ring index j0 + position, wrapped once).
 __device__ __forceinline__ void store_kept(const CdParams& p, int d, size_t colbase, int j0, int pos, float2 y)
@@ -525,13 +566,11 @@ __global__ void __launch_bounds__(512) codedisp_reg_kernel(CdParams p, int d, in
     const int t = threadIdx.x;
     load_step2_tables<R1>(t1k, p.tw, t);
     const int ngrp = p.PA / C;
-    uint32_t nxt[16];  // two raw samples per register: value i = c R1 + n1
+    uint32_t nxt[32];  // the next unit's raw samples
     auto fetch = [&](int u) {
         const int cg = u % ngrp, fs = u / ngrp;
         const int f = fs / p.nseg, s = fs % p.nseg;
-        const long b = p.in0 + (long)s * p.hop;
-#pragma unroll
-        for(int c = 0; c < C; ++c) load_column<R1 / 2>(p, f, cg * C + c, b, t, nxt + c * (R1 / 2));
+        load_unit<R1>(p, f, cg * C, p.in0 + (long)s * p.hop, t, nxt);
     };
     if(blockIdx.x < nunits) fetch(blockIdx.x);
     __syncthreads();  // twiddle tables
@@ -542,10 +581,7 @@ __global__ void __launch_bounds__(512) codedisp_reg_kernel(CdParams p, int d, in
         const int f = fs / p.nseg, s = fs % p.nseg;
         float2 v[32];
 #pragma unroll
-        for(int i = 0; i < 16; ++i) {
-            v[2 * i]     = unpack_c8(nxt[i]);
-            v[2 * i + 1] = unpack_c8(nxt[i] >> 16);
-        }
+        for(int i = 0; i < 32; ++i) v[i] = unpack_c8(nxt[i]);
         if(u + (int)gridDim.x < nunits) fetch(u + gridDim.x);  // in flight during the transforms
         // no barrier: step 1 writes the column t that this thread alone read
         // in the previous unit's step 1'
@@ -562,7 +598,11 @@ __global__ void __launch_bounds__(512) codedisp_reg_kernel(CdParams p, int d, in
 // transform: per unit the spectrum X stays in registers while each DM's
 // chirp, inverse transform and stores run in turn, so a unit costs one
 // forward and p.ndm inverse transforms instead of p.ndm of each.  The next
-// unit's input is fetched during the last DM, once X is no longer needed.
+// unit's input is fetched during the last DM, once X is no longer needed,
+// and packed two to a register at once: one round trip per unit.  (Held one
+// to a register, in flight behind the last inverse or the forward
+// transform, it spilled 50-110 registers: eight DMs of 64 channels took 9.7
+// ms instead of 7.7.)
 template <int R1>
 __global__ void __launch_bounds__(512) codedisp_regm_kernel(CdParams p, int nunits)
 {
@@ -574,15 +614,25 @@ __global__ void __launch_bounds__(512) codedisp_regm_kernel(CdParams p, int nuni
     const int t = threadIdx.x;
     load_step2_tables<R1>(t1k, p.tw, t);
     const int ngrp = p.PA / C;
-    uint32_t nxt[16];  // two raw samples per register: value i = c R1 + n1
-    auto fetch = [&](int u) {
+    auto fetch = [&](int u, uint32_t (&nxt)[32]) {
         const int cg = u % ngrp, fs = u / ngrp;
         const int f = fs / p.nseg, s = fs % p.nseg;
-        const long b = p.in0 + (long)s * p.hop;
-#pragma unroll
-        for(int c = 0; c < C; ++c) load_column<R1 / 2>(p, f, cg * C + c, b, t, nxt + c * (R1 / 2));
+        load_unit<R1>(p, f, cg * C, p.in0 + (long)s * p.hop, t, nxt);
     };
-    if(blockIdx.x < nunits) fetch(blockIdx.x);
+    // the next unit's raw samples, two per register: held beside X and v
+    uint32_t pk[16];
+    auto pack = [&](const uint32_t (&nxt)[32]) {
+#pragma unroll
+        for(int i = 0; i < 16; ++i) {
+            pk[i] = nxt[2 * i] | (nxt[2 * i + 1] << 16);
+            asm volatile("" : "+v"(pk[i]));  // packed here, not where it is used
+        }
+    };
+    if(blockIdx.x < nunits) {
+        uint32_t nxt[32];
+        fetch(blockIdx.x, nxt);
+        pack(nxt);
+    }
     __syncthreads();  // twiddle tables
     // step-1 twiddles W_N^(t k1), the same for every unit; from R1 = 16
     // they are rebuilt at each use (held beside X they would spill)
@@ -594,10 +644,7 @@ __global__ void __launch_bounds__(512) codedisp_regm_kernel(CdParams p, int nuni
         const int f = fs / p.nseg, s = fs % p.nseg;
         float2 X[32];
 #pragma unroll
-        for(int i = 0; i < 16; ++i) {
-            X[2 * i]     = unpack_c8(nxt[i]);
-            X[2 * i + 1] = unpack_c8(nxt[i] >> 16);
-        }
+        for(int i = 0; i < 32; ++i) X[i] = unpack_c8(pk[i / 2] >> (16 * (i & 1)));
         // no barrier: step 1 writes the column t that this thread alone read
         // in the previous DM's step 1'
         float2 hk0[16];  // no chirp prefetch here: each DM has its own chirp
@@ -605,7 +652,11 @@ __global__ void __launch_bounds__(512) codedisp_regm_kernel(CdParams p, int nuni
         const int j0 = (int)(p.y0 + (long)s * p.hop) - p.O / 2;  // ring index of position 0
         for(int d = 0; d < p.ndm; ++d) {
             if(d > 0) __syncthreads();  // the previous DM's step-1' readers of every row
-            if(d == p.ndm - 1 && u + (int)gridDim.x < nunits) fetch(u + gridDim.x);
+            if(d == p.ndm - 1 && u + (int)gridDim.x < nunits) {
+                uint32_t nxt[32];
+                fetch(u + gridDim.x, nxt);
+                pack(nxt);
+            }
             float2 v[32];
             reg_chirp_inverse<R1, HELD>(X, v, lds, tw, t1k, t, p.chirp[d] + (size_t)f * N, wk, hk0);
             store_unit<R1>(p, d, (size_t)f * p.PA + cg * C, j0, t, v);  // v already / N (chirp)
