@@ -348,7 +348,8 @@ int sw_codedisp_run(sw_codedisp* plan, const void* d_ftpa, void* const* d_out,
                     void* stream);
 /* The last run's int8 output of DM dm in the plan's time-major ring:
  * sample t of column (f, p, a) at ring + ((f*2A + p*A + a) * ld + offset + t) * 2
- * (ld a multiple of the gulp length, offset a multiple of it).  Valid until
+ * (ld a multiple of the gulp length, offset a multiple of it).  With
+ * history_in_place the window of a DM of 0 may be the gulp itself.  Valid until
  * the next run. */
 int sw_codedisp_window(const sw_codedisp* plan, int dm, const void** d_ring, int* ld, int* offset);
 /* End the gulp d_ftpa: advance the overlap-save history and the segment

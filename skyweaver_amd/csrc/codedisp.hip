@@ -868,6 +868,46 @@ __global__ void chirp_kernel(float2* out, int nchans, int N, int RP, int R1, dou
     out[((size_t)chan * RP + r) * L + mp] = make_float2((float)c * scale, (float)s * scale);
 }
 
+// A DM of exactly 0 has the chirp H = 1: its transform pair returns the int8
+// input, since the FP32 pair's error (relative L2 norm 1e-6 over a segment,
+// below 0.1 in any one sample for int8 input up to N = 262144) never reaches
+// the half that rounding needs.  So its segments' kept samples are copied:
+// ring samples [y0, y0 + n) (mod R) of every column from input samples
+// [i0, i0 + n) relative to the gulp start, below 0 from the history lo (ll
+// samples per column, ending at the gulp start).  The caller keeps
+// -ll <= i0 and i0 + n <= T.
+// HBM-bound: a thread writes one 16-byte block of a column's ring (V8: the
+// ring's columns are whole blocks) from one unaligned 16-byte read; only a
+// column's first and last blocks and the block that straddles the gulp start
+// go sample by sample.  64 channels x 128 columns x 65536 samples: 0.39 ms
+// (5.5 TB/s) where the transform pair at N = 1024 takes 1.25 ms.
+template <bool V8>
+__global__ void __launch_bounds__(256)
+codedisp_copy_kernel(const uint16_t* __restrict__ cur, const uint16_t* __restrict__ lo, int ll, int T,
+                     uint16_t* __restrict__ ring, int R, int i0, int y0, int n, int ncols)
+{
+    constexpr int B = V8 ? 8 : 1;  // samples per block
+    const int k0 = y0 / B;         // first block touched (before the wrap)
+    const int k = k0 + (int)(blockIdx.x * 256 + threadIdx.x);
+    const int q0 = k * B - y0;     // the block's first sample, counted from y0
+    if(q0 >= n) return;
+    const int j = k * B >= R ? k * B - R : k * B;
+    const int tau = i0 + q0;
+    for(int col = blockIdx.y; col < ncols; col += gridDim.y) {
+        const uint16_t* c = cur + (size_t)col * T;
+        const uint16_t* l = lo + (size_t)col * ll + ll;
+        uint16_t* o = ring + (size_t)col * R + j;
+        if(V8 && q0 >= 0 && q0 + B <= n && (tau >= 0 || tau + B <= 0)) {
+            uint4 v;
+            __builtin_memcpy(&v, (tau >= 0 ? c : l) + tau, 16);  // 2-byte aligned
+            *reinterpret_cast<uint4*>(o) = v;
+        } else {
+            for(int e = 0; e < B; ++e)
+                if(q0 + e >= 0 && q0 + e < n) o[e] = (tau + e >= 0 ? c : l)[tau + e];
+        }
+    }
+}
+
 // new history = the last Oh samples of (old history ++ gulp), per column
 __global__ void history_kernel(int8_t* dst, const int8_t* old, const int8_t* cur, int ncols, int T, int Oh)
 {
@@ -1010,7 +1050,9 @@ struct sw_codedisp {
     std::vector<int8_t*> ytm;            // per DM: output ring [F][PA][ylen], time-major
     std::vector<float2*> ytf;            // per DM, on demand: float output ring, same layout
     std::vector<int> ylen;               // per DM ring length: T + lat rounded up to a multiple of T
-    std::vector<int> wstart;             // per DM: ring index of the last run's emitted window
+    std::vector<int> wstart;             // per DM: index of the last run's emitted window in its source
+    std::vector<const int8_t*> wsrc;     // per DM: that source: the ring, or the gulp itself (DM 0 in place)
+    std::vector<int> wld;                // per DM: samples per column of the source
     bool hist_ref = false;               // history read in place from the previous gulp
     const int8_t* prev = nullptr;        // that gulp (null before the first)
     std::vector<int> lat;                // per DM output latency
@@ -1146,6 +1188,8 @@ extern "C" int sw_codedisp_create(const sw_codedisp_config* cfg, void* stream, s
     p->lat.assign(p->dms.size(), 0);
     p->ylen.assign(p->dms.size(), p->T);
     p->wstart.assign(p->dms.size(), 0);
+    p->wld.assign(p->dms.size(), p->T);
+    p->wsrc.assign(p->dms.size(), nullptr);
     for(auto& g : p->groups) {
         // history: the input a gulp's first segment can reach back to
         p->Oh = std::max(p->Oh, g.lat > 0 ? g.N : g.O);
@@ -1205,6 +1249,8 @@ extern "C" int sw_codedisp_create(const sw_codedisp_config* cfg, void* stream, s
         const size_t yb = (size_t)p->F * p->PA * p->ylen[d] * 2;
         SW_HIP_TRY(hipMalloc(&p->ytm[d], yb));
         SW_HIP_TRY(hipMemsetAsync(p->ytm[d], 0, yb, st));  // outputs before the stream start are zero
+        p->wsrc[d] = p->ytm[d];
+        p->wld[d] = p->ylen[d];
     }
     (void)slots;
     if(zmax) {
@@ -1424,8 +1470,8 @@ static const int8_t* time_major_input(sw_codedisp* plan, const void* d_in, hipSt
 extern "C" int sw_codedisp_window(const sw_codedisp* plan, int dm, const void** d_ring, int* ld, int* offset)
 {
     SW_CHECK_ARG(plan && dm >= 0 && dm < (int)plan->dms.size(), "bad plan or DM index");
-    if(d_ring) *d_ring = plan->ytm[dm];
-    if(ld) *ld = plan->ylen[dm];
+    if(d_ring) *d_ring = plan->wsrc[dm];
+    if(ld) *ld = plan->wld[dm];
     if(offset) *offset = plan->wstart[dm];
     return SW_OK;
 }
@@ -1452,6 +1498,75 @@ extern "C" int sw_codedisp_push_history(sw_codedisp* plan, const void* d_in, voi
     return SW_OK;
 }
 
+// The window that DM d's ring emits for the gulp at stream sample gT, ring
+// [gT mod R, +T) (two pieces if it wraps, which the gulp-multiple ring length
+// rules out), turned to FTPA in out unless null; outf (or null) likewise from
+// the float ring.
+static int emit_window(sw_codedisp* plan, int d, long long gT, void* out, void* outf, hipStream_t st)
+{
+    const long long R = plan->ylen[d];
+    const int start = (int)(gT % R);
+    plan->wsrc[d] = plan->ytm[d];
+    plan->wld[d] = (int)R;
+    plan->wstart[d] = start;
+    if(!out) return SW_OK;
+    const int n1 = (int)std::min<long long>(plan->T, R - start), n2 = plan->T - n1;
+    const size_t PA = plan->PA;
+    int rc = sw::corner_turn(plan->ytm[d] + (size_t)start * 2, out, plan->F, plan->PA, n1, st, (int)R, plan->T);
+    if(rc) return rc;
+    if(n2 > 0) {
+        rc = sw::corner_turn(plan->ytm[d], static_cast<int8_t*>(out) + (size_t)n1 * PA * 2, plan->F, plan->PA, n2, st,
+                             (int)R, plan->T);
+        if(rc) return rc;
+    }
+    if(outf) {
+        rc = sw::corner_turn_f64(plan->ytf[d] + start, outf, plan->F, plan->PA, n1, st, (int)R, plan->T);
+        if(rc) return rc;
+        if(n2 > 0) {
+            rc = sw::corner_turn_f64(plan->ytf[d], static_cast<float2*>(outf) + (size_t)n1 * PA, plan->F, plan->PA, n2,
+                                     st, (int)R, plan->T);
+            if(rc) return rc;
+        }
+    }
+    return SW_OK;
+}
+
+// DM 0 of group g for the gulp `cur` (time-major): no transform (see
+// codedisp_copy_kernel).  When the segments tile the gulp (no overlap, no
+// latency) and the caller keeps the gulp until the next run
+// (history_in_place), its window is the gulp itself and nothing is moved.
+static int run_dm0(sw_codedisp* plan, const sw::CodedispGroup& g, int d, const int8_t* cur, long long m0, int nseg,
+                   long long gT, void* out, hipStream_t st)
+{
+    if(plan->hist_ref && g.O == 0 && g.lat == 0) {
+        plan->wsrc[d] = cur;
+        plan->wld[d] = plan->T;
+        plan->wstart[d] = 0;
+        return out ? sw::corner_turn(cur, out, plan->F, plan->PA, plan->T, st, plan->T, plan->T) : SW_OK;
+    }
+    const long long n = (long long)nseg * g.hop;
+    if(n > 0) {
+        const int R = plan->ylen[d], ncols = plan->F * plan->PA;
+        const int i0 = (int)(m0 * g.hop - g.O / 2 - gT), y0 = (int)((m0 * g.hop + g.lat) % R);
+        const bool prev = plan->hist_ref && plan->prev;
+        const auto* c = reinterpret_cast<const uint16_t*>(cur);
+        const auto* lo = reinterpret_cast<const uint16_t*>(prev ? plan->prev : plan->hist);
+        const int ll = prev ? plan->T : plan->Oh;
+        auto* ring = reinterpret_cast<uint16_t*>(plan->ytm[d]);
+        const bool v8 = R % 8 == 0;
+        const int nblk = v8 ? (int)((y0 + n - 1) / 8 - y0 / 8 + 1) : (int)n;
+        const dim3 grid((unsigned)((nblk + 255) / 256), (unsigned)std::min(ncols, 65535));
+        if(v8)
+            hipLaunchKernelGGL(sw::codedisp_copy_kernel<true>, grid, dim3(256), 0, st, c, lo, ll, plan->T, ring, R, i0,
+                               y0, (int)n, ncols);
+        else
+            hipLaunchKernelGGL(sw::codedisp_copy_kernel<false>, grid, dim3(256), 0, st, c, lo, ll, plan->T, ring, R,
+                               i0, y0, (int)n, ncols);
+        SW_LAUNCH_CHECK();
+    }
+    return emit_window(plan, d, gT, out, nullptr, st);
+}
+
 extern "C" int sw_codedisp_run(sw_codedisp* plan, const void* d_in, void* const* d_out,
                                void* const* d_out_f32, int dm_begin, int dm_count, int batched,
                                void* stream)
@@ -1464,14 +1579,23 @@ extern "C" int sw_codedisp_run(sw_codedisp* plan, const void* d_in, void* const*
     const int8_t* cur = time_major_input(plan, d_in, st, rc);
     if(rc) return rc;
     for(auto& g : plan->groups) {
-        std::vector<int> todo;
-        for(int d : g.dms)
-            if(d >= dm_begin && d < dm_begin + dm_count) todo.push_back(d);
         // segments of this gulp: all grid segments whose input ends within it
         const long long gT = plan->gulps * (long long)plan->T;
         const long long m0 = g.mdone;
         const long long m1 = (gT + plan->T) / g.hop;
         const int nseg = (int)(m1 - m0);
+        std::vector<int> todo;
+        for(int d : g.dms) {
+            if(d < dm_begin || d >= dm_begin + dm_count) continue;
+            // DM 0 moves samples; asked for float outputs (a diagnostic path)
+            // it is transformed like the others
+            if(plan->dms[d] == 0.0f && !(d_out_f32 && d_out_f32[d])) {
+                rc = run_dm0(plan, g, d, cur, m0, nseg, gT, d_out[d], st);
+                if(rc) return rc;
+            } else {
+                todo.push_back(d);
+            }
+        }
         if(nseg <= 0 && !todo.empty()) {
             // nothing new to transform (possible only when a gulp is shorter than hop)
         }
@@ -1547,35 +1671,12 @@ extern "C" int sw_codedisp_run(sw_codedisp* plan, const void* d_in, void* const*
                     SW_LAUNCH_CHECK();
                 }
             }
-            // emitted window, ring [gT mod R, +T) (two pieces if it wraps, which
-            // the gulp-multiple ring length rules out), -> FTPA for the
-            // beamformers unless d_out[d] is null (left in the ring)
+            // the emitted windows -> FTPA for the beamformers unless d_out[d]
+            // is null (left in the ring)
             for(int k = 0; k < nb; ++k) {
                 const int d = todo[b0 + k];
-                const long long R = plan->ylen[d];
-                const int start = (int)(gT % R);
-                plan->wstart[d] = start;
-                if(!d_out[d]) continue;
-                const int n1 = (int)std::min<long long>(plan->T, R - start), n2 = plan->T - n1;
-                const size_t PA = plan->PA;
-                rc = sw::corner_turn(plan->ytm[d] + (size_t)start * 2, d_out[d], plan->F, plan->PA, n1, st,
-                                     (int)R, plan->T);
+                rc = emit_window(plan, d, gT, d_out[d], p.outf[k] ? d_out_f32[d] : nullptr, st);
                 if(rc) return rc;
-                if(n2 > 0) {
-                    rc = sw::corner_turn(plan->ytm[d], static_cast<int8_t*>(d_out[d]) + (size_t)n1 * PA * 2, plan->F,
-                                         plan->PA, n2, st, (int)R, plan->T);
-                    if(rc) return rc;
-                }
-                if(p.outf[k]) {
-                    rc = sw::corner_turn_f64(plan->ytf[d] + start, d_out_f32[d], plan->F, plan->PA, n1, st, (int)R,
-                                             plan->T);
-                    if(rc) return rc;
-                    if(n2 > 0) {
-                        rc = sw::corner_turn_f64(plan->ytf[d], static_cast<float2*>(d_out_f32[d]) + (size_t)n1 * PA,
-                                                 plan->F, plan->PA, n2, st, (int)R, plan->T);
-                        if(rc) return rc;
-                    }
-                }
             }
         }
     }

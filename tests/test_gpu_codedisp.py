@@ -330,3 +330,33 @@ def test_codedisp_autotune(sw, dev):
     p(DB.from_host(sw.synth_voltages((16, A, F, 256, 2, 2), seed=2, sigma=16.0)))
     p.close()
     assert got == [0, 1, 2]
+
+
+@pytest.mark.parametrize("fpat,in_place", [(True, True), (True, False), (False, False)])
+@pytest.mark.parametrize("T,N,O", [(2048, 1024, 0),   # the segments tile the gulp: no latency
+                                   (1536, 1024, 0),   # latency, aligned
+                                   (1536, 1024, 62),  # latency, overlap: unaligned blocks
+                                   (1500, 512, 10),   # a ring of no whole 16-byte blocks
+                                   (640, 1024, 20)])  # a gulp shorter than a segment: empty gulps
+def test_codedisp_dm0_is_a_delay(sw, dev, fpat, in_place, T, N, O):
+    """DM 0 has the chirp 1: output sample x of the stream is input sample x - O / 2 (zero
+    before the stream), bit for bit, also when a DM of the same length is transformed beside it."""
+    from skyweaver_amd import DeviceBuffer as DB
+    F, A, G = 3, 16, 5
+    rng = np.random.default_rng(T + N + O)
+    x = rng.integers(-128, 128, (F, G * T, 2, A, 2)).astype(np.int8)  # FTPA stream
+    plan = sw.CoherentDedisperser(F, A, T, F_LOW, CHAN_BW, TSAMP, [0.0, 30.0], fft_len=[N, N], overlap=[O, O],
+                                  input_fpat=fpat, history_in_place=in_place)
+    L = plan.latency(0)
+    stream = np.concatenate([np.zeros((F, L + O // 2) + x.shape[2:], np.int8), x], 1)
+    bufs = []
+    for g in range(G):
+        cur = x[:, g * T:(g + 1) * T]
+        if fpat:
+            cur = cur.transpose(0, 2, 3, 1, 4)
+        bufs.append(DB.from_host(np.ascontiguousarray(cur)))
+        out = DB.empty((F, T, 2, A, 2), np.int8, fill=0x55)
+        other = DB.empty((F, T, 2, A, 2), np.int8, fill=0x55)
+        plan.run(bufs[-1], [out, other])
+        plan.push_history(bufs[-1])
+        assert np.array_equal(out.download(), stream[:, g * T:(g + 1) * T]), g
