@@ -10,121 +10,214 @@
 // to every beamset and caps the antenna count at 64), every beamset uses its
 // own weight row and any antenna count works.
 //
-// Each lane owns one output sample (t', f) and accumulates in exactly the
-// oracle's order (time ascending, antenna ascending, one rounding for the
-// product and one for the sum), so raw powers are bit-identical to the
-// oracle for any weights, not only when the sums happen to be exact.  The
-// rows are staged through LDS so that the HBM reads are coalesced.
+// The float chain sums in exactly the oracle's order (time ascending, antenna
+// ascending, one rounding for the product and one for the sum), so raw powers
+// are bit-identical to the oracle for any weights, not only when the sums
+// happen to be exact.
 //
-// Exact fast path (Stokes I, antenna weights all 0 or 1): every term
-// w_a (re^2 + im^2) is a non-negative integer, so while the total stays
-// below 2^24 every partial sum of the oracle's float chain is exact and the
-// float result equals the integer sum.  The kernel then sums with
-// v_dot4_i32_i8 (two antennas of one polarisation per word, masked by the
-// beamset's 0/1 weights) in int32 and converts once; a wave whose total
-// reaches 2^24 on any lane recomputes its outputs with the float chain.
+// Exact fast path (antenna weights all 0 or 1): every term of the float chain
+// is an integer, and the terms of Q, U and V are no larger than Stokes I's
+// (|2 p0 conj(p1)| <= |p0|^2 + |p1|^2), so while the Stokes I total stays below
+// 2^24 every partial sum of any of the four chains is exact and the float
+// results equal the integer sums, whatever their order.  The kernel then sums
+// with v_dot4_i32_i8 (two antennas of one polarisation per word, masked by the
+// beamset's 0/1 weights) and converts once; a workgroup with a Stokes I total
+// of 2^24 or more recomputes its outputs with the float chain.
 #include "sw_common.hpp"
+
+#include <type_traits>
 
 namespace sw {
 namespace {
 
-constexpr int kOut = 64;        // output samples per workgroup (one wave)
+constexpr int kIbThreads = 256;
 constexpr int kMaskWords = 64;  // 0/1 weight masks for up to 128 antennas
 
-// One wave per (64 consecutive output samples, channel).  For each step tt of
-// the scrunch window the 64 rows t'*ts + tt (one per output) are staged in
-// LDS with coalesced 16-byte loads; each lane then accumulates its own row,
-// antennas ascending, for every beamset.
-template <int S, int SMAX>
-__global__ void __launch_bounds__(kOut)
+// 2^24: integers below it are exact in FP32
+constexpr int kExact = 1 << 24;
+
+// The power sums of one output: |p0|^2, |p1|^2, and for U and V the halves
+// r0 r1 + i0 i1, i0 r1 and r0 i1 of two antennas per word.  The two squares
+// saturate (a total past int32 must still read as >= 2^24).
+template <int S>
+struct IbSums {
+    static constexpr bool kU = S == SW_STOKES_U || S == SW_STOKES_IQUV;
+    static constexpr bool kV = S == SW_STOKES_V || S == SW_STOKES_IQUV;
+    int p0 = 0, p1 = 0, u = 0, v0 = 0, v1 = 0;
+    __device__ __forceinline__ void add(uint32_t x0, uint32_t x1, uint32_t m)
+    {
+        const uint32_t a0 = x0 & m;
+        p0 = __builtin_amdgcn_sdot4((int)a0, (int)x0, p0, true);
+        p1 = __builtin_amdgcn_sdot4((int)(x1 & m), (int)x1, p1, true);
+        if constexpr(kU) u = __builtin_amdgcn_sdot4((int)a0, (int)x1, u, false);
+        if constexpr(kV) {
+            // [i, 0] and [0, r] of each antenna against x1's [r, i]
+            const uint32_t im = __builtin_amdgcn_perm(a0, a0, 0x0C030C01u);
+            const uint32_t re = __builtin_amdgcn_perm(a0, a0, 0x020C000Cu);
+            v0 = __builtin_amdgcn_sdot4((int)im, (int)x1, v0, false);
+            v1 = __builtin_amdgcn_sdot4((int)re, (int)x1, v1, false);
+        }
+    }
+    // Stokes I, at most 2^24 (64 of these sum without overflow)
+    __device__ __forceinline__ int total() const { return min(min(p0, kExact) + min(p1, kExact), kExact); }
+    // the wanted Stokes parameters but I, exact while I's total is below 2^24
+    __device__ __forceinline__ int q() const { return (int)((uint32_t)p0 - (uint32_t)p1); }
+    __device__ __forceinline__ int uu() const { return 2 * u; }
+    __device__ __forceinline__ int vv() const { return 2 * (int)((uint32_t)v0 - (uint32_t)v1); }
+};
+
+// the sum over `lanes` (a power of two) neighbouring lanes
+__device__ __forceinline__ int lanes_sum(int v, int lanes)
+{
+    for(int m = 1; m < lanes; m <<= 1) v += __shfl_xor(v, m, 64);
+    return v;
+}
+
+// A workgroup owns `batches` runs of ob = 256 / lanes consecutive outputs of
+// one channel.  HBM-bound: `lanes` neighbouring lanes share an output, each
+// reading 4 W bytes (2 W antennas) of both polarisations of every (lanes /
+// chunks)-th row of its scrunch window, up to four rows' loads in flight, so
+// that a wave reads whole rows and nothing goes through LDS; the lanes' sums
+// meet in a shuffle tree.  (Staged through LDS by one wave per 64 outputs,
+// each lane then summing a whole window, the loads of a row were waited for
+// before the sums of it: 64 channels x 16384 samples x 64 antennas, two
+// beamsets, took 150 us, IQUV of 16 channels x 32768 samples 206 us.)
+template <int S, int SMAX, int W>
+__global__ void __launch_bounds__(kIbThreads)
 ib_kernel(const uint8_t* __restrict__ ftpa, float* __restrict__ raw, int8_t* __restrict__ out,
           const float* __restrict__ scale, const float* __restrict__ offset,
           const float* __restrict__ antw, int nchans, int nsamples, int nant, int tscrunch,
-          int nbeamsets)
+          int nbeamsets, int lanes, int batches)
 {
     constexpr int NV = nstokes(S);
-    extern __shared__ uint4 rows[];           // [kOut][rowq + 1]
+    using P = typename std::conditional<W == 4, uint4, uint2>::type;
+    extern __shared__ uint4 rows[];           // float chain: [ob batches][rowq + 1]
     const int f    = blockIdx.y;
-    const int lane = threadIdx.x;
+    const int tid  = threadIdx.x;
     const int nsamps_out = nsamples / tscrunch;
-    const int tp0  = blockIdx.x * kOut;
-    const int tp   = tp0 + lane;
-    const int rowq = nant / 4;                // 16-byte chunks per (t) row: 4*nant bytes
-    const int ldsq = rowq + 1;
-    const int nrows = min(kOut, nsamps_out - tp0);
-    float power[SMAX][NV];
-#pragma unroll
-    for(int s = 0; s < SMAX; ++s)
-#pragma unroll
-        for(int k = 0; k < NV; ++k) power[s][k] = 0.0f;
-    const uint4* chan = reinterpret_cast<const uint4*>(ftpa + (size_t)f * nsamples * 4 * nant);
+    const int ob   = kIbThreads / lanes;
+    const int tp0  = blockIdx.x * ob * batches;
+    const uint8_t* chan = ftpa + (size_t)f * nsamples * 4 * nant;
+
+    auto store = [&](int s, int tp, const float* power) {
+        const size_t o  = ((size_t)s * nsamps_out + tp) * nchans + f;
+        const float sc  = scale[s * nchans + f];
+        const float off = offset[s * nchans + f];
+        if constexpr(NV == 1) {
+            raw[o] = power[0];
+            out[o] = clamp_i8(rescale<S>(power[0], off, sc));
+        } else {
+            reinterpret_cast<float4*>(raw)[o] = make_float4(power[0], power[1], power[2], power[3]);
+            char4 q;
+            q.x = clamp_i8(rescale<SW_STOKES_I>(power[0], off, sc));
+            q.y = clamp_i8(rescale<SW_STOKES_Q>(power[1], off, sc));
+            q.z = clamp_i8(rescale<SW_STOKES_U>(power[2], off, sc));
+            q.w = clamp_i8(rescale<SW_STOKES_V>(power[3], off, sc));
+            reinterpret_cast<char4*>(out)[o] = q;
+        }
+    };
 
     // ---- exact integer path
     __shared__ uint32_t wmask[SMAX][kMaskWords];  // per word: 0xFFFF per antenna of weight 1
-    bool exact = false;
-    if constexpr(S == SW_STOKES_I) {
-        if(nant <= 2 * kMaskWords) {
-            bool binary = true;
-            for(int i = lane; i < nbeamsets * nant / 2; i += kOut) {
-                const int sb = i / (nant / 2), j = i % (nant / 2);
-                const float w0 = antw[sb * nant + 2 * j], w1 = antw[sb * nant + 2 * j + 1];
-                binary = binary && (w0 == 0.0f || w0 == 1.0f) && (w1 == 0.0f || w1 == 1.0f);
-                wmask[sb][j] = (w0 != 0.0f ? 0x0000FFFFu : 0u) | (w1 != 0.0f ? 0xFFFF0000u : 0u);
-            }
-            exact = __syncthreads_and(binary);
+    bool exact = nant <= 2 * kMaskWords;
+    if(exact) {
+        bool binary = true;
+        for(int i = tid; i < nbeamsets * nant / 2; i += kIbThreads) {
+            const int sb = i / (nant / 2), j = i % (nant / 2);
+            const float w0 = antw[sb * nant + 2 * j], w1 = antw[sb * nant + 2 * j + 1];
+            binary = binary && (w0 == 0.0f || w0 == 1.0f) && (w1 == 0.0f || w1 == 1.0f);
+            wmask[sb][j] = (w0 != 0.0f ? 0x0000FFFFu : 0u) | (w1 != 0.0f ? 0xFFFF0000u : 0u);
         }
+        exact = __syncthreads_and(binary);
     }
     if(exact) {
-        int isum[SMAX];
+        const int chunks = nant / (2 * W);        // loads per polarisation of a row
+        const int krow   = max(1, lanes / chunks);  // rows an output's lanes read together
+        const int l = tid % lanes;
+        bool big = false;
+        for(int b = 0; b < batches; ++b) {
+            const int tp = tp0 + b * ob + tid / lanes;
+            IbSums<S> sum[SMAX];
+            if(l < krow * chunks && tp < nsamps_out) {
+                for(int q = l % chunks; q < chunks; q += lanes) {  // once unless lanes < chunks
+                    uint32_t m[SMAX][W];
 #pragma unroll
-        for(int s = 0; s < SMAX; ++s) isum[s] = 0;
-        const int hw = nant / 2;  // words per polarisation
-        for(int tt = 0; tt < tscrunch; ++tt) {
-            __syncthreads();
-            for(int i = lane; i < nrows * rowq; i += kOut) {
-                const int r = i / rowq, q = i % rowq;
-                rows[r * ldsq + q] = chan[((size_t)(tp0 + r) * tscrunch + tt) * rowq + q];
-            }
-            __syncthreads();
-            if(lane < nrows) {
-                const uint32_t* rw = reinterpret_cast<const uint32_t*>(rows + lane * ldsq);
+                    for(int s = 0; s < SMAX; ++s)
 #pragma unroll
-                for(int s = 0; s < SMAX; ++s) {
-                    if(s < nbeamsets) {
-                        int acc = 0;
-                        for(int j = 0; j < hw; ++j) {
-                            const int m = (int)wmask[s][j];
-                            const int x0 = (int)rw[j], x1 = (int)rw[hw + j];
-                            acc = __builtin_amdgcn_sdot4(x0 & m, x0, acc, false);
-                            acc = __builtin_amdgcn_sdot4(x1 & m, x1, acc, false);
+                        for(int j = 0; j < W; ++j) m[s][j] = s < nbeamsets ? wmask[s][q * W + j] : 0u;
+                    const P* x = reinterpret_cast<const P*>(chan) + (size_t)tp * tscrunch * 2 * chunks + q;
+                    auto row = [&](const P& v0, const P& v1) {
+                        const uint32_t* x0 = reinterpret_cast<const uint32_t*>(&v0);
+                        const uint32_t* x1 = reinterpret_cast<const uint32_t*>(&v1);
+#pragma unroll
+                        for(int s = 0; s < SMAX; ++s)
+                            if(s < nbeamsets)
+#pragma unroll
+                                for(int j = 0; j < W; ++j) sum[s].add(x0[j], x1[j], m[s][j]);
+                    };
+                    int tt = l / chunks;
+                    for(; tt + 3 * krow < tscrunch; tt += 4 * krow) {
+                        P v[8];
+#pragma unroll
+                        for(int k = 0; k < 4; ++k) {
+                            const P* r = x + (size_t)(tt + k * krow) * 2 * chunks;
+                            v[2 * k]     = r[0];
+                            v[2 * k + 1] = r[chunks];
                         }
-                        isum[s] += acc;
+#pragma unroll
+                        for(int k = 0; k < 4; ++k) row(v[2 * k], v[2 * k + 1]);
+                    }
+                    for(; tt < tscrunch; tt += krow) {
+                        const P* r = x + (size_t)tt * 2 * chunks;
+                        row(r[0], r[chunks]);
                     }
                 }
             }
-        }
-        bool big = false;
 #pragma unroll
-        for(int s = 0; s < SMAX; ++s) {
-            big = big || (isum[s] >= (1 << 24));
-            power[s][0] = (float)isum[s];
+            for(int s = 0; s < SMAX; ++s) {
+                if(s < nbeamsets) {  // uniform
+                    float power[NV];
+                    const int tot = lanes_sum(sum[s].total(), lanes);
+                    if constexpr(S == SW_STOKES_I || NV == 4) power[0] = (float)tot;
+                    if constexpr(S == SW_STOKES_Q) power[0] = (float)lanes_sum(sum[s].q(), lanes);
+                    if constexpr(S == SW_STOKES_U) power[0] = (float)lanes_sum(sum[s].uu(), lanes);
+                    if constexpr(S == SW_STOKES_V) power[0] = (float)lanes_sum(sum[s].vv(), lanes);
+                    if constexpr(NV == 4) {
+                        power[1] = (float)lanes_sum(sum[s].q(), lanes);
+                        power[2] = (float)lanes_sum(sum[s].uu(), lanes);
+                        power[3] = (float)lanes_sum(sum[s].vv(), lanes);
+                    }
+                    big = big || tot >= kExact;
+                    if(l == 0 && tp < nsamps_out) store(s, tp, power);
+                }
+            }
         }
-        exact = !__any(big);  // wave-uniform
+        exact = !__syncthreads_or(big);
+        if(exact) return;
     }
-    if(!exact) {
+
+    // ---- float chain: the rows t' ts + tt (one per output) staged in LDS with
+    // coalesced 16-byte loads; each output's lane then sums its own row,
+    // antennas ascending, for every beamset
+    const int nout = ob * batches;  // at most 64
+    const int rowq = nant / 4;      // 16-byte pieces per row: 4 nant bytes
+    const int ldsq = rowq + 1;
+    const int nrows = min(nout, nsamps_out - tp0);
+    const uint4* chan16 = reinterpret_cast<const uint4*>(chan);
+    float power[SMAX][NV];
 #pragma unroll
     for(int s = 0; s < SMAX; ++s)
 #pragma unroll
         for(int k = 0; k < NV; ++k) power[s][k] = 0.0f;
     for(int tt = 0; tt < tscrunch; ++tt) {
         __syncthreads();
-        for(int i = lane; i < nrows * rowq; i += kOut) {
+        for(int i = tid; i < nrows * rowq; i += kIbThreads) {
             const int r = i / rowq, q = i % rowq;
-            rows[r * ldsq + q] = chan[((size_t)(tp0 + r) * tscrunch + tt) * rowq + q];
+            rows[r * ldsq + q] = chan16[((size_t)(tp0 + r) * tscrunch + tt) * rowq + q];
         }
         __syncthreads();
-        if(lane < nrows) {
-            const uint8_t* rb = reinterpret_cast<const uint8_t*>(rows + lane * ldsq);
+        if(tid < nrows) {
+            const uint8_t* rb = reinterpret_cast<const uint8_t*>(rows + tid * ldsq);
             for(int a4 = 0; a4 < nant; a4 += 4) {
                 // 4 antennas of pol 0 and of pol 1 (8 bytes each, 8-byte aligned)
                 const uint2 q0 = *reinterpret_cast<const uint2*>(rb + a4 * 2);
@@ -158,29 +251,10 @@ ib_kernel(const uint8_t* __restrict__ ftpa, float* __restrict__ raw, int8_t* __r
             }
         }
     }
-    }
-    if(tp >= nsamps_out) return;
+    if(tid >= nrows) return;
 #pragma unroll
-    for(int s = 0; s < SMAX; ++s) {
-        if(s < nbeamsets) {
-            const size_t o  = ((size_t)s * nsamps_out + tp) * nchans + f;
-            const float sc  = scale[s * nchans + f];
-            const float off = offset[s * nchans + f];
-            if constexpr(NV == 1) {
-                raw[o] = power[s][0];
-                out[o] = clamp_i8(rescale<S>(power[s][0], off, sc));
-            } else {
-                reinterpret_cast<float4*>(raw)[o] =
-                    make_float4(power[s][0], power[s][1], power[s][2], power[s][3]);
-                char4 q;
-                q.x = clamp_i8(rescale<SW_STOKES_I>(power[s][0], off, sc));
-                q.y = clamp_i8(rescale<SW_STOKES_Q>(power[s][1], off, sc));
-                q.z = clamp_i8(rescale<SW_STOKES_U>(power[s][2], off, sc));
-                q.w = clamp_i8(rescale<SW_STOKES_V>(power[s][3], off, sc));
-                reinterpret_cast<char4*>(out)[o] = q;
-            }
-        }
-    }
+    for(int s = 0; s < SMAX; ++s)
+        if(s < nbeamsets) store(s, tp0 + tid, power[s]);
 }
 
 // Time-major input (the coherent dedisperser's ring): sample t of column
@@ -274,20 +348,40 @@ int launch_ib(const uint8_t* ftpa, float* raw, int8_t* out, const float* scale,
               const float* offset, const float* antw, const sw_bf_dims& d, hipStream_t st)
 {
     const int nout = d.nsamples / d.tscrunch;
-    dim3 grid((nout + kOut - 1) / kOut, d.nchans);
-    const size_t lds = (size_t)kOut * (d.nantennas / 4 + 1) * 16;
-#define SW_IB_LAUNCH(SM)                                                                     \
-    hipLaunchKernelGGL((ib_kernel<S, SM>), grid, dim3(kOut), lds, st, ftpa, raw, out,         \
-                       scale, offset, antw, d.nchans, d.nsamples, d.nantennas, d.tscrunch,   \
-                       d.nbeamsets)
-    if(d.nbeamsets <= 1)
-        SW_IB_LAUNCH(1);
-    else if(d.nbeamsets <= 4)
-        SW_IB_LAUNCH(4);
-    else if(d.nbeamsets <= 8)
-        SW_IB_LAUNCH(8);
-    else
-        SW_IB_LAUNCH(16);
+    const bool w4 = d.nantennas % 8 == 0;  // 16-byte loads, else 8-byte
+    const int chunks = d.nantennas / (w4 ? 8 : 4);
+    // 8 lanes per output (a row of 64 antennas' polarisation at 16 bytes a
+    // lane), more where a row takes more loads; then, while the chip is not
+    // filled four times over with workgroups, more lanes with fewer rows
+    // each, down to the four rows a lane has in flight
+    int lanes = 8;
+    while(lanes < 64 && lanes < chunks) lanes *= 2;
+    auto groups = [&](int ob) { return (long)((nout + ob - 1) / ob) * d.nchans; };
+    while(lanes < 64 && groups(kIbThreads / lanes) < 1024 && (long)d.tscrunch * chunks >= 8L * lanes) lanes *= 2;
+    const int ob = kIbThreads / lanes;
+    // 64 outputs per workgroup where enough workgroups are left: the float
+    // chain then fills its wave
+    const int batches = groups(64) >= 2048 ? 64 / ob : 1;
+    const dim3 grid((unsigned)((nout + ob * batches - 1) / (ob * batches)), d.nchans);
+    const size_t lds = (size_t)ob * batches * (d.nantennas / 4 + 1) * 16;
+#define SW_IB_LAUNCH(SM)                                                                                    \
+    if(w4)                                                                                                  \
+        hipLaunchKernelGGL((ib_kernel<S, SM, 4>), grid, dim3(kIbThreads), lds, st, ftpa, raw, out, scale,   \
+                           offset, antw, d.nchans, d.nsamples, d.nantennas, d.tscrunch, d.nbeamsets, lanes, \
+                           batches);                                                                        \
+    else                                                                                                    \
+        hipLaunchKernelGGL((ib_kernel<S, SM, 2>), grid, dim3(kIbThreads), lds, st, ftpa, raw, out, scale,   \
+                           offset, antw, d.nchans, d.nsamples, d.nantennas, d.tscrunch, d.nbeamsets, lanes, \
+                           batches);
+    if(d.nbeamsets <= 1) {
+        SW_IB_LAUNCH(1)
+    } else if(d.nbeamsets <= 2) {
+        SW_IB_LAUNCH(2)
+    } else if(d.nbeamsets <= 4) {
+        SW_IB_LAUNCH(4)
+    } else {
+        SW_IB_LAUNCH(16)
+    }
 #undef SW_IB_LAUNCH
     SW_LAUNCH_CHECK();
     return SW_OK;

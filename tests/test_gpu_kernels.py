@@ -177,6 +177,32 @@ def test_ib_parity_exact_path_overflow(sw, orc, dev, A, ts, S):
     np.testing.assert_array_equal(out, eout)
 
 
+@pytest.mark.parametrize("stokes", ["I", "Q", "U", "V", "IQUV"])
+@pytest.mark.parametrize("F,T,A,ts,S", [(1, 64, 4, 1, 1),       # one 8-byte piece per row, 8 rows wide
+                                        (2, 4096, 20, 32, 3),   # 8-byte pieces, lanes left idle
+                                        (3, 1500, 48, 5, 2),    # a window of no power of two, a partial workgroup
+                                        (2, 2048, 64, 64, 5),   # 64 lanes per output
+                                        (2, 1024, 128, 8, 1),
+                                        (64, 2048, 16, 1, 1)])  # 64 outputs per workgroup, in batches
+def test_ib_exact_path_splits(sw, orc, dev, stokes, F, T, A, ts, S):
+    """The ways a workgroup's lanes share outputs, rows and antennas; 0/1 weights with antennas
+    left out.  Full-scale values push some of the totals past 2^24 where the shape allows, and
+    those workgroups to the float chain."""
+    v = _rand_c8((F, T, 2, A), 17 + A, sigma=40.0)
+    v[0, :ts] = -128
+    w = (_rng(S).random((S, A)) > 0.4).astype(np.float32)
+    w[0] = 1
+    scale, offset = _ib_scales(F, S, A, ts)
+    raw, out = _run_ib(sw, dev, v, w, scale, offset, ts, stokes)
+    if F > 8:  # the oracle on a few channels
+        pick = [0, F // 2, F - 1]
+        v, raw, out = v[pick], raw[:, :, pick], out[:, :, pick]
+        scale, offset = (x.reshape(S, F)[:, pick].reshape(-1).copy() for x in (scale, offset))
+    eraw, eout = orc.ib_beamform(np.ascontiguousarray(v), ts, scale, offset, w, S, stokes)
+    np.testing.assert_array_equal(raw, eraw)
+    np.testing.assert_array_equal(out, eout)
+
+
 # --------------------------------------------------------- coherent beamformer
 def _cb_scales(F, S, A, ts, level=32.0):
     # CoherentBeamformerTester.cu:224-242
