@@ -165,9 +165,7 @@ fpat_stats_partial(const uint32_t* __restrict__ tm, long long* __restrict__ part
 // (chunk of kFusedHeaps heaps, antenna, channel): per heap it loads the
 // channel's 256 samples x 2 pols (16 bytes a lane), writes the two pols'
 // 512-byte runs and adds the sums of x, x^2, x^3, x^4 over re and im with
-// dot-product instructions: sdot4 for x and x^2; for x^3 and x^4 the values
-// are sign-extended to 16-bit pairs (v_perm), squared with a packed 16-bit
-// multiply (x^2 <= 2^14 fits) and summed by sdot2 / udot2.  Bounds per lane
+// dot-product instructions (power_sums).  Bounds per lane
 // and pol over one chunk: |sum x^3| <= 16 heaps x 8 values x 2^21 = 2^28 and
 // a heap's x^4 sum <= 8 x 2^28 = 2^31 (unsigned), so the 32-bit partials are
 // exact; the wave reduction and the x^4 total run in 64 bits.  Partials go
@@ -177,24 +175,6 @@ fpat_stats_partial(const uint32_t* __restrict__ tm, long long* __restrict__ part
 // scratch array.
 constexpr int kFusedHeaps = 16;
 constexpr int kFusedHeapsMax = 64;
-
-typedef short sw_short2 __attribute__((ext_vector_type(2)));
-typedef unsigned short sw_ushort2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ void power_sums(uint32_t x, int& s1, int& s2, int& s3, uint32_t& s4)
-{
-    s1 = __builtin_amdgcn_sdot4((int)x, 0x01010101, s1, false);
-    s2 = __builtin_amdgcn_sdot4((int)x, (int)x, s2, false);
-    // [x0, x2] and [x1, x3] as sign-extended 16-bit pairs (selector 8 / 9
-    // replicate the sign bits of bytes 1 / 3)
-    const sw_short2 e0 = __builtin_bit_cast(sw_short2, __builtin_amdgcn_perm(x << 8, x << 8, 0x09030801u));
-    const sw_short2 e1 = __builtin_bit_cast(sw_short2, __builtin_amdgcn_perm(x, x, 0x09030801u));
-    const sw_short2 q0 = e0 * e0, q1 = e1 * e1;
-    s3 = __builtin_amdgcn_sdot2(q0, e0, s3, false);
-    s3 = __builtin_amdgcn_sdot2(q1, e1, s3, false);
-    s4 = __builtin_amdgcn_udot2(__builtin_bit_cast(sw_ushort2, q0), __builtin_bit_cast(sw_ushort2, q0), s4, false);
-    s4 = __builtin_amdgcn_udot2(__builtin_bit_cast(sw_ushort2, q1), __builtin_bit_cast(sw_ushort2, q1), s4, false);
-}
 
 __device__ __forceinline__ long long wave_sum(long long v)
 {

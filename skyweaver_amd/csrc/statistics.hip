@@ -23,6 +23,13 @@ constexpr int kThreads = 256;
 
 // Partial sums over the rows of one time chunk of one channel.
 // part layout: [chunk][f][col][4] int64.
+//
+// HBM-bound: a thread reads one 16-byte group (8 columns) of every R-th row,
+// four rows' loads in flight.  The rows are taken in pairs: a column's words
+// of two rows make one word of four of its values, which power_sums adds with
+// ten instructions.  (Value by value, with 64-bit x^4 sums, the kernel was
+// bound by the VALU: 64 channels x 16384 samples x 64 antennas took 118 us
+// (2.3 TB/s).)
 __global__ void __launch_bounds__(kThreads)
 stats_partial(const uint4* __restrict__ ftpa, long long* __restrict__ part,
               int nchans, int nsamples, int pa, int rows_per_chunk)
@@ -34,37 +41,44 @@ stats_partial(const uint4* __restrict__ ftpa, long long* __restrict__ part,
     const int tid   = threadIdx.x;
     const int g     = tid % G;
     const int r     = tid / G;
-    // int32 partials are flushed to int64 every 256 rows: |x+y| <= 2^8,
-    // x^2+y^2 <= 2^15, |x^3+y^3| <= 2^22 per row.
+    // Two pairs of rows (8 values a column) are added to 32-bit x^4 sums
+    // (<= 2^31) and flushed; the x^3 sums (|4 values| <= 2^23 a pair) and the
+    // x^2 sums every 64 times that (<= 2^30); the x sums fit 32 bits.
     int s1[8], s2p[8], s3p[8];
-    long long s2[8], s3[8], s4[8];
+    long long s2[8], s3[8];
+    unsigned long long s4[8];
 #pragma unroll
     for(int j = 0; j < 8; ++j) {
         s1[j] = 0; s2p[j] = 0; s3p[j] = 0; s2[j] = 0; s3[j] = 0; s4[j] = 0;
     }
+    // rows a and b of the group: four values of each of its columns
+    auto pair = [&](const uint4& a, const uint4& b, uint32_t (&q4)[8]) {
+        const uint32_t wa[4] = {a.x, a.y, a.z, a.w}, wb[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+        for(int q = 0; q < 4; ++q) {
+            power_sums(__builtin_amdgcn_perm(wb[q], wa[q], 0x05040100u), s1[2 * q], s2p[2 * q], s3p[2 * q], q4[2 * q]);
+            power_sums(__builtin_amdgcn_perm(wb[q], wa[q], 0x07060302u), s1[2 * q + 1], s2p[2 * q + 1],
+                       s3p[2 * q + 1], q4[2 * q + 1]);
+        }
+    };
     const int t0 = chunk * rows_per_chunk;
     const int t1 = min(nsamples, t0 + rows_per_chunk);
     if(r < R) {
         const uint4* base = ftpa + (size_t)f * nsamples * G + g;
         int iter = 0;
-        for(int t = t0 + r; t < t1; t += R) {
-            const uint4 v = base[(size_t)t * G];
-            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+        for(int t = t0 + r; t < t1; t += 4 * R) {
+            uint4 v[4];
 #pragma unroll
-            for(int q = 0; q < 4; ++q) {
-#pragma unroll
-                for(int h = 0; h < 2; ++h) {
-                    const int j  = q * 2 + h;   // column within the group
-                    const int re = (int)(int8_t)(w[q] >> (16 * h));
-                    const int im = (int)(int8_t)(w[q] >> (16 * h + 8));
-                    const int re2 = re * re, im2 = im * im;
-                    s1[j] += re + im;
-                    s2p[j] += re2 + im2;
-                    s3p[j] += re * re2 + im * im2;
-                    s4[j] += (long long)(re2 * re2 + im2 * im2);
-                }
+            for(int k = 0; k < 4; ++k) {
+                v[k] = make_uint4(0, 0, 0, 0);  // adds nothing to any sum
+                if(t + k * R < t1) v[k] = base[(size_t)(t + k * R) * G];
             }
-            if(++iter == 256) {
+            uint32_t q4[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+            pair(v[0], v[1], q4);
+            pair(v[2], v[3], q4);
+#pragma unroll
+            for(int j = 0; j < 8; ++j) s4[j] += q4[j];
+            if(++iter == 64) {
 #pragma unroll
                 for(int j = 0; j < 8; ++j) {
                     s2[j] += s2p[j]; s2p[j] = 0;
@@ -77,26 +91,22 @@ stats_partial(const uint4* __restrict__ ftpa, long long* __restrict__ part,
 #pragma unroll
     for(int j = 0; j < 8; ++j) { s2[j] += s2p[j]; s3[j] += s3p[j]; }
 
-    // block reduction over the R row lanes, one moment at a time
+    // block reduction over the R row lanes, one moment at a time; a thread
+    // sums a column
     __shared__ long long red[kThreads * 8];
-    long long* out = part + (((size_t)chunk * nchans + f) * pa + (size_t)g * 8) * 4;
+    long long* out = part + ((size_t)chunk * nchans + f) * pa * 4;
 #pragma unroll
     for(int m = 0; m < 4; ++m) {
+        if(m) __syncthreads();
 #pragma unroll
-        for(int j = 0; j < 8; ++j) {
-            long long v = (m == 0) ? s1[j] : (m == 1) ? s2[j] : (m == 2) ? s3[j] : s4[j];
-            red[tid * 8 + j] = v;
-        }
+        for(int j = 0; j < 8; ++j)
+            red[tid * 8 + j] = (m == 0) ? s1[j] : (m == 1) ? s2[j] : (m == 2) ? s3[j] : (long long)s4[j];
         __syncthreads();
-        if(r == 0) {
-#pragma unroll
-            for(int j = 0; j < 8; ++j) {
-                long long acc = 0;
-                for(int rr = 0; rr < R; ++rr) acc += red[(rr * G + g) * 8 + j];
-                out[j * 4 + m] = acc;
-            }
+        for(int c = tid; c < pa; c += kThreads) {
+            long long acc = 0;
+            for(int rr = 0; rr < R; ++rr) acc += red[rr * pa + c];
+            out[c * 4 + m] = acc;
         }
-        __syncthreads();
     }
 }
 
@@ -106,6 +116,7 @@ __global__ void stats_finalize(const long long* __restrict__ part, float4* __res
     const int c = blockIdx.x * blockDim.x + threadIdx.x;  // f*pa + col
     if(c >= ncols_total) return;
     long long S1 = 0, S2 = 0, S3 = 0, S4 = 0;
+#pragma unroll 8
     for(int k = 0; k < nchunks; ++k) {
         const long long* p = part + ((size_t)k * ncols_total + c) * 4;
         S1 += p[0]; S2 += p[1]; S3 += p[2]; S4 += p[3];
@@ -163,7 +174,8 @@ extern "C" int sw_statistics(const void* d_ftpa, float* d_stats, int nchans, int
                        static_cast<long long*>(ws), nchans, nsamples, pa, rows);
     SW_LAUNCH_CHECK();
     const int ncols = nchans * pa;
-    hipLaunchKernelGGL(sw::stats_finalize, dim3((ncols + 255) / 256), dim3(256), 0,
+    // one wave per workgroup: the columns are few, spread over the CUs
+    hipLaunchKernelGGL(sw::stats_finalize, dim3((ncols + 63) / 64), dim3(64), 0,
                        sw::as_stream(stream), static_cast<const long long*>(ws),
                        reinterpret_cast<float4*>(d_stats), chunks, ncols,
                        (long long)nsamples * 2);

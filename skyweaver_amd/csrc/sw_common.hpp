@@ -66,6 +66,28 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void* base, 
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
 }
 
+// Power sums of the four int8 values of x into 32-bit partials, with dot
+// products: x and x^2 by sdot4; for x^3 and x^4 the values are sign-extended
+// to 16-bit pairs, squared with a packed 16-bit multiply (x^2 <= 2^14 fits)
+// and summed by sdot2 / udot2.
+typedef short sw_short2 __attribute__((ext_vector_type(2)));
+typedef unsigned short sw_ushort2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ void power_sums(uint32_t x, int& s1, int& s2, int& s3, uint32_t& s4)
+{
+    s1 = __builtin_amdgcn_sdot4((int)x, 0x01010101, s1, false);
+    s2 = __builtin_amdgcn_sdot4((int)x, (int)x, s2, false);
+    // [x0, x2] and [x1, x3] as sign-extended 16-bit pairs (selector 8 / 9
+    // replicate the sign bits of bytes 1 / 3)
+    const sw_short2 e0 = __builtin_bit_cast(sw_short2, __builtin_amdgcn_perm(x << 8, x << 8, 0x09030801u));
+    const sw_short2 e1 = __builtin_bit_cast(sw_short2, __builtin_amdgcn_perm(x, x, 0x09030801u));
+    const sw_short2 q0 = e0 * e0, q1 = e1 * e1;
+    s3 = __builtin_amdgcn_sdot2(q0, e0, s3, false);
+    s3 = __builtin_amdgcn_sdot2(q1, e1, s3, false);
+    s4 = __builtin_amdgcn_udot2(__builtin_bit_cast(sw_ushort2, q0), __builtin_bit_cast(sw_ushort2, q0), s4, false);
+    s4 = __builtin_amdgcn_udot2(__builtin_bit_cast(sw_ushort2, q1), __builtin_bit_cast(sw_ushort2, q1), s4, false);
+}
+
 struct cf32 {
     float x, y;
 };

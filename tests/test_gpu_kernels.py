@@ -75,6 +75,27 @@ def test_statistics_parity(sw, orc, dev, F, T, A):
     np.testing.assert_allclose(got, exp, rtol=1e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize("F,T,A", [(1, 2, 4), (2, 1001, 12), (2048, 300, 4), (1, 70001, 64), (1, 700, 1024)])
+def test_statistics_sums_exact(sw, orc, dev, F, T, A):
+    """Odd row counts, idle row lanes, a chunk past the 32-bit sums' flush and the values that
+    reach their bounds: every moment to the float rounding of the FP64 closed form."""
+    v = _rand_c8((F, T, 2, A), 4 + T, sigma=20.0)
+    v[0, :, 0, 0] = -128
+    v[0, ::2, 0, 0] = 127
+    d_st = _empty((F, 2, A, 4), np.float32, dev)
+    sw.statistics(_to_dev(v, dev), d_st, F, T, A)
+    got = _to_host(d_st).astype(np.float64)
+    x = v[:2].astype(np.float64)
+    s = [(x ** k).sum(axis=(1, 4)) for k in (1, 2, 3, 4)]  # exact in float64
+    n = 2.0 * T
+    m = s[0] / n
+    m2 = s[1] - m * s[0]
+    m3 = s[2] - 3 * m * s[1] + 2 * m * m * s[0]
+    m4 = s[3] - 4 * m * s[2] + 6 * m * m * s[1] - 3 * m ** 3 * s[0]
+    exp = np.stack((m, np.sqrt(m2 / (n - 1)), np.sqrt(n) * m3 / m2 ** 1.5, n * m4 / (m2 * m2) - 3), -1)
+    np.testing.assert_allclose(got[:2], exp, rtol=2e-7, atol=1e-9)
+
+
 @pytest.mark.parametrize("H,A_in,A_out,F", [(16, 16, 64, 64), (37, 57, 64, 5), (3, 80, 80, 8), (33, 4, 16, 16)])
 def test_transpose_fpat_stats_fused(sw, orc, dev, H, A_in, A_out, F):
     """The fused TAFTP -> FPAT transpose + statistics equals the separate
