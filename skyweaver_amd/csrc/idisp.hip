@@ -21,18 +21,16 @@
 // at most 256 biased bytes; longer sums (nchans * ts > 256) are flushed into
 // 32-bit accumulators.
 //
-// Matrix-core form (idisp_mfma_kernel, used whenever nchans % 4 == 0 and the
-// rows of one DM fit the stage): one DM's channel sum is a chain of
+// Matrix-core form (idisp_tile, used whenever nchans % 4 == 0 and the rows of
+// one DM fit the stage): one DM's channel sum is a chain of
 // v_mfma_i32_16x16x64_i8 products.  The B operand carries data: lane
 // (n, g) = (l % 16, l / 16) holds the 16 beam bytes [b0, b0 + 16) of channel
 // f0 + g at the input row of output sample n.  The A operand is a constant
 // selector, row m holding a single 1 at byte m of every k-group, so
 // C[m][n] = sum over g of beam b0 + m of channel f0 + g at sample n: four
 // channels x 16 beams x 16 samples per instruction, summed exactly in int32.
-// For tscrunch <= 2 with 16-byte rows the same products run in
-// idisp_dma_kernel: 16 waves of one DM each, 32 output samples per
-// workgroup, each quad of channels loaded straight into one of two LDS stage
-// buffers while the other quad's products run.
+// It runs as idisp_dma_kernel (tscrunch <= 2, 32 output samples per
+// workgroup) and idisp_mfma_kernel (tscrunch 3-8, 16 samples).
 #include "sw_common.hpp"
 
 #include <algorithm>
@@ -55,8 +53,10 @@ struct sw_idisp {
     int dpw = 2, tt = 16, rows_cap = 0;
     bool wide = false;
     bool mfma = false;                // matrix-core kernel (else the 16-bit-lane one)
+    bool small = false;               // its small form: 8 waves, two workgroups per CU
     std::vector<int2> tiles;          // (first DM, count)
     int* d_delays = nullptr;
+    uint8_t* d_rel = nullptr;         // matrix-core form: [ntiles][F][waves] delta_max - delta
     int2* d_span = nullptr;           // [ntiles][F] (delta_min, delta_max)
     int2* d_tiles = nullptr;
 };
@@ -244,372 +244,241 @@ constexpr int kRowsCap = 256;  // staged rows per channel: 64 KB of LDS
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 
-constexpr int kMfWaves = 8;    // waves per workgroup
-constexpr int kMfDpw   = 2;    // DMs per wave
-constexpr int kDmaWaves = 16;  // waves (one DM each) per workgroup of the double-buffered form
-constexpr int kMfRows  = 128;  // staged rows per channel
-constexpr int kMfPitch = 144;  // bytes between staged rows: 128 B of beams + 16;
-                               // 16 consecutive rows start on distinct banks
+constexpr int kMfRows  = 128;   // staged rows per channel, 16 waves (one DM each) per workgroup
+constexpr int kMfWaves = 16;
+constexpr int kSmRows  = 64;    // the same where 8 DMs' rows are few: 8 waves, two workgroups per CU
+constexpr int kSmWaves = 8;
+constexpr int kMfTabCh = 512;   // channels whose delay tables are held in LDS at a time
+constexpr int kMfMaxTs = 8;
 
-template <typename P>
-__device__ __forceinline__ P zero_piece()
-{
-    if constexpr(std::is_same<P, uint4>::value)
-        return make_uint4(0, 0, 0, 0);
-    else
-        return 0u;
-}
+// Rows that a channel's stage of `rcap` rows holds at tscrunch ts (a whole
+// number of rows per phase of ts).
+constexpr int id_stage_rows(int rcap, int ts) { return rcap / ts * ts; }
 
-// A workgroup of NW waves owns TT = 16 NTT output samples, 128 bytes of beams
-// (a chunk) and a tile of up to NW * DPW consecutive DMs (wave w takes the
-// tile's DMs w, w + NW, ...).  Per quad of channels it stages into LDS the
-// union of the rows its DMs read, [in0 - max delay, in0 + TT ts - min delay)
-// per channel, while the rows of the next two quads are loaded into
-// registers.  Input byte (t, f, b) lives at t * stride_t + f * stride_f + b
-// (TFB or FTB).
-//
 // Work items are dealt to the 8 XCDs in contiguous runs, and a run is walked
 // in groups of kIdTbGroup time blocks x kIdTileGroup DM tiles of one chunk:
 // the 32 workgroups that one XCD runs together read overlapping rows (next
 // time blocks; DM tiles of neighbouring delays), which its L2 then serves.
 constexpr int kIdTbGroup = 8, kIdTileGroup = 4;
 
-template <int NW, int DPW, int NTT, int RCAP, bool VEC16, bool PF>
-__global__ void __launch_bounds__(NW * 64, PF ? 1 : 2)
-idisp_mfma_kernel(const int8_t* __restrict__ in, int8_t* __restrict__ tdb, const int* __restrict__ delays,
-                  const int2* __restrict__ span, const int2* __restrict__ tiles, int ntiles, int nchunks,
-                  int ntb, long w0, long nwork, int nchans, int W, int ndms, int ts, int max_delay,
-                  long nsamples, int nout, float scale, long stride_t, long stride_f)
-{
-    constexpr int NT    = NW * 64;
-    constexpr int TT    = 16 * NTT;
-    constexpr int PIECE = VEC16 ? 16 : 4;  // bytes per staging load
-    constexpr int PPR   = 128 / PIECE;     // loads per staged row
-    static_assert((RCAP * PPR) % NT == 0, "a thread's loads must stay in one channel each");
-    constexpr int NPF = 4 * RCAP * PPR / NT;
-    using P = typename std::conditional<VEC16, uint4, uint32_t>::type;
-    __shared__ __attribute__((aligned(16))) int8_t stage[4 * RCAP * kMfPitch];
+struct IdArgs {
+    const int8_t* in;
+    int8_t* tdb;
+    const uint8_t* rel;  // [tile][channel][NW]: the tile's largest delay in the channel less the DM's
+    const int2* span;    // [tile][channel]: the tile's smallest and largest delay
+    const int2* tiles;   // [tile]: first DM, DMs
+    int ntiles, chunk0, nchunks, ntb;
+    long w0, nwork;
+    int nchans, W, ndms, max_delay;
+    long nsamples;
+    int nout;
+    float scale;
+    long stride_t, stride_f;  // bytes
+};
 
-    const long per = (nwork + 7) / 8;
-    const long wl  = (long)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    if(wl >= nwork) return;  // whole workgroup, before any barrier
-    const long w = w0 + wl;
-    constexpr int GRP = kIdTbGroup * kIdTileGroup;
-    const int gi = (int)(w % GRP);
-    const long rest  = w / GRP;
-    const int chunk  = (int)(rest % nchunks);
-    const long blk   = rest / nchunks;
-    const int ntbb   = (ntb + kIdTbGroup - 1) / kIdTbGroup;
-    const int tb     = (int)(blk % ntbb) * kIdTbGroup + gi % kIdTbGroup;
-    const int tile   = (int)(blk / ntbb) * kIdTileGroup + gi / kIdTbGroup;
-    if(tb >= ntb || tile >= ntiles) return;  // whole workgroup, before any barrier
-    const int2 td    = tiles[tile];
-    const int t0     = tb * TT;
-    const long in0   = (long)max_delay + (long)t0 * ts;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int n = lane & 15, g = lane >> 4;
-    const int b0 = chunk * 128;
-    const int nq = nchans / 4;
-    const int2* tspan = span + (size_t)tile * nchans;
-
-    P preA[NPF], preB[NPF];
-    auto fetch = [&](int q, P (&pre)[NPF]) {
-#pragma unroll
-        for(int k = 0; k < NPF; ++k) {
-            const int s = threadIdx.x + NT * k;
-            const int j = (NT * k) / (RCAP * PPR);  // compile-time: NT divides RCAP * PPR
-            const int r = (s / PPR) % RCAP, c = s % PPR;
-            const int2 spj = tspan[4 * q + j];
-            const long row = in0 - spj.y + r;
-            const int b = b0 + c * PIECE;
-            P v = zero_piece<P>();
-            if(r < TT * ts + spj.y - spj.x && b < W && row < nsamples)
-                v = *reinterpret_cast<const P*>(in + row * stride_t + (long)(4 * q + j) * stride_f + b);
-            pre[k] = v;
-        }
-    };
-    // only the rows the quad's DMs read are written: a channel of quad q
-    // needs TT ts + (its span of delays) rows, often far fewer than RCAP
-    auto stash = [&](int q, const P (&pre)[NPF]) {
-#pragma unroll
-        for(int k = 0; k < NPF; ++k) {
-            const int s = threadIdx.x + NT * k;
-            const int j = (NT * k) / (RCAP * PPR);
-            const int r = (s / PPR) % RCAP, c = s % PPR;
-            const int2 spj = tspan[4 * q + j];
-            if(r < TT * ts + spj.y - spj.x)
-                *reinterpret_cast<P*>(stage + (j * RCAP + r) * kMfPitch + c * PIECE) = pre[k];
-        }
-    };
-    // this lane's channel of quad q: its span and the delays of the wave's DMs
-    auto lane_delays = [&](int q, int2& spg, int (&dly)[DPW]) {
-        spg = tspan[4 * q + g];
-#pragma unroll
-        for(int jd = 0; jd < DPW; ++jd) {
-            const int dl = wave + NW * jd;
-            dly[jd] = dl < td.y ? delays[(size_t)(td.x + dl) * nchans + 4 * q + g] : spg.y;
-        }
-    };
-
-    v4i sel = {0, 0, 0, 0};
-    sel[n >> 2] = 1 << (8 * (n & 3));
-    v4i acc[DPW][NTT][8];
-#pragma unroll
-    for(int jd = 0; jd < DPW; ++jd)
-#pragma unroll
-        for(int tt = 0; tt < NTT; ++tt)
-#pragma unroll
-            for(int bg = 0; bg < 8; ++bg) acc[jd][tt][bg] = v4i{0, 0, 0, 0};
-
-    auto products = [&](int2 spc, const int (&dc)[DPW]) {
-#pragma unroll
-        for(int jd = 0; jd < DPW; ++jd) {
-            if(wave + NW * jd >= td.y) continue;  // wave-uniform
-            const int8_t* base = stage + (g * RCAP + spc.y - dc[jd] + n * ts) * kMfPitch;
-#pragma unroll
-            for(int tt = 0; tt < NTT; ++tt)
-                for(int s = 0; s < ts; ++s) {
-                    const int8_t* rp = base + (tt * 16 * ts + s) * kMfPitch;
-                    if constexpr(!PF) {
-                        // the row's eight reads in flight together (the
-                        // scheduler would otherwise issue them one by one)
-                        v4i bv[8];
-#pragma unroll
-                        for(int bg = 0; bg < 8; ++bg) bv[bg] = *reinterpret_cast<const v4i*>(rp + bg * 16);
-                        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                        for(int bg = 0; bg < 8; ++bg)
-                            acc[jd][tt][bg] =
-                                __builtin_amdgcn_mfma_i32_16x16x64_i8(sel, bv[bg], acc[jd][tt][bg], 0, 0, 0);
-                    } else {
-#pragma unroll
-                        for(int bg = 0; bg < 8; ++bg) {
-                            const v4i b = *reinterpret_cast<const v4i*>(rp + bg * 16);
-                            acc[jd][tt][bg] = __builtin_amdgcn_mfma_i32_16x16x64_i8(sel, b, acc[jd][tt][bg], 0, 0, 0);
-                        }
-                    }
-                }
-        }
-    };
-
-    if constexpr(!PF) {
-        // no register prefetch (two workgroups share a CU and hide each
-        // other's loads): stage quad q, then its products
-        for(int q = 0; q < nq; ++q) {
-            int2 spc;
-            int dc[DPW];
-            lane_delays(q, spc, dc);  // issued with the row loads, before any wait
-            fetch(q, preA);
-            __syncthreads();  // the previous quad's reads are done
-            stash(q, preA);
-            __syncthreads();
-            products(spc, dc);
-        }
-    } else {
-    // quads alternate between two register sets: A holds even quads, B odd
-    int2 spA, spB;
-    int dA[DPW], dB[DPW];
-    fetch(0, preA);
-    lane_delays(0, spA, dA);
-    if(nq > 1) {
-        fetch(1, preB);
-        lane_delays(1, spB, dB);
-    }
-    for(int q = 0; q < nq; q += 2) {
-        {
-            __syncthreads();  // the previous quad's reads are done
-            stash(q, preA);
-            __syncthreads();
-            const int2 spc = spA;
-            int dc[DPW];
-#pragma unroll
-            for(int jd = 0; jd < DPW; ++jd) dc[jd] = dA[jd];
-            if(q + 2 < nq) {  // in flight during two quads' products
-                fetch(q + 2, preA);
-                lane_delays(q + 2, spA, dA);
-            }
-            products(spc, dc);
-        }
-        if(q + 1 < nq) {
-            __syncthreads();
-            stash(q + 1, preB);
-            __syncthreads();
-            const int2 spc = spB;
-            int dc[DPW];
-#pragma unroll
-            for(int jd = 0; jd < DPW; ++jd) dc[jd] = dB[jd];
-            if(q + 3 < nq) {
-                fetch(q + 3, preB);
-                lane_delays(q + 3, spB, dB);
-            }
-            products(spc, dc);
-        }
-    }
-    }
-
-    // C lane (n, g), register r: beam b0 + 16 bg + 4 g + r at sample t0 + 16 tt + n
-#pragma unroll
-    for(int jd = 0; jd < DPW; ++jd) {
-        const int dl = wave + NW * jd;
-        if(dl >= td.y) continue;
-#pragma unroll
-        for(int tt = 0; tt < NTT; ++tt) {
-            const int t = t0 + 16 * tt + n;
-            if(t >= nout) continue;
-            int8_t* o = tdb + ((size_t)t * ndms + td.x + dl) * W;
-#pragma unroll
-            for(int bg = 0; bg < 8; ++bg) {
-                const int b = b0 + 16 * bg + 4 * g;
-                if(b >= W) continue;
-                const v4i a = acc[jd][tt][bg];
-                const uint32_t packed = (uint32_t)(uint8_t)id_quant(a[0], scale) |
-                                        ((uint32_t)(uint8_t)id_quant(a[1], scale) << 8) |
-                                        ((uint32_t)(uint8_t)id_quant(a[2], scale) << 16) |
-                                        ((uint32_t)(uint8_t)id_quant(a[3], scale) << 24);
-                *reinterpret_cast<uint32_t*>(o + b) = packed;
-            }
-        }
-    }
-}
-
-// Double-buffered form: a workgroup of NW = 16 waves (one DM each) owns TT =
-// 16 NTT output samples, a 128-byte chunk of beams and a tile of up to 16
-// consecutive DMs.  Each quad's rows go from global memory straight into one
-// of two LDS stage buffers (global_load_lds_dwordx4: lane L of a wave's load
-// writes the 16-byte slot L of a 1 KB block) while the previous quad's
-// products read the other buffer, one barrier per quad and no staging
-// registers.  The stage keeps idisp_mfma_kernel's layout (row pitch
-// kMfPitch: nine 16-byte slots, the ninth padding that no lane loads), and
-// the products read it exactly as there.  The two buffers take 144 KB: one
-// workgroup of 16 waves per CU.  Slots that no lane loads (padding, rows
-// past the tile's span or the input, beams past W) keep stale bytes: no
-// stored output reads them (rows past the span are read by no DM of the
-// tile, rows past the input feed only output samples >= nout, beams past W
-// only beams >= W, and the one-hot products sum each beam from its own
+// A workgroup of NW waves owns 16 NTT output samples, 128 bytes of beams (a
+// chunk) and a tile of up to NW consecutive DMs, one per wave.  Per quad of
+// channels the union of the rows its DMs read, [in0 - max delay, in0 +
+// 16 NTT TS - min delay) per channel, goes from global memory straight into
+// one of two LDS stage buffers (global_load_lds_dwordx4: lane L of a wave's
+// load writes the 16-byte slot L of a 1 KB block, eight rows) while the
+// previous quad's products read the other, one barrier per quad.  Input byte
+// (t, f, b) lives at t * stride_t + f * stride_f + b (TFB or FTB).  NBG: 16-beam
+// groups of the chunk (4 where only 64 bytes of it hold beams).
+//
+// Stage layout: rows of 128 bytes.  Logical row r lies at row (r mod TS) RP +
+// r / TS, so that the 16 rows TS apart that one read takes are neighbours,
+// and 16-byte piece c of stored row r' in slot c ^ ((r' / 2) mod 8): any 16
+// consecutive rows then start on distinct banks.  (Rows TS apart put a read
+// on 16 / TS banks: 300 DMs x 404 beams x 64 channels x 3000 samples at
+// tscrunch 4 took 5.4 ms.)
+//
+// What bounds it: the round trip of a quad's row loads, issued after the
+// barrier that frees their buffer, together with the LDS reads of the
+// products, 8 cycles of the CU per 1024 channel sums.  1024 DMs x 512 beams x
+// 256 channels x 4096 samples take 9.8 ms (5.6e13 sums/s), 6.6 ms without the
+// loads, 8.4 ms without the products.  A load therefore costs no address
+// arithmetic: per channel a table in LDS, filled once per kMfTabCh channels,
+// holds where its rows begin and end, a buffer resource over them takes the
+// lane's fixed offset and its range check stands for the row tests, and a
+// wave loads rows of one channel only.  (With 64-bit addresses and the tests
+// formed per load, and the delays loaded per quad, the VALU was busy with
+// them for two thirds of the time: 13.5 ms.  Touching the rows of the quad
+// after the next ahead of time, 16.5 ms with that form.)
+//
+// Slots past the tile's rows or the input are zero or keep stale bytes, those
+// past W keep stale bytes, and a row's last piece may hold the next row's
+// first bytes: no stored output reads them (rows past the span are read by no
+// DM of the tile, rows past the input feed only output samples >= nout, beams
+// past W only beams >= W, and the one-hot products sum each beam from its own
 // bytes).
-template <int NW, int NTT, int RCAP>
-__global__ void __launch_bounds__(NW * 64, 1)
-idisp_dma_kernel(const int8_t* __restrict__ in, int8_t* __restrict__ tdb, const int* __restrict__ delays,
-                 const int2* __restrict__ span, const int2* __restrict__ tiles, int ntiles, int nchunks,
-                 int ntb, long w0, long nwork, int nchans, int W, int ndms, int ts, int max_delay,
-                 long nsamples, int nout, float scale, long stride_t, long stride_f)
+template <int NW, int NTT, int NBG, int RCAP, int TS, bool BIG>
+__device__ __forceinline__ void idisp_tile(const IdArgs& p)
 {
     constexpr int TT  = 16 * NTT;
-    constexpr int SPR = kMfPitch / 16;  // 16-byte slots per staged row
-    constexpr int SPC = RCAP * SPR;     // slots per channel
-    static_assert(kMfPitch % 16 == 0 && SPC % 64 == 0, "a wave's 64-slot block stays in one channel");
-    constexpr int NBLK = 4 * SPC / 64;          // 1 KB blocks per quad
-    constexpr int NB   = (NBLK + NW - 1) / NW;  // blocks per wave per quad (the last round partial)
-    constexpr int QB   = 4 * RCAP * kMfPitch;
+    constexpr int RP  = RCAP / TS;       // stored rows per phase
+    constexpr int QB  = 4 * RCAP * 128;
+    static_assert(RCAP == 8 * NW, "a wave loads eight rows (1 KB) of each channel of a quad");
     // two arrays, not one: the compiler then knows that a buffer's reads do
     // not touch the loads in flight into the other (with one array it waits
     // for every row load before any read)
     __shared__ __attribute__((aligned(16))) int8_t stage0[QB];
     __shared__ __attribute__((aligned(16))) int8_t stage1[QB];
+    __shared__ __attribute__((aligned(16))) int4 tab[kMfTabCh];  // offset of the first row (64 bits), bytes, rows
+    __shared__ __attribute__((aligned(16))) uint8_t tab_rel[kMfTabCh * NW];  // [channel][wave]: rows to the DM's first
 
-    const long per = (nwork + 7) / 8;
+    const long per = (p.nwork + 7) / 8;
     const long wl  = (long)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    if(wl >= nwork) return;  // whole workgroup, before any barrier
-    const long w = w0 + wl;
+    if(wl >= p.nwork) return;  // whole workgroup, before any barrier
+    const long w = p.w0 + wl;
     constexpr int GRP = kIdTbGroup * kIdTileGroup;
     const int gi = (int)(w % GRP);
     const long rest  = w / GRP;
-    const int chunk  = (int)(rest % nchunks);
-    const long blk   = rest / nchunks;
-    const int ntbb   = (ntb + kIdTbGroup - 1) / kIdTbGroup;
+    const int chunk  = p.chunk0 + (int)(rest % p.nchunks);
+    const long blk   = rest / p.nchunks;
+    const int ntbb   = (p.ntb + kIdTbGroup - 1) / kIdTbGroup;
     const int tb     = (int)(blk % ntbb) * kIdTbGroup + gi % kIdTbGroup;
     const int tile   = (int)(blk / ntbb) * kIdTileGroup + gi / kIdTbGroup;
-    if(tb >= ntb || tile >= ntiles) return;  // whole workgroup, before any barrier
-    const int2 td    = tiles[tile];
+    if(tb >= p.ntb || tile >= p.ntiles) return;  // whole workgroup, before any barrier
+    const int2 td    = p.tiles[tile];
     const int t0     = tb * TT;
-    const long in0   = (long)max_delay + (long)t0 * ts;
+    const long in0   = (long)p.max_delay + (long)t0 * TS;
     const int lane = threadIdx.x & 63;
-    // the wave index made uniform: the spans below are scalar loads whose
-    // waits do not hold back the row loads
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 15, g = lane >> 4;
     const int b0 = chunk * 128;
-    const int nq = nchans / 4;
-    const int2* tspan = span + (size_t)tile * nchans;
-    const bool active = wv < td.y;  // this wave's DM is in the tile
+    const bool active = wv < td.y;        // this wave's DM is in the tile
+    const bool ragged = (p.W & 15) != 0;  // a row's last piece may pass the input's end
 
-    // quad q's rows into stg: block k NW + wave of the quad, slot lane
-    auto issue = [&](int q, int8_t* stg) {
-        // the quad's four spans: scalar loads in flight together
-        const int2 sq0 = tspan[4 * q], sq1 = tspan[4 * q + 1], sq2 = tspan[4 * q + 2], sq3 = tspan[4 * q + 3];
-        int ln = lane;
-        asm volatile("" : "+v"(ln));  // the slot arithmetic is redone per quad, not held in registers
+    // Staging: wave w loads 8-row blocks w mod WPC + WPC k (k < 4) of channel
+    // w / WPC of every quad, so a quad costs a wave one table entry.  A lane's
+    // offsets within a channel's rows are the same for all quads.
+    constexpr int WPC = NW / 4;
+    const int sc = wv / WPC;  // the wave's channel of a quad
+    auto stored_row = [&](int k) { return (wv % WPC + WPC * k) * 8 + (lane >> 3); };
+    auto piece = [&](int rs) { return b0 + (((lane & 7) ^ ((rs >> 1) & 7)) << 4); };
+    uint32_t voff[4];
 #pragma unroll
-        for(int k = 0; k < NB; ++k) {
-            const int bk = k * NW + wv;  // wave-uniform
-            if(NBLK % NW != 0 && bk >= NBLK) break;
-            const int j  = bk * 64 / SPC;  // channel of the quad, wave-uniform
-            const int s  = bk * 64 - j * SPC + ln;
-            const int r = s / SPR, c = s % SPR;
-            const int2 spj = j == 0 ? sq0 : j == 1 ? sq1 : j == 2 ? sq2 : sq3;
-            const long row = in0 - spj.y + r;
-            const int b = b0 + c * 16;
-            if(c < 8 && r < TT * ts + spj.y - spj.x && b < W && row < nsamples)
-                __builtin_amdgcn_global_load_lds(in + row * stride_t + (long)(4 * q + j) * stride_f + b,
-                                                 (__attribute__((address_space(3))) void*)(stg + bk * 1024), 16,
-                                                 0, 0);
+    for(int k = 0; k < 4; ++k) {
+        const int rs = stored_row(k), b = piece(rs);
+        const bool in = rs < RP * TS && b < p.W;
+        voff[k] = in ? (uint32_t)(rs % RP * TS + rs / RP) * (uint32_t)p.stride_t + b : 0xFFFFFFF0u;
+    }
+    // quad q's rows into stg: through a buffer resource that ends with the
+    // channel's last row (a load past it stores zeros), or where 32 bits do
+    // not span the stage's rows (BIG) by 64-bit addresses
+    auto issue = [&](int f0, int q, int8_t* stg) {
+        const int4 e = tab[4 * q + sc];
+        const unsigned lo = __builtin_amdgcn_readfirstlane(e.x), hi = __builtin_amdgcn_readfirstlane(e.y);
+        const int nr = __builtin_amdgcn_readfirstlane(e.w);
+        const int8_t* src = p.in + ((unsigned long)hi << 32 | lo);
+        if constexpr(BIG) {
+#pragma unroll
+            for(int k = 0; k < 4; ++k) {
+                const int rs = stored_row(k), b = piece(rs), r = rs % RP * TS + rs / RP;
+                const bool end = ragged && f0 + 4 * q + sc == p.nchans - 1 && r == nr - 1;
+                if(rs < RP * TS && r < nr && (end ? b + 16 <= p.W : b < p.W))
+                    __builtin_amdgcn_global_load_lds(
+                        src + (unsigned long)r * p.stride_t + b,
+                        (__attribute__((address_space(3))) void*)(stg + (sc * RCAP + (wv % WPC + WPC * k) * 8) * 128),
+                        16, 0, 0);
+            }
+        } else {
+            const auto rs = buffer_rsrc(src, __builtin_amdgcn_readfirstlane(e.z));
+#pragma unroll
+            for(int k = 0; k < 4; ++k)
+                if(TS > 1 || (wv % WPC + WPC * k) * 8 < nr)  // uniform
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                        rs, (__attribute__((address_space(3))) void*)(stg + (sc * RCAP + (wv % WPC + WPC * k) * 8) * 128),
+                        16, voff[k], 0, 0, 0);
         }
     };
-    // this lane's channel of quad q: its span and the delay of the wave's DM
-    // (a wave past the tile's DMs loads the last DM's and does not use it, so
-    // neither load waits on the other)
-    const int dmw = td.x + min(wv, td.y - 1);
-    auto lane_delay = [&](int q, int2& spg, int& dly) {
-        spg = tspan[4 * q + g];
-        dly = delays[(size_t)dmw * nchans + 4 * q + g];
+    // the last piece of the input's last row (the last channel's), W mod 16
+    // bytes, by words: a whole piece would pass the input's end.  Called once
+    // the wave's loads have arrived, by the wave that loaded the row (its load
+    // of the slot stored zeros).
+    auto finish = [&](int f0, int q, int8_t* stg) {
+        if(!ragged || f0 + 4 * q + 4 < p.nchans || p.W - b0 > 128) return;  // wave-uniform
+        const int r = tab[4 * q + 3].w - 1;
+        const int rs = r % TS * RP + r / TS, c = (p.W - b0) >> 4;
+        if(in0 - p.span[(size_t)tile * p.nchans + p.nchans - 1].y + r != p.nsamples - 1 ||
+           wv != 3 * WPC + rs / 8 % WPC || lane >= (p.W & 15) / 4)
+            return;
+        *reinterpret_cast<uint32_t*>(stg + (3 * RCAP + rs) * 128 + ((c ^ ((rs >> 1) & 7)) << 4) + 4 * lane) =
+            *reinterpret_cast<const uint32_t*>(p.in + (p.nsamples - 1) * p.stride_t +
+                                               (long)(p.nchans - 1) * p.stride_f + b0 + 16 * c + 4 * lane);
     };
 
     v4i sel = {0, 0, 0, 0};
     sel[n >> 2] = 1 << (8 * (n & 3));
-    v4i acc[NTT][8];
+    v4i acc[NTT][NBG];
 #pragma unroll
     for(int tt = 0; tt < NTT; ++tt)
 #pragma unroll
-        for(int bg = 0; bg < 8; ++bg) acc[tt][bg] = v4i{0, 0, 0, 0};
+        for(int bg = 0; bg < NBG; ++bg) acc[tt][bg] = v4i{0, 0, 0, 0};
 
-    auto products = [&](const int8_t* stg, int2 spc, int dc) {
+    auto products = [&](int q, const int8_t* stg) {
         if(!active) return;  // wave-uniform
-        const int8_t* base = stg + (g * RCAP + spc.y - dc + n * ts) * kMfPitch;
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
+        const int n = ln & 15, g = ln >> 4;
+        const int rel = tab_rel[(4 * q + g) * NW + wv];
 #pragma unroll
-        for(int tt = 0; tt < NTT; ++tt)
-            for(int s = 0; s < ts; ++s) {
-                const int8_t* rp = base + (tt * 16 * ts + s) * kMfPitch;
-                v4i bv[8];  // the row's eight reads in flight together
+        for(int s = 0; s < TS; ++s) {
+            const int k = rel + s;
+            const int rs = k % TS * RP + k / TS + n;
+            const int base = (g * RCAP + rs) * 128 + (((rs >> 1) & 7) << 4);
 #pragma unroll
-                for(int bg = 0; bg < 8; ++bg) bv[bg] = *reinterpret_cast<const v4i*>(rp + bg * 16);
+            for(int tt = 0; tt < NTT; ++tt) {
+                v4i bv[NBG];  // the row's reads in flight together
+#pragma unroll
+                for(int bg = 0; bg < NBG; ++bg)
+                    bv[bg] = *reinterpret_cast<const v4i*>(stg + (base ^ (bg << 4)) + tt * 2048);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for(int bg = 0; bg < 8; ++bg)
+                for(int bg = 0; bg < NBG; ++bg)
                     acc[tt][bg] = __builtin_amdgcn_mfma_i32_16x16x64_i8(sel, bv[bg], acc[tt][bg], 0, 0, 0);
             }
+        }
+    };
+    // quad q's rows are in stg, and every wave is done with the other buffer
+    auto settle = [&](int f0, int q, int8_t* stg) {
+        __builtin_amdgcn_s_waitcnt(0);
+        finish(f0, q, stg);
+        __syncthreads();
     };
 
-    // quads alternate between the buffers: even quads in stage0, odd in stage1
-    int2 spA, spB;
-    int dA, dB;
-    lane_delay(0, spA, dA);
-    issue(0, stage0);
-    for(int q = 0; q < nq; q += 2) {
-        __builtin_amdgcn_s_waitcnt(0);  // this wave's loads of quad q
-        __syncthreads();                // every wave's; quad q - 1's products are done, stage1 is free
-        if(q + 1 < nq) {
-            lane_delay(q + 1, spB, dB);
-            issue(q + 1, stage1);
+    for(int f0 = 0; f0 < p.nchans; f0 += kMfTabCh) {
+        const int nf = min(kMfTabCh, p.nchans - f0), nq = nf / 4;
+        // workgroups that run together on an XCD take each eight quads in
+        // rotated order (the sums are exact in any): their row loads then
+        // fall on different channels' lines
+        auto order = [&](int q) { return (q | 7) < nq ? (q & ~7) | ((q + (int)wl) & 7) : q; };
+        __syncthreads();  // the last range's products are done
+        for(int i = threadIdx.x; i < nf; i += NW * 64) {
+            const int2 sp = p.span[(size_t)tile * p.nchans + f0 + i];
+            const long lo = in0 - sp.y, at = lo * p.stride_t + (f0 + i) * p.stride_f;
+            const int nr = (int)min((long)(TT * TS + sp.y - sp.x), p.nsamples - lo);
+            // the input's very last piece, where it is no whole one, is finish()'s
+            const bool end = ragged && f0 + i == p.nchans - 1 && lo + nr == p.nsamples;
+            const long bytes = (nr - 1) * p.stride_t + (end ? p.W & ~15 : p.W);
+            tab[i] = make_int4((int)at, (int)(at >> 32), (int)bytes, nr);
+            using R = typename std::conditional<NW == 16, uint4, uint2>::type;
+            reinterpret_cast<R*>(tab_rel)[i] =
+                reinterpret_cast<const R*>(p.rel)[(size_t)tile * p.nchans + f0 + i];
         }
-        products(stage0, spA, dA);
-        if(q + 1 < nq) {
-            __builtin_amdgcn_s_waitcnt(0);
-            __syncthreads();  // quad q + 1 staged; quad q's products are done, stage0 is free
-            if(q + 2 < nq) {
-                lane_delay(q + 2, spA, dA);
-                issue(q + 2, stage0);
+        __syncthreads();
+        // quads alternate between the buffers: even positions in stage0, odd in stage1
+        issue(f0, order(0), stage0);
+        for(int q = 0; q < nq; q += 2) {
+            settle(f0, order(q), stage0);
+            if(q + 1 < nq) issue(f0, order(q + 1), stage1);
+            products(order(q), stage0);
+            if(q + 1 < nq) {
+                settle(f0, order(q + 1), stage1);
+                if(q + 2 < nq) issue(f0, order(q + 2), stage0);
+                products(order(q + 1), stage1);
             }
-            products(stage1, spB, dB);
         }
     }
 
@@ -618,28 +487,67 @@ idisp_dma_kernel(const int8_t* __restrict__ in, int8_t* __restrict__ tdb, const 
 #pragma unroll
     for(int tt = 0; tt < NTT; ++tt) {
         const int t = t0 + 16 * tt + n;
-        if(t >= nout) continue;
-        int8_t* o = tdb + ((size_t)t * ndms + td.x + wv) * W;
+        if(t >= p.nout) continue;
+        int8_t* o = p.tdb + ((size_t)t * p.ndms + td.x + wv) * p.W;
 #pragma unroll
-        for(int bg = 0; bg < 8; ++bg) {
+        for(int bg = 0; bg < NBG; ++bg) {
             const int b = b0 + 16 * bg + 4 * g;
-            if(b >= W) continue;
+            if(b >= p.W) continue;
             const v4i a = acc[tt][bg];
-            const uint32_t packed = (uint32_t)(uint8_t)id_quant(a[0], scale) |
-                                    ((uint32_t)(uint8_t)id_quant(a[1], scale) << 8) |
-                                    ((uint32_t)(uint8_t)id_quant(a[2], scale) << 16) |
-                                    ((uint32_t)(uint8_t)id_quant(a[3], scale) << 24);
+            const uint32_t packed = (uint32_t)(uint8_t)id_quant(a[0], p.scale) |
+                                    ((uint32_t)(uint8_t)id_quant(a[1], p.scale) << 8) |
+                                    ((uint32_t)(uint8_t)id_quant(a[2], p.scale) << 16) |
+                                    ((uint32_t)(uint8_t)id_quant(a[3], p.scale) << 24);
             *reinterpret_cast<uint32_t*>(o + b) = packed;
         }
     }
 }
 
+// 32 output samples per workgroup
+template <int NW, int NBG, int RCAP, int TS, bool BIG>
+__global__ void __launch_bounds__(NW * 64, 4) idisp_dma_kernel(IdArgs p)
+{
+    idisp_tile<NW, 2, NBG, RCAP, TS, BIG>(p);
+}
+
+// 16 output samples per workgroup: tscrunch above 2, where 32 samples' rows
+// would leave the stage no room for the DMs' delays
+template <int NBG, int TS, bool BIG>
+__global__ void __launch_bounds__(kMfWaves * 64, 4) idisp_mfma_kernel(IdArgs p)
+{
+    idisp_tile<kMfWaves, 1, NBG, kMfRows, TS, BIG>(p);
+}
+
+template <int NBG, bool BIG>
+int idisp_launch_mfma(int ts, bool small, const IdArgs& a, hipStream_t st)
+{
+    const dim3 grid((unsigned)(8 * ((a.nwork + 7) / 8))), block(64 * (small ? kSmWaves : kMfWaves));
+    switch(small ? 0 : ts) {
+#define SW_IDM(TS, ...) \
+    case TS: hipLaunchKernelGGL((__VA_ARGS__), grid, block, 0, st, a); break;
+        SW_IDM(0, idisp_dma_kernel<kSmWaves, NBG, kSmRows, 1, BIG>)
+        SW_IDM(1, idisp_dma_kernel<kMfWaves, NBG, kMfRows, 1, BIG>)
+        SW_IDM(2, idisp_dma_kernel<kMfWaves, NBG, kMfRows, 2, BIG>)
+        SW_IDM(3, idisp_mfma_kernel<NBG, 3, BIG>)
+        SW_IDM(4, idisp_mfma_kernel<NBG, 4, BIG>)
+        SW_IDM(5, idisp_mfma_kernel<NBG, 5, BIG>)
+        SW_IDM(6, idisp_mfma_kernel<NBG, 6, BIG>)
+        SW_IDM(7, idisp_mfma_kernel<NBG, 7, BIG>)
+        SW_IDM(8, idisp_mfma_kernel<NBG, 8, BIG>)
+#undef SW_IDM
+    }
+    SW_LAUNCH_CHECK();
+    return SW_OK;
+}
+
 void free_plan_device(sw_idisp* p)
 {
     (void)hipFree(p->d_delays);
+    (void)hipFree(p->d_rel);
     (void)hipFree(p->d_span);
     (void)hipFree(p->d_tiles);
     p->d_delays = nullptr;
+    p->d_rel = nullptr;
     p->d_span = nullptr;
     p->d_tiles = nullptr;
 }
@@ -753,15 +661,64 @@ extern "C" int sw_idisp_create(const sw_idisp_config* cfg, sw_idisp** out)
 
     // tiling: TT output samples per workgroup, tiles of consecutive DMs whose
     // union of read rows fits the LDS stage
-    int cap = sw::kRowsCap, dmax_tile = 8;
+    const int F = p->nchans;
+    std::vector<int2> span;
+    auto tile_dms = [&](int cap, int dmax_tile) {
+        p->tiles.clear();
+        span.clear();
+        p->rows_cap = 0;
+        for(int d = 0; d < p->ndms;) {
+            int n = 1;
+            while(n < dmax_tile && d + n < p->ndms) {
+                int worst = 0;
+                for(int f = 0; f < F; ++f) {
+                    int lo = INT32_MAX, hi = INT32_MIN;
+                    for(int k = 0; k <= n; ++k) {
+                        lo = std::min(lo, p->delays[(size_t)(d + k) * F + f]);
+                        hi = std::max(hi, p->delays[(size_t)(d + k) * F + f]);
+                    }
+                    worst = std::max(worst, hi - lo);
+                }
+                if(worst + p->tt * p->tscrunch > cap) break;
+                ++n;
+            }
+            p->tiles.push_back(make_int2(d, n));
+            int rows = 0;
+            for(int f = 0; f < F; ++f) {
+                int lo = INT32_MAX, hi = INT32_MIN;
+                for(int k = 0; k < n; ++k) {
+                    lo = std::min(lo, p->delays[(size_t)(d + k) * F + f]);
+                    hi = std::max(hi, p->delays[(size_t)(d + k) * F + f]);
+                }
+                span.push_back(make_int2(lo, hi));
+                rows = std::max(rows, hi - lo + p->tt * p->tscrunch);
+            }
+            p->rows_cap = std::max(p->rows_cap, rows);
+            d += n;
+        }
+    };
+    std::vector<uint8_t> rel;
     p->mfma = cfg->kernel == 0 && p->nchans % 4 == 0 && 16 * p->tscrunch <= sw::kMfRows;
     if(p->mfma) {
-        // 32 output samples per workgroup of 16 waves (one DM each), the
-        // quads' rows double-buffered in LDS; 16 samples per workgroup of 8
-        // waves (two DMs each) where 32 samples' rows would not fit the stage
+        static_assert(16 * sw::kMfMaxTs <= sw::kMfRows && 16 * (sw::kMfMaxTs + 1) > sw::kMfRows, "every tscrunch has a kernel");
+        // 32 output samples per workgroup while that leaves half of the stage
+        // for the DMs' delays, else 16
         p->tt = 32 * p->tscrunch <= sw::kMfRows / 2 ? 32 : 16;
-        cap = sw::kMfRows;
-        dmax_tile = p->tt == 32 ? sw::kDmaWaves : sw::kMfWaves * sw::kMfDpw;
+        // where every run of 8 DMs fits the small stage, two workgroups of 8
+        // waves share a CU and one's products cover the other's waits;
+        // otherwise 16 DMs share the staged rows
+        if(p->tscrunch == 1) {
+            tile_dms(sw::kSmRows, sw::kSmWaves);
+            p->small = (int)p->tiles.size() == (p->ndms + sw::kSmWaves - 1) / sw::kSmWaves;
+        }
+        if(!p->small) tile_dms(sw::id_stage_rows(sw::kMfRows, p->tscrunch), sw::kMfWaves);
+        const int nw = p->small ? sw::kSmWaves : sw::kMfWaves;
+        rel.assign(p->tiles.size() * F * nw, 0);
+        for(size_t t = 0; t < p->tiles.size(); ++t)
+            for(int f = 0; f < F; ++f)
+                for(int k = 0; k < p->tiles[t].y; ++k)
+                    rel[(t * F + f) * nw + k] =
+                        (uint8_t)(span[t * F + f].y - p->delays[(size_t)(p->tiles[t].x + k) * F + f]);
     } else {
         p->wide = (long)p->nchans * p->tscrunch > 256;
         p->tt = p->wide ? 8 : 16;
@@ -771,37 +728,11 @@ extern "C" int sw_idisp_create(const sw_idisp_config* cfg, sw_idisp** out)
             return SW_ERR_UNSUPPORTED;
         }
         p->dpw = 2;
+        tile_dms(sw::kRowsCap, 8);
     }
-    const int F = p->nchans;
-    std::vector<int2> span;
-    for(int d = 0; d < p->ndms;) {
-        int n = 1;
-        while(n < dmax_tile && d + n < p->ndms) {
-            int worst = 0;
-            for(int f = 0; f < F; ++f) {
-                int lo = INT32_MAX, hi = INT32_MIN;
-                for(int k = 0; k <= n; ++k) {
-                    lo = std::min(lo, p->delays[(size_t)(d + k) * F + f]);
-                    hi = std::max(hi, p->delays[(size_t)(d + k) * F + f]);
-                }
-                worst = std::max(worst, hi - lo);
-            }
-            if(worst + p->tt * p->tscrunch > cap) break;
-            ++n;
-        }
-        p->tiles.push_back(make_int2(d, n));
-        int rows = 0;
-        for(int f = 0; f < F; ++f) {
-            int lo = INT32_MAX, hi = INT32_MIN;
-            for(int k = 0; k < n; ++k) {
-                lo = std::min(lo, p->delays[(size_t)(d + k) * F + f]);
-                hi = std::max(hi, p->delays[(size_t)(d + k) * F + f]);
-            }
-            span.push_back(make_int2(lo, hi));
-            rows = std::max(rows, hi - lo + p->tt * p->tscrunch);
-        }
-        p->rows_cap = std::max(p->rows_cap, rows);
-        d += n;
+    if(!rel.empty()) {
+        SW_HIP_TRY(hipMalloc(&p->d_rel, rel.size()));
+        SW_HIP_TRY(hipMemcpy(p->d_rel, rel.data(), rel.size(), hipMemcpyHostToDevice));
     }
     SW_HIP_TRY(hipMalloc(&p->d_delays, sizeof(int) * p->delays.size()));
     SW_HIP_TRY(hipMalloc(&p->d_span, sizeof(int2) * span.size()));
@@ -879,40 +810,26 @@ int sw::idisp_launch(sw_idisp* p, const void* d_tfb, size_t nsamples, int nbeams
     const long stride_t = ftb ? nwords : (long)p->nchans * nwords;
     const long stride_f = ftb ? (long)nsamples * nwords : nwords;
     if(p->mfma) {
-        const long nchunks128 = (nbv + 127) / 128;
-        const long ntb128 = (nout + p->tt - 1) / p->tt;
+        // chunks of 128 bytes of beams; a last one of at most 64 by itself,
+        // with half of the products.  big: 32 bits do not span a stage's rows
+        const bool big = 128 * stride_t * 4 + nbv >= 0xFFFFFFF0L;
+        const int last = (int)(nbv % 128), nfull = (int)(nbv / 128) + (last > 64 || (big && last > 0));
         const long ntiles = (long)p->tiles.size();
-        const long nwork = (ntiles + sw::kIdTileGroup - 1) / sw::kIdTileGroup * sw::kIdTileGroup * nchunks128 *
-                           ((ntb128 + sw::kIdTbGroup - 1) / sw::kIdTbGroup * sw::kIdTbGroup);
-        const long max_launch = 8L << 20;  // work items per launch (grid x threads < 2^32)
-        const bool v16 = nbv % 16 == 0 && stride_t % 4 == 0 && stride_f % 4 == 0;  // strides in words
-        for(long w0 = 0; w0 < nwork; w0 += max_launch) {
-            const long nw = std::min(max_launch, nwork - w0);
-            const unsigned nblk = (unsigned)(8 * ((nw + 7) / 8));
-#define SW_IDM_LAUNCH(NTT, V16)                                                                              \
-    hipLaunchKernelGGL((sw::idisp_mfma_kernel<sw::kMfWaves, sw::kMfDpw, NTT, sw::kMfRows, V16, NTT == 2>), dim3(nblk), \
-                       dim3(sw::kMfWaves * 64), 0, st, static_cast<const int8_t*>(d_tfb),                   \
-                       static_cast<int8_t*>(d_tdb), p->d_delays, p->d_span, p->d_tiles, (int)ntiles,          \
-                       (int)nchunks128, (int)ntb128, w0, nw, p->nchans, (int)nbv, p->ndms, p->tscrunch, p->max_delay,      \
-                       (long)nsamples, nout, p->scale, stride_t * 4, stride_f * 4)
-            if(p->tt == 32) {
-                if(v16)
-                    hipLaunchKernelGGL((sw::idisp_dma_kernel<sw::kDmaWaves, 2, sw::kMfRows>), dim3(nblk),
-                                       dim3(sw::kDmaWaves * 64), 0, st, static_cast<const int8_t*>(d_tfb),
-                                       static_cast<int8_t*>(d_tdb), p->d_delays, p->d_span, p->d_tiles,
-                                       (int)ntiles, (int)nchunks128, (int)ntb128, w0, nw, p->nchans, (int)nbv,
-                                       p->ndms, p->tscrunch, p->max_delay, (long)nsamples, nout, p->scale,
-                                       stride_t * 4, stride_f * 4);
-                else
-                    SW_IDM_LAUNCH(2, false);
-            } else {
-                if(v16)
-                    SW_IDM_LAUNCH(1, true);
-                else
-                    SW_IDM_LAUNCH(1, false);
+        for(int half = 0; half < 2; ++half) {
+            const int chunk0 = half ? nfull : 0, nchunks128 = half ? (last > 0 && last <= 64 && !big) : nfull;
+            const long nwork = (ntiles + sw::kIdTileGroup - 1) / sw::kIdTileGroup * sw::kIdTileGroup * nchunks128 *
+                               (((long)ntb + sw::kIdTbGroup - 1) / sw::kIdTbGroup * sw::kIdTbGroup);
+            const long max_launch = 4L << 20;  // work items per launch (grid x threads < 2^32)
+            for(long w0 = 0; w0 < nwork; w0 += max_launch) {
+                const sw::IdArgs a{static_cast<const int8_t*>(d_tfb), static_cast<int8_t*>(d_tdb), p->d_rel,
+                                   p->d_span, p->d_tiles, (int)ntiles, chunk0, nchunks128, ntb, w0,
+                                   std::min(max_launch, nwork - w0), p->nchans, (int)nbv, p->ndms, p->max_delay,
+                                   (long)nsamples, nout, p->scale, stride_t * 4, stride_f * 4};
+                const int rc = half  ? sw::idisp_launch_mfma<4, false>(p->tscrunch, p->small, a, st)
+                               : big ? sw::idisp_launch_mfma<8, true>(p->tscrunch, p->small, a, st)
+                                     : sw::idisp_launch_mfma<8, false>(p->tscrunch, p->small, a, st);
+                if(rc) return rc;
             }
-#undef SW_IDM_LAUNCH
-            SW_LAUNCH_CHECK();
         }
         return SW_OK;
     }

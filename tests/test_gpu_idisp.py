@@ -86,6 +86,48 @@ def test_vs_oracle(sw, orc, dev, case, valu):
         np.testing.assert_array_equal(out, want, err_msg=layout)
 
 
+@pytest.mark.parametrize("F,B,ts,dms,nout,band", [
+    (516, 20, 1, np.arange(0, 30, 3.0, dtype=np.float32), 35, (1284e6, 107.8359375e6, 16)),  # past one delay table
+    (64, 404, 4, np.arange(0, 40, 1.25, dtype=np.float32), 33, (1284e6, 13.375e6, 4)),       # a last chunk of 20 bytes
+    (8, 132, 3, np.arange(0, 90, 9.0, dtype=np.float32), 17, (1284e6, 26.75e6, 8)),          # of 4 bytes
+    (12, 196, 5, np.arange(0, 60, 6.0, dtype=np.float32), 18, (1284e6, 26.75e6, 8)),         # of 68 bytes
+    (16, 60, 6, np.arange(0, 60, 6.0, dtype=np.float32), 31, (1284e6, 26.75e6, 8)),
+    (16, 64, 7, np.arange(0, 60, 6.0, dtype=np.float32), 16, (1284e6, 26.75e6, 8)),
+    (16, 4, 8, np.arange(0, 9, 1.0, dtype=np.float32), 1, (1284e6, 26.75e6, 8)),             # one output sample
+    (128, 252, 2, np.arange(0, 70, 2.0, dtype=np.float32), 65, (1284e6, 26.75e6, 16)),
+    (64, 68, 1, np.arange(0, 70, 0.5, dtype=np.float32), 97, (1284e6, 13.375e6, 16)),        # 8-DM tiles, ragged
+    (256, 36, 1, np.arange(0, 330, 1.0, dtype=np.float32), 40, (1284e6, 53.5e6, 8)),         # 16-DM tiles, ragged
+])
+def test_matrix_core_forms(sw, orc, dev, F, B, ts, dms, nout, band):
+    """Every tscrunch of the matrix-core forms, rows that are no whole 16-byte pieces (the last
+    row ends the buffer), half-empty chunks, both tile sizes."""
+    fc, bw, cbts = band
+    idd = sw.IncoherentDedisperser(F, fc, bw, cbts, dms, tscrunch=ts)
+    assert idd.kernel != "idisp_kernel"
+    T = idd.max_delay + ts * nout
+    tfb = _rand((T, F, B), 7 + F + ts, sigma=40.0)
+    tfb.reshape(-1)[::997] = -128
+    tfb[-1, -1] = np.arange(B) % 251 - 125  # the piece that ends the input
+    want = orc.incoherent_dedisperse(tfb, idd.delays, idd.max_delay, ts)
+    for layout in ("tfb", "ftb"):
+        np.testing.assert_array_equal(_run(sw, idd, tfb, 1, layout), want, err_msg=layout)
+
+
+def test_matrix_core_rows_past_32_bits(sw, orc, dev):
+    # a stage's rows span more than 4 GiB: 64-bit addresses; the beams repeat with period 64
+    F, B, nout = 1024, 32784, 3
+    idd = sw.IncoherentDedisperser(F, 1284e6, 214e6, 16, np.arange(0, 0.6, 0.2, dtype=np.float32))
+    assert idd.max_delay > 0
+    T = idd.max_delay + nout
+    x = _rand((T, F, 64), 8, sigma=40.0)
+    tfb = np.concatenate([np.tile(x, B // 64), x[:, :, :B % 64]], 2)
+    out = _run(sw, idd, tfb, 1)
+    want = orc.incoherent_dedisperse(x, idd.delays, idd.max_delay, 1)
+    np.testing.assert_array_equal(out[:, :, :64], want)
+    np.testing.assert_array_equal(out[:, :, -80:-16], want)
+    np.testing.assert_array_equal(out[:, :, -16:], want[:, :, :16])
+
+
 def test_saturating_sums(sw, orc, dev):
     # every input at the extremes: the quantised output clamps at -128 / 127
     F, B = 64, 32
