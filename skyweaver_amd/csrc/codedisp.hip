@@ -102,16 +102,6 @@ __device__ __forceinline__ float2 input_sample(const CdParams& p, int f, int col
     return make_float2(0.0f, 0.0f);
 }
 
-// raw complex int8 sample (re | im << 8), zero outside history + gulp
-__device__ __forceinline__ uint32_t input_raw(const CdParams& p, int f, int col, int tau)
-{
-    if(tau < 0 && p.prev)
-        return *reinterpret_cast<const uint16_t*>(p.prev + (((size_t)f * p.PA + col) * p.T + p.T + tau) * 2);
-    if(tau < 0) return *reinterpret_cast<const uint16_t*>(p.hist + (((size_t)f * p.PA + col) * p.Oh + p.Oh + tau) * 2);
-    if(tau < p.T) return *reinterpret_cast<const uint16_t*>(p.cur + (((size_t)f * p.PA + col) * p.T + tau) * 2);
-    return 0;
-}
-
 __device__ __forceinline__ float2 unpack_c8(uint32_t v)
 {
     return make_float2((float)(int8_t)(v & 0xff), (float)(int8_t)((v >> 8) & 0xff));
@@ -401,38 +391,6 @@ __device__ __forceinline__ void reg_chirp_inverse(const float2* X, float2* v, fl
     for(int c = 0; c < C; ++c) dft_mul<R1, true>(v + c * R1, wc);
 }
 
-// Raw complex int8 samples b + 512 i + t, i = 0..2 n - 1, of one column,
-// two per register, where b is the first sample of a segment relative to
-// the gulp start (negative: history).
-template <int NP>
-__device__ __forceinline__ void load_column(const CdParams& p, int f, int col, long b, int t, uint32_t* dst)
-{
-    constexpr int NS = 1024 * NP;  // samples spanned
-    const size_t cc = (size_t)f * p.PA + col;
-    const uint16_t* cur = reinterpret_cast<const uint16_t*>(p.cur) + cc * p.T;
-    if(b >= 0 && b + NS <= p.T) {  // inside this gulp (uniform branch)
-        const uint16_t* x = cur + b;
-#pragma unroll
-        for(int i = 0; i < NP; ++i)
-            dst[i] = (uint32_t)x[1024 * i + t] | ((uint32_t)x[1024 * i + 512 + t] << 16);
-    } else if(b < 0 && b + NS <= p.T) {  // history, then this gulp
-        // lo[tau] for tau < 0: the previous gulp's tail or the history buffer
-        const uint16_t* lo = p.prev ? reinterpret_cast<const uint16_t*>(p.prev) + cc * p.T + p.T
-                                    : reinterpret_cast<const uint16_t*>(p.hist) + cc * p.Oh + p.Oh;
-        const int b32 = (int)b;
-#pragma unroll
-        for(int i = 0; i < NP; ++i) {
-            const int t0 = b32 + 1024 * i + t, t1 = t0 + 512;
-            dst[i] = (uint32_t)(t0 < 0 ? lo : cur)[t0] | ((uint32_t)(t1 < 0 ? lo : cur)[t1] << 16);
-        }
-    } else {
-#pragma unroll
-        for(int i = 0; i < NP; ++i)
-            dst[i] = input_raw(p, f, col, (int)(b + 1024 * i + t)) |
-                     (input_raw(p, f, col, (int)(b + 1024 * i + 512 + t)) << 16);
-    }
-}
-
 // The raw samples (re | im << 8) of one unit of the register kernels: value
 // i = c R1 + n1 is sample b + 512 n1 + t of column col0 + c, b the segment's
 // first sample relative to the gulp start (negative: history).  The uniform
@@ -443,10 +401,10 @@ __device__ __forceinline__ void load_column(const CdParams& p, int f, int col, l
 // round trips per unit at N = 1024, none behind the transforms; 256 channels
 // x 128 columns x 65536 samples took 8.47 ms, now 4.88; N = 16384 at 64
 // channels 1.71, now 1.57.)
-template <int R1>
-__device__ __forceinline__ void load_unit(const CdParams& p, int f, int col0, long b, int t, uint32_t (&raw)[32])
+template <int R1, int NV>
+__device__ __forceinline__ void load_unit(const CdParams& p, int f, int col0, long b, int t, uint32_t (&raw)[NV])
 {
-    constexpr int C = 32 / R1;
+    constexpr int C = NV / R1;
     const size_t cc = (size_t)f * p.PA + col0;
     const uint16_t* cur = reinterpret_cast<const uint16_t*>(p.cur) + cc * p.T;
     if(b >= 0 && b + 512 * R1 <= p.T) {  // inside this gulp
@@ -664,18 +622,29 @@ __global__ void __launch_bounds__(512) codedisp_regm_kernel(CdParams p, int nuni
     }
 }
 
+// a pointer that is the same in every lane, as a scalar
+template <typename P>
+__device__ __forceinline__ P* uniform_ptr(P* p)
+{
+    const unsigned long a = reinterpret_cast<unsigned long>(p);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)a);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(a >> 32));
+    return reinterpret_cast<P*>((unsigned long)hi << 32 | lo);
+}
+
 // N = 32768 as two interleaved 16384-point halves (radix-2 decimation in
 // frequency, RP = 2, L = N / 2), fused into one persistent kernel:
 //   Z_r[n] = W_N^(n r) (x[n] + (-1)^r x[n + L]),  X[2m + r] = FFT_L(Z_r)[m]
 //   V_r = IFFT_L(X[2m + r] H[2m + r])
 //   y[n] = V_0[n] + W_N^(-n) V_1[n],  y[n + L] = V_0[n] - W_N^(-n) V_1[n]
-// Each thread holds samples n = 512 n1 + t (and n + L) of one column.  V_0
-// waits in a per-workgroup slice of `scratch` (each thread reads back only
-// what it wrote) while V_1 is transformed; the chirp is stored [F][r][L] in
-// the register order of the halves.  The raw samples are loaded for each
-// half (the second load hits L2) rather than held across a transform, which
-// would not fit the registers.
-__global__ void __launch_bounds__(512) codedisp_reg2_kernel(CdParams p, int d, int nunits, float2* scratch)
+// Each thread holds samples n = 512 n1 + t (and n + L) of one column; the
+// chirp is stored [F][r][L] in the register order of the halves.  The 64
+// registers that hold the raw samples while half 0 is transformed hold V_0
+// while half 1 is: nothing but the samples, the tables and the outputs goes
+// through memory.  (With V_0 in a per-workgroup slice of memory, 128 KB that
+// L2 does not hold for all workgroups, and the samples loaded for each half,
+// 32 channels x 128 columns x 131072 samples took 3.26 ms; now 1.95.)
+__global__ void __launch_bounds__(512) codedisp_reg2_kernel(CdParams p, int d, int nunits)
 {
     constexpr int L = 16384, N = 2 * L;
     __shared__ float2 lds[kRegLds + TwiddleLds<L>::SIZE + 1024];
@@ -683,58 +652,66 @@ __global__ void __launch_bounds__(512) codedisp_reg2_kernel(CdParams p, int d, i
     float2* t1k = lds + kRegLds + TwiddleLds<L>::SIZE;  // step 2/3 twiddle tables
     const int t = threadIdx.x;
     load_step2_tables<32>(t1k, p.tw, t);
-    uint32_t raw[32];  // x[512 n1 + t] at 0..15, x[L + 512 n1 + t] at 16..31, two per register
+    // x[512 n1 + t] | x[L + 512 n1 + t] << 16 in the x of n1, then V_0
+    float2 held[32];
+    auto fetch = [&](int u, uint32_t (&x)[64]) {
+        const int col = u % p.PA, fs = u / p.PA;
+        load_unit<64>(p, fs / p.nseg, col, p.in0 + (long)(fs % p.nseg) * p.hop, t, x);
+    };
+    auto pack = [&](const uint32_t (&x)[64]) {
+#pragma unroll
+        for(int n1 = 0; n1 < 32; ++n1) {
+            held[n1] = make_float2(__uint_as_float(x[n1] | (x[32 + n1] << 16)), 0.0f);
+            asm volatile("" : "+v"(held[n1].x));  // packed here, not where it is used
+        }
+    };
+    if((int)blockIdx.x < nunits) {
+        uint32_t x[64];
+        fetch(blockIdx.x, x);
+        pack(x);
+    }
+    // W_N^(512 n1 + t) by buffer loads: one offset register, a scalar offset per n1
+    const auto wrs = buffer_rsrc(p.twN, (uint32_t)L * 8u);
+    auto wn = [&](int n1) {
+        const auto x = __builtin_amdgcn_raw_buffer_load_b64(wrs, 8 * t, 4096 * n1, 0);
+        return make_float2(__uint_as_float(x[0]), __uint_as_float(x[1]));
+    };
     for(int u = blockIdx.x; u < nunits; u += gridDim.x) {
         const int col = u % p.PA, fs = u / p.PA;
         const int f = fs / p.nseg, s = fs % p.nseg;
-        const long b = p.in0 + (long)s * p.hop;
         const float2* H = p.chirp[d] + (size_t)f * N;
         float2 v[32];
+#pragma unroll
+        for(int n1 = 0; n1 < 32; ++n1) {  // Z_0 = x[n] + x[n + L]
+            const uint32_t x = __float_as_uint(held[n1].x);
+            v[n1] = cadd(unpack_c8(x), unpack_c8(x >> 16));
+        }
         // the two halves share one copy of the transform code (a loop that
         // is not unrolled): the kernel then fits the instruction cache
 #pragma unroll 1
         for(int r = 0; r < 2; ++r) {
-            // the thread's slots, formed afresh per half (an opaque offset
-            // keeps the compiler from holding 32 precomputed addresses in
-            // registers across the transforms)
-            int off = t;
-            asm volatile("" : "+v"(off));
-            float2* mine = scratch + (size_t)blockIdx.x * L + off;  // [n1][512]
-            const float2* wn = p.twN + off;                         // W_N^(512 n1 + t) at wn[512 n1]
-            load_column<32>(p, f, col, b, off, raw);
-            if(r == 0) {  // Z_0 = x[n] + x[n + L]
-#pragma unroll
-                for(int i = 0; i < 16; ++i) {
-                    v[2 * i]     = cadd(unpack_c8(raw[i]), unpack_c8(raw[16 + i]));
-                    v[2 * i + 1] = cadd(unpack_c8(raw[i] >> 16), unpack_c8(raw[16 + i] >> 16));
-                }
-            } else {  // Z_1 = W_N^n (x[n] - x[n + L])
-#pragma unroll
-                for(int i = 0; i < 16; ++i) {
-                    v[2 * i]     = csub(unpack_c8(raw[i]), unpack_c8(raw[16 + i]));
-                    v[2 * i + 1] = csub(unpack_c8(raw[i] >> 16), unpack_c8(raw[16 + i] >> 16));
-                }
-#pragma unroll
-                for(int n1 = 0; n1 < 32; ++n1) v[n1] = cmul(v[n1], wn[512 * n1]);
-            }
             __syncthreads();  // twiddle tables; previous readers of the exchange buffer
             // step-1 twiddles rebuilt at each use (held, they would not fit
             // the registers)
-            float2 hk0[16];  // no chirp prefetch (registers)
-            reg_forward<32, false>(v, lds, tw, t1k, t, nullptr, nullptr, hk0);
-            reg_chirp_inverse<32, false>(v, v, lds, tw, t1k, t, H + r * L, nullptr, hk0);
-            if(r == 0) {
+            const float2* Hr = uniform_ptr(H + r * L);
+            float2 hk0[16];
+            reg_forward<32, false, true>(v, lds, tw, t1k, t, nullptr, Hr, hk0);
+            reg_chirp_inverse<32, false, true>(v, v, lds, tw, t1k, t, Hr, nullptr, hk0);
+            if(r == 0) {  // Z_1 = W_N^n (x[n] - x[n + L])
 #pragma unroll
-                for(int n1 = 0; n1 < 32; ++n1) mine[512 * n1] = v[n1];
+                for(int n1 = 0; n1 < 32; ++n1) {
+                    const uint32_t x = __float_as_uint(held[n1].x);
+                    held[n1] = v[n1];
+                    v[n1] = cmul(csub(unpack_c8(x), unpack_c8(x >> 16)), wn(n1));
+                }
             }
         }
         // ---- y[n] = V_0 + W_N^(-n) V_1, y[n + L] = V_0 - W_N^(-n) V_1
+        // (V_0, V_1 already / N: the chirp)
         const int j0 = (int)(p.y0 + (long)s * p.hop) - p.O / 2;
         const size_t cb = ((size_t)f * p.PA + col) * p.ylen;
         int tt = t;  // opaque: addresses and position tests formed here, not held across units
         asm volatile("" : "+v"(tt));
-        const float2* mine = scratch + (size_t)blockIdx.x * L + tt;
-        const float2* wn = p.twN + tt;
         const int half = p.O / 2;
         if(half <= 512 && !p.outf[d]) {
             // as store_unit: byte offsets from the column's base wrapped by
@@ -751,19 +728,24 @@ __global__ void __launch_bounds__(512) codedisp_reg2_kernel(CdParams p, int d, i
             const bool lo_kept = tt >= half, hi_kept = tt < 512 - half;
 #pragma unroll
             for(int n1 = 0; n1 < 32; ++n1) {
-                const float2 a = mine[512 * n1];
-                const float2 b = cmul(v[n1], cconj(wn[512 * n1]));  // V_0, V_1 already / N (chirp)
+                const float2 a = held[n1];
+                const float2 b = cmul(v[n1], cconj(wn(n1)));
                 if(n1 > 0 || lo_kept) put(n1, cadd(a, b));
                 if(n1 < 31 || hi_kept) put(32 + n1, csub(a, b));
             }
         } else {
 #pragma unroll
             for(int n1 = 0; n1 < 32; ++n1) {
-                const float2 a = mine[512 * n1];
-                const float2 b = cmul(v[n1], cconj(wn[512 * n1]));
+                const float2 a = held[n1];
+                const float2 b = cmul(v[n1], cconj(wn(n1)));
                 store_output(p, d, cb, j0, 512 * n1 + tt, N, cadd(a, b));
                 store_output(p, d, cb, j0, L + 512 * n1 + tt, N, csub(a, b));
             }
+        }
+        if(u + (int)gridDim.x < nunits) {
+            uint32_t x[64];
+            fetch(u + gridDim.x, x);
+            pack(x);
         }
     }
 }
@@ -984,12 +966,12 @@ int reg_r1(int N, int RP, int PA)
 // segment, column) for N = 32768.  N <= 16384: several DMs (p.ndm > 1) share
 // one forward transform in codedisp_regm_kernel, one DM alone runs in
 // codedisp_reg_kernel; N = 32768: one DM per launch.
-int launch_reg(int R1, const CdParams& p, int nunits, float2* scratch, hipStream_t st)
+int launch_reg(int R1, const CdParams& p, int nunits, hipStream_t st)
 {
     const dim3 grid((unsigned)std::min(nunits, persistent_blocks()));
     if(p.RP == 2) {
         for(int d = 0; d < p.ndm; ++d) {
-            hipLaunchKernelGGL(codedisp_reg2_kernel, grid, dim3(512), 0, st, p, d, nunits, scratch);
+            hipLaunchKernelGGL(codedisp_reg2_kernel, grid, dim3(512), 0, st, p, d, nunits);
             SW_LAUNCH_CHECK();
         }
         return SW_OK;
@@ -1058,7 +1040,6 @@ struct sw_codedisp {
     std::vector<int> lat;                // per DM output latency
     long long gulps = 0;                 // gulps completed (push_history calls)
     float2* zbuf = nullptr;              // DIF stage output (N > kMaxL)
-    float2* reg2 = nullptr;              // N = 32768 kernel: one 16384-point half per workgroup
     std::vector<float2*> vbuf;           // per DM slot (N > kMaxL)
     ~sw_codedisp()
     {
@@ -1070,7 +1051,6 @@ struct sw_codedisp {
         for(auto* y : ytm) (void)hipFree(y);
         for(auto* y : ytf) (void)hipFree(y);
         (void)hipFree(zbuf);
-        (void)hipFree(reg2);
         for(auto* v : vbuf) (void)hipFree(v);
     }
 };
@@ -1201,22 +1181,17 @@ extern "C" int sw_codedisp_create(const sw_codedisp_config* cfg, void* stream, s
         }
     }
     size_t zmax = 0, slots = 1, vslots = 0;
-    bool reg2 = false;
     for(auto& g : p->groups) {
         if(!sw::twiddle_table(p.get(), g.L, st)) return SW_ERR_ALLOC;
         slots = std::max(slots, std::min<size_t>(sw::kMaxDm, g.dms.size()));
         if(g.RP > 1) {
             if(!sw::twiddle_table(p.get(), g.N, st)) return SW_ERR_ALLOC;
-            if(sw::reg_r1(g.N, g.RP, p->PA) > 0) {
-                reg2 = true;
-            } else {
+            if(sw::reg_r1(g.N, g.RP, p->PA) == 0) {
                 zmax = std::max(zmax, (size_t)p->F * g.nseg * g.N * p->PA * sizeof(float2));
                 vslots = std::max(vslots, std::min<size_t>(sw::kMaxDm, g.dms.size()));
             }
         }
     }
-    if(reg2)
-        SW_HIP_TRY(hipMalloc(&p->reg2, sizeof(float2) * 16384 * (size_t)sw::persistent_blocks()));
     p->chirp.resize(p->dms.size(), nullptr);
     for(int d = 0; d < (int)p->dms.size(); ++d) {
         const int N = p->N[d], RP = N / std::min(N, sw::kMaxL);
@@ -1643,7 +1618,7 @@ extern "C" int sw_codedisp_run(sw_codedisp* plan, const void* d_in, void* const*
                 // no segment completes in this gulp
             } else if(R1 > 0) {
                 const int units = g.RP == 2 ? plan->F * p.nseg * plan->PA : plan->F * p.nseg * (plan->PA / (32 / R1));
-                rc = sw::launch_reg(R1, p, units, plan->reg2, st);
+                rc = sw::launch_reg(R1, p, units, st);
                 if(rc) return rc;
             } else if(g.RP == 1) {
                 rc = sw::launch_lds<false>(g.L, p, plan->F * p.nseg * G, st);

@@ -296,7 +296,7 @@ struct IdArgs {
 // What bounds it: the round trip of a quad's row loads, issued after the
 // barrier that frees their buffer, together with the LDS reads of the
 // products, 8 cycles of the CU per 1024 channel sums.  1024 DMs x 512 beams x
-// 256 channels x 4096 samples take 9.8 ms (5.6e13 sums/s), 6.6 ms without the
+// 256 channels x 4096 samples take 10.2 ms (5.4e13 sums/s), 6.6 ms without the
 // loads, 8.4 ms without the products.  A load therefore costs no address
 // arithmetic: per channel a table in LDS, filled once per kMfTabCh channels,
 // holds where its rows begin and end, a buffer resource over them takes the
