@@ -360,3 +360,22 @@ def test_codedisp_dm0_is_a_delay(sw, dev, fpat, in_place, T, N, O):
         plan.run(bufs[-1], [out, other])
         plan.push_history(bufs[-1])
         assert np.array_equal(out.download(), stream[:, g * T:(g + 1) * T]), g
+
+
+@pytest.mark.parametrize("T,N,O", [(1500, 512, 12),     # 12 samples of history: no whole 16-byte blocks
+                                   (500, 1024, 24),     # a gulp shorter than the history: a block straddles its start
+                                   (1512, 256, 4)])     # 252 samples a segment, history of one odd half block
+def test_codedisp_history_blocks(sw, dev, T, N, O):
+    """The pushed history, block by block: a DM of 0 returns the stream delayed, bit for bit."""
+    from skyweaver_amd import DeviceBuffer as DB
+    F, A, G = 2, 16, 6
+    x = np.random.default_rng(T + N).integers(-128, 128, (F, G * T, 2, A, 2)).astype(np.int8)
+    plan = sw.CoherentDedisperser(F, A, T, F_LOW, CHAN_BW, TSAMP, [0.0], fft_len=[N], overlap=[O], input_fpat=True)
+    L = plan.latency(0)
+    stream = np.concatenate([np.zeros((F, L + O // 2) + x.shape[2:], np.int8), x], 1)
+    out = DB.empty((F, T, 2, A, 2), np.int8)
+    for g in range(G):
+        buf = DB.from_host(np.ascontiguousarray(x[:, g * T:(g + 1) * T].transpose(0, 2, 3, 1, 4)))
+        plan.run(buf, [out])
+        plan.push_history(buf)
+        assert np.array_equal(out.download(), stream[:, g * T:(g + 1) * T]), g
