@@ -24,6 +24,7 @@
 #include "sw_common.hpp"
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <condition_variable>
 #include <cstring>
@@ -842,8 +843,8 @@ int run_gulp(sw_pipeline* p, const void* in, hipEvent_t consumed)
         p->stats = p->stats_bufs[par];
         wk->wait_free(p->stats);
     }
-    SW_HIP_TRY(hipEventRecord(p->ev_w[0], st));
     if(p->delays) {
+        SW_HIP_TRY(hipEventRecord(p->ev_w[0], st));
         // DelayManager::delays + WeightsManager::weights at the gulp's unix time
         // (BeamformerPipeline.cu:292-295: utc_start + utc_offset + n ticks / clock)
         const long double unix_ts = (long double)p->header.utc_start + (long double)p->header.utc_offset +
@@ -864,10 +865,15 @@ int run_gulp(sw_pipeline* p, const void* in, hipEvent_t consumed)
             rc = sw_cb_pack_weights(p->weights, p->packed, F, c.nbeams, A, st);
             if(rc) return rc;
         }
+        SW_HIP_TRY(hipEventRecord(p->ev_w[1], st));
     }
-    SW_HIP_TRY(hipEventRecord(p->ev_w[1], st));
     if(c.graph && !p->scalings_dirty) return run_gulp_graph(p, in, consumed, par, utc_offset_gulp);
-    SW_HIP_TRY(hipEventRecord(p->ev[0], st));
+    // The stages are timed between events recorded on the stream.  Each costs
+    // the stream about 5 us (64 beams of 64 channels x 8192 samples at DM 0:
+    // 238 us a gulp with one at either end of every stage, 201 us so), so
+    // stages that meet share the one between them.
+    hipEvent_t e_start = p->delays ? p->ev_w[1] : p->ev[0];
+    if(!p->delays) SW_HIP_TRY(hipEventRecord(e_start, st));
     // the gulp is held time-major (FPAT) up to the dedisperser; the two FPAT
     // buffers alternate so that the previous gulp stays readable as history
     std::swap(p->ftpa, p->ftpa_prev);
@@ -882,7 +888,6 @@ int run_gulp(sw_pipeline* p, const void* in, hipEvent_t consumed)
         if(rc) return rc;
     }
     SW_HIP_TRY(hipEventRecord(p->ev[1], st));
-    SW_HIP_TRY(hipEventRecord(p->ev[2], st));
     if(p->scalings_dirty) {
         // update_scalings on the first gulp (BeamformerPipeline.cu:171-176)
         // and on the first gulp after the beamsets change
@@ -917,17 +922,24 @@ int run_gulp(sw_pipeline* p, const void* in, hipEvent_t consumed)
     SW_HIP_TRY(hipEventRecord(p->ev[3], st));
 
     const size_t T2 = p->tout();
+    hipEvent_t e_last = p->ev[3];  // the end of the last stage so far
+    std::vector<std::array<hipEvent_t, 4>> e_dm(c.ndms);  // as ev_dm
     for(int dm = 0; dm < c.ndms; ++dm) {
         if(wk) {  // this DM's output buffers of this gulp parity, once their last blocks are delivered
             p->cb_out = p->cb_bufs[2 * dm + par];
             p->ib_q = p->ib_bufs[2 * dm + par];
             wk->wait_free(p->cb_out);
             wk->wait_free(p->ib_q);
+            e_last = p->ev_dm[4 * dm];  // the wait may have left the stream idle
+            SW_HIP_TRY(hipEventRecord(e_last, st));
         }
-        SW_HIP_TRY(hipEventRecord(p->ev_dm[4 * dm], st));
-        rc = enqueue_beams(p, dm, ring_direct, fuse_ib, st, p->ev_dm[4 * dm + 1]);
+        auto& e = e_dm[dm];
+        e[0] = e_last;
+        e[1] = fuse_ib ? e_last : p->ev_dm[4 * dm + 1];
+        rc = enqueue_beams(p, dm, ring_direct, fuse_ib, st, fuse_ib ? nullptr : e[1]);
         if(rc) return rc;
-        SW_HIP_TRY(hipEventRecord(p->ev_dm[4 * dm + 2], st));
+        e[2] = e[3] = e_last = p->ev_dm[4 * dm + 2];
+        SW_HIP_TRY(hipEventRecord(e_last, st));
         sw_block blk, iblk;
         double utc = 0;
         dm_blocks(p, dm, utc_offset_gulp, blk, iblk, utc);
@@ -947,9 +959,11 @@ int run_gulp(sw_pipeline* p, const void* in, hipEvent_t consumed)
             rc = sw_idpipe_push(p->idp, dm, p->cb_out, T2, 1, utc, blk.tsamp, st);
             if(rc) return rc;
         }
-        SW_HIP_TRY(hipEventRecord(p->ev_dm[4 * dm + 3], st));
+        if(p->idp || (!wk && (p->cb_sink || p->ib_sink))) {  // handlers called in line take their time
+            e[3] = e_last = p->ev_dm[4 * dm + 3];
+            SW_HIP_TRY(hipEventRecord(e_last, st));
+        }
     }
-    SW_HIP_TRY(hipEventRecord(p->ev[4], st));
     {
         sw_block blk;
         stats_block(p, utc_offset_gulp, blk);
@@ -964,25 +978,28 @@ int run_gulp(sw_pipeline* p, const void* in, hipEvent_t consumed)
     // per-stage device times of this gulp
     float t = 0;
     for(int i = 0; i < SW_NSTAGES; ++i) p->stage_ms[i] = 0;
-    SW_HIP_TRY(hipEventElapsedTime(&t, p->ev[0], p->ev[1]));
+    // (the statistics, stage 1, run inside the transpose)
+    SW_HIP_TRY(hipEventElapsedTime(&t, e_start, p->ev[1]));
     p->stage_ms[0] = t;
-    SW_HIP_TRY(hipEventElapsedTime(&t, p->ev[1], p->ev[2]));
-    p->stage_ms[1] = t;
-    SW_HIP_TRY(hipEventElapsedTime(&t, p->ev[2], p->ev[3]));
+    SW_HIP_TRY(hipEventElapsedTime(&t, p->ev[1], p->ev[3]));
     p->stage_ms[2] = t;
-    for(int dm = 0; dm < c.ndms; ++dm) {
-        SW_HIP_TRY(hipEventElapsedTime(&t, p->ev_dm[4 * dm], p->ev_dm[4 * dm + 1]));
-        p->stage_ms[3] += t;
-        SW_HIP_TRY(hipEventElapsedTime(&t, p->ev_dm[4 * dm + 1], p->ev_dm[4 * dm + 2]));
+    for(const auto& e : e_dm) {
+        if(e[0] != e[1]) {
+            SW_HIP_TRY(hipEventElapsedTime(&t, e[0], e[1]));
+            p->stage_ms[3] += t;
+        }
+        SW_HIP_TRY(hipEventElapsedTime(&t, e[1], e[2]));
         p->stage_ms[4] += t;
         if(p->idp) {
-            SW_HIP_TRY(hipEventElapsedTime(&t, p->ev_dm[4 * dm + 2], p->ev_dm[4 * dm + 3]));
+            SW_HIP_TRY(hipEventElapsedTime(&t, e[2], e[3]));
             p->stage_ms[5] += t;
         }
     }
-    SW_HIP_TRY(hipEventElapsedTime(&t, p->ev_w[0], p->ev_w[1]));
-    p->stage_ms[6] = t;
-    SW_HIP_TRY(hipEventElapsedTime(&t, p->ev[0], p->ev[4]));
+    if(p->delays) {
+        SW_HIP_TRY(hipEventElapsedTime(&t, p->ev_w[0], p->ev_w[1]));
+        p->stage_ms[6] = t;
+    }
+    SW_HIP_TRY(hipEventElapsedTime(&t, e_start, e_last));
     p->stage_ms[7] = t - (p->stage_ms[0] + p->stage_ms[1] + p->stage_ms[2] + p->stage_ms[3] + p->stage_ms[4] +
                           p->stage_ms[5]);
     ++p->call_count;
@@ -1080,8 +1097,10 @@ int run_gulp_graph(sw_pipeline* p, const void* in, hipEvent_t consumed, int par,
     // the graph is timed as a whole: its time is reported as "other"
     float t = 0;
     for(int i = 0; i < SW_NSTAGES; ++i) p->stage_ms[i] = 0;
-    SW_HIP_TRY(hipEventElapsedTime(&t, p->ev_w[0], p->ev_w[1]));
-    p->stage_ms[6] = t;
+    if(p->delays) {
+        SW_HIP_TRY(hipEventElapsedTime(&t, p->ev_w[0], p->ev_w[1]));
+        p->stage_ms[6] = t;
+    }
     SW_HIP_TRY(hipEventElapsedTime(&t, p->ev[0], p->ev[4]));
     p->stage_ms[7] = t;
     ++p->call_count;
