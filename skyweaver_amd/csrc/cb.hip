@@ -447,7 +447,7 @@ cb_mfma_kernel(const uint8_t* __restrict__ ftpa, const uint8_t* __restrict__ pac
     constexpr int LPR = A / 4 > 0 ? A / 4 : 1;  // lanes per row
     constexpr int RPI = 64 / LPR;               // rows per read
     unsigned ibm[4] = {0, 0, 0, 0};
-    if constexpr(TMI && S == SW_STOKES_I && kPre && 256 % A == 0 && TS >= RPI) {
+    if constexpr(TMI && S == SW_STOKES_I && kPre && 256 % A == 0 && TS >= RPI && TS >= 4) {
         if(fib.raw) {
 #pragma unroll
             for(int j = 0; j < 4; ++j) {
@@ -472,7 +472,7 @@ cb_mfma_kernel(const uint8_t* __restrict__ ftpa, const uint8_t* __restrict__ pac
                 *reinterpret_cast<uint16_t*>(stg + (8 * q + j) * SPITCH + c * 2) = (uint16_t)(w[j >> 1] >> (16 * (j & 1)));
         }
         __syncthreads();
-        if constexpr(S == SW_STOKES_I && kPre && 256 % A == 0 && TS >= RPI) {
+        if constexpr(S == SW_STOKES_I && kPre && 256 % A == 0 && TS >= RPI && TS >= 4) {
             if(fib.raw) {  // uniform: the incoherent beam from the staged rows
                 const int o0 = tc * NO_WG;
                 const int r0 = lane / LPR, g = lane % LPR;
@@ -480,38 +480,59 @@ cb_mfma_kernel(const uint8_t* __restrict__ ftpa, const uint8_t* __restrict__ pac
                 // antennas are summed by one dot product, no masks
                 const bool all1 =
                     nbeamsets == 1 && __all(((ibm[0] & ibm[1] & ibm[2] & ibm[3]) & 3u) == 3u);
+                // the wave's own rows, OW outputs: their sums and shuffle
+                // trees side by side, then lane k finishes output k (one
+                // output after the other, each tree and each division was a
+                // latency of its own: 64 beams of 64 channels x 8192 samples
+                // at tscrunch 4 took 120 us, now 88)
+                constexpr int OW = NO_WG / WV;
+                int lo[OW][4], hi[OW][4], tot[OW];
 #pragma unroll
-                for(int oi = 0; oi < NO_WG / WV; ++oi) {
-                    const int o = wave * (NO_WG / WV) + oi;  // this wave's own rows
-                    int lo[4] = {0, 0, 0, 0}, hi[4] = {0, 0, 0, 0}, tot = 0;
+                for(int oi = 0; oi < OW; ++oi) {
+                    const int o = wave * OW + oi;
+                    tot[oi] = 0;
+#pragma unroll
+                    for(int j = 0; j < 4; ++j) lo[oi][j] = hi[oi][j] = 0;
 #pragma unroll
                     for(int i = 0; i < TS / RPI; ++i) {
                         const uint4 v = *reinterpret_cast<const uint4*>(stg + (o * TS + RPI * i + r0) * SPITCH + 16 * g);
                         const int w[4] = {(int)v.x, (int)v.y, (int)v.z, (int)v.w};
                         if(all1) {
 #pragma unroll
-                            for(int j = 0; j < 4; ++j) tot = __builtin_amdgcn_sdot4(w[j], w[j], tot, false);
+                            for(int j = 0; j < 4; ++j) tot[oi] = __builtin_amdgcn_sdot4(w[j], w[j], tot[oi], false);
                         } else {
 #pragma unroll
                             for(int j = 0; j < 4; ++j) {
-                                lo[j] = __builtin_amdgcn_sdot4(w[j], w[j] & 0xFFFF, lo[j], false);
-                                hi[j] = __builtin_amdgcn_sdot4(w[j], (int)((unsigned)w[j] & 0xFFFF0000u), hi[j], false);
+                                lo[oi][j] = __builtin_amdgcn_sdot4(w[j], w[j] & 0xFFFF, lo[oi][j], false);
+                                hi[oi][j] = __builtin_amdgcn_sdot4(w[j], (int)((unsigned)w[j] & 0xFFFF0000u), hi[oi][j], false);
                             }
                         }
                     }
-                    for(int sb = 0; sb < nbeamsets; ++sb) {
-                        int part = tot;
+                }
+                for(int sb = 0; sb < nbeamsets; ++sb) {
+                    int part[OW];
+#pragma unroll
+                    for(int oi = 0; oi < OW; ++oi) {
+                        part[oi] = tot[oi];
                         if(!all1) {
 #pragma unroll
                             for(int j = 0; j < 4; ++j) {
-                                if(ibm[j] >> (2 * sb) & 1u) part += lo[j];
-                                if(ibm[j] >> (2 * sb) & 2u) part += hi[j];
+                                if(ibm[j] >> (2 * sb) & 1u) part[oi] += lo[oi][j];
+                                if(ibm[j] >> (2 * sb) & 2u) part[oi] += hi[oi][j];
                             }
                         }
+                    }
 #pragma unroll
-                        for(int m = 32; m > 0; m >>= 1) part += __shfl_xor(part, m, 64);
-                        float power = (float)part;  // the float chain's value while below 2^24
-                        if(part >= (1 << 24)) {     // the oracle's float chain: time, then antenna ascending
+                    for(int m = 32; m > 0; m >>= 1)
+#pragma unroll
+                        for(int oi = 0; oi < OW; ++oi) part[oi] += __shfl_xor(part[oi], m, 64);
+                    int sum = part[0];
+#pragma unroll
+                    for(int oi = 1; oi < OW; ++oi) sum = lane == oi ? part[oi] : sum;
+                    if(lane < OW) {
+                        const int o = wave * OW + lane;
+                        float power = (float)sum;  // the float chain's value while below 2^24
+                        if(sum >= (1 << 24)) {     // the oracle's float chain: time, then antenna ascending
                             power = 0.0f;
                             for(int tt = 0; tt < TS; ++tt) {
                                 const uint8_t* r = stg + (o * TS + tt) * SPITCH;
@@ -525,15 +546,13 @@ cb_mfma_kernel(const uint8_t* __restrict__ ftpa, const uint8_t* __restrict__ pac
                                 }
                             }
                         }
-                        if(lane == 0) {
-                            if(o0 + o < nsamps_out) {
-                                const size_t oi2 = ((size_t)sb * nsamps_out + o0 + o) * nchans + f;
-                                fib.raw[oi2] = power;
-                                fib.out[oi2] = clamp_i8(rescale<SW_STOKES_I>(power, fib.offset[sb * nchans + f],
-                                                                             fib.scale[sb * nchans + f]));
-                            }
-                            if(tabs) tb_ib[sb * NO_WG + o] = ib_sub ? power : 0.0f;
+                        if(o0 + o < nsamps_out) {
+                            const size_t oi2 = ((size_t)sb * nsamps_out + o0 + o) * nchans + f;
+                            fib.raw[oi2] = power;
+                            fib.out[oi2] = clamp_i8(rescale<SW_STOKES_I>(power, fib.offset[sb * nchans + f],
+                                                                         fib.scale[sb * nchans + f]));
                         }
+                        if(tabs) tb_ib[sb * NO_WG + o] = ib_sub ? power : 0.0f;
                     }
                 }
             }

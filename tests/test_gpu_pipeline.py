@@ -654,3 +654,39 @@ def test_pipeline_table_fft_lengths_must_fit_the_band(sw, dev, tmp_path):
     p.close()
     assert t["cb_waves"] == 2 and t["source"] == "table"
     assert t["fft_len"][0] > 1024
+
+
+@pytest.mark.parametrize("A,ts,S", [(64, 4, 1), (64, 4, 3), (64, 32, 2), (128, 4, 2), (16, 16, 1), (32, 8, 4)])
+def test_pipeline_fused_ib_outputs(sw, orc, dev, A, ts, S):
+    """The incoherent beam inside the beamformer, one to eight outputs a wave, one beamset over all
+    antennas and several over some; full-scale samples push outputs to 2^24 and past it where the
+    shape allows, to the float chain."""
+    F, B, H = 3, 40, 8
+    taftp = sw.synth_voltages((H, A, F, 256, 2, 2), seed=77 + A + ts, sigma=30.0)
+    taftp[0, :, 0, :64] = -128
+    weights = sw.synth_weights((F, B, A, 2), seed=5)
+    antw = np.ones((S, A), np.float32)
+    for s in range(1, S):
+        antw[s, s::s + 1] = 0
+    bmap = (np.arange(B) % S).astype(np.int32)
+    p = sw.BeamformerPipeline(A, F, B, H * 256, ts, [0.0], 1284e6, 13.375e6 * F / 64, fft_len=[1024])
+    p.set_weights(weights)
+    p.set_beamsets(bmap, antw)
+    p.init(A)
+    got = {}
+
+    def grab(key):
+        def f(blk):
+            got[key] = sw.download_block(blk)
+        return f
+    p.set_sinks(cb=grab("cb"), ib=grab("ib"), stats=grab("stats"))
+    p(sw.DeviceBuffer.from_host(taftp))
+    p.close()
+    ftpa = orc.transpose(taftp, A)
+    stats = got["stats"].view(np.float32).reshape(F, 2, A, 4)
+    scal = orc.update_scalings(stats[..., 1], antw, S, ts, ts, 24.0)
+    raw, ib = orc.ib_beamform(ftpa, ts, scal["ib_scaling"], scal["ib_offsets"], antw, S, "I")
+    assert (raw >= 2 ** 24).any() == (A * ts >= 256)
+    cb = orc.cb_beamform(ftpa, weights, ts, scal["cb_scaling"], scal["cb_offsets"], antw, bmap, S, "I", True)
+    np.testing.assert_array_equal(got["ib"].view(np.int8).reshape(ib.shape), ib)
+    np.testing.assert_array_equal(got["cb"].view(np.int8).reshape(cb.shape), cb)
