@@ -817,7 +817,8 @@ constexpr size_t cb_mfma_lds_bytes()
 
 // workgroup shapes (waves of 32 time rows) instantiated per form: the
 // pipeline's forms (Stokes I, on the ring or on FTPA, and full Stokes on
-// FTPA) take 2, 4 or 8 waves, the others 4
+// FTPA) take 2, 4 or 8 waves, the others (full Stokes on the ring among
+// them) 4
 template <int S, bool TMI>
 constexpr bool cb_wave_variants()
 {
@@ -949,7 +950,7 @@ extern "C" int sw_cb_pack_weights(const void* d_weights, void* d_packed, int nch
 }
 
 namespace sw {
-// The MFMA form on the coherent dedisperser's time-major ring (Stokes I):
+// The MFMA form on the coherent dedisperser's time-major ring (Stokes I or IQUV):
 // sample t of column (f, p, a) at d_ring + ((f 2A + p A + a) ld + w0 + t) 2.
 // With d_ib_out_raw non-null the incoherent beam is computed here too (see
 // FusedIb; requires cb_fused_ib_supported) and written to d_ib_out_raw /
@@ -966,7 +967,8 @@ int cb_beamform_packed_tm(const void* d_ring, long ld, long w0, const void* d_pa
     SW_CHECK_ARG((reinterpret_cast<uintptr_t>(d_ring) & 15) == 0 && (reinterpret_cast<uintptr_t>(d_packed) & 15) == 0
                      && ld % 8 == 0 && w0 % 8 == 0 && d.nsamples % 8 == 0,
                  "ring and packed weights must be 16-byte aligned, rows 8-sample aligned");
-    SW_CHECK_ARG(d.stokes == SW_STOKES_I, "time-major beamformer input: Stokes I only");
+    SW_CHECK_ARG(d.stokes == SW_STOKES_I || (d.stokes == SW_STOKES_IQUV && waves == kMfmaWaves),
+                 "time-major beamformer input: Stokes I, or IQUV with 4 waves, only");
     if(!cb_mfma_supported(d)) {
         set_error("cb_beamform_packed_tm: shape not supported by the MFMA form");
         return SW_ERR_UNSUPPORTED;
@@ -982,12 +984,15 @@ int cb_beamform_packed_tm(const void* d_ring, long ld, long w0, const void* d_pa
     auto* out = static_cast<int8_t*>(d_out);
     // every scale checked by the caller: the division by div_by, for the
     // 64-antenna, 4-wave shapes at tscrunch 16 and 8
-    if(fastdiv && waves == kMfmaWaves && d.nantennas == 64 && d.tscrunch == 16)
+    if(fastdiv && d.stokes == SW_STOKES_I && waves == kMfmaWaves && d.nantennas == 64 && d.tscrunch == 16)
         return launch_mfma_wv<SW_STOKES_I, 16, 4, true, kMfmaWaves, true>(ring, pk, out, d_scale, d_offset,
                                                                           d_beamset_map, d_ib_raw, d, st, ld, w0, fib);
-    if(fastdiv && waves == kMfmaWaves && d.nantennas == 64 && d.tscrunch == 8)
+    if(fastdiv && d.stokes == SW_STOKES_I && waves == kMfmaWaves && d.nantennas == 64 && d.tscrunch == 8)
         return launch_mfma_wv<SW_STOKES_I, 8, 4, true, kMfmaWaves, true>(ring, pk, out, d_scale, d_offset,
                                                                          d_beamset_map, d_ib_raw, d, st, ld, w0, fib);
+    if(d.stokes == SW_STOKES_IQUV)
+        return launch_mfma<SW_STOKES_IQUV, true>(ring, pk, out, d_scale, d_offset, d_beamset_map, d_ib_raw, d, st, ld,
+                                                 w0, fib, waves);
     return launch_mfma<SW_STOKES_I, true>(ring, pk, out, d_scale, d_offset, d_beamset_map, d_ib_raw, d, st, ld, w0,
                                           fib, waves);
 }

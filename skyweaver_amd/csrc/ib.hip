@@ -66,6 +66,24 @@ struct IbSums {
     __device__ __forceinline__ int vv() const { return 2 * (int)((uint32_t)v0 - (uint32_t)v1); }
 };
 
+// Output o: the powers, and the powers requantised
+template <int S>
+__device__ __forceinline__ void ib_store(float* raw, int8_t* out, size_t o, const float* power, float off, float sc)
+{
+    if constexpr(nstokes(S) == 1) {
+        raw[o] = power[0];
+        out[o] = clamp_i8(rescale<S>(power[0], off, sc));
+    } else {
+        reinterpret_cast<float4*>(raw)[o] = make_float4(power[0], power[1], power[2], power[3]);
+        char4 q;
+        q.x = clamp_i8(rescale<SW_STOKES_I>(power[0], off, sc));
+        q.y = clamp_i8(rescale<SW_STOKES_Q>(power[1], off, sc));
+        q.z = clamp_i8(rescale<SW_STOKES_U>(power[2], off, sc));
+        q.w = clamp_i8(rescale<SW_STOKES_V>(power[3], off, sc));
+        reinterpret_cast<char4*>(out)[o] = q;
+    }
+}
+
 // the sum over `lanes` (a power of two) neighbouring lanes
 __device__ __forceinline__ int lanes_sum(int v, int lanes)
 {
@@ -100,21 +118,8 @@ ib_kernel(const uint8_t* __restrict__ ftpa, float* __restrict__ raw, int8_t* __r
     const uint8_t* chan = ftpa + (size_t)f * nsamples * 4 * nant;
 
     auto store = [&](int s, int tp, const float* power) {
-        const size_t o  = ((size_t)s * nsamps_out + tp) * nchans + f;
-        const float sc  = scale[s * nchans + f];
-        const float off = offset[s * nchans + f];
-        if constexpr(NV == 1) {
-            raw[o] = power[0];
-            out[o] = clamp_i8(rescale<S>(power[0], off, sc));
-        } else {
-            reinterpret_cast<float4*>(raw)[o] = make_float4(power[0], power[1], power[2], power[3]);
-            char4 q;
-            q.x = clamp_i8(rescale<SW_STOKES_I>(power[0], off, sc));
-            q.y = clamp_i8(rescale<SW_STOKES_Q>(power[1], off, sc));
-            q.z = clamp_i8(rescale<SW_STOKES_U>(power[2], off, sc));
-            q.w = clamp_i8(rescale<SW_STOKES_V>(power[3], off, sc));
-            reinterpret_cast<char4*>(out)[o] = q;
-        }
+        ib_store<S>(raw, out, ((size_t)s * nsamps_out + tp) * nchans + f, power, offset[s * nchans + f],
+                    scale[s * nchans + f]);
     };
 
     // ---- exact integer path
@@ -258,87 +263,113 @@ ib_kernel(const uint8_t* __restrict__ ftpa, float* __restrict__ raw, int8_t* __r
 }
 
 // Time-major input (the coherent dedisperser's ring): sample t of column
-// c = p A + a of channel f at ring + ((f 2A + c) ld + w0 + t) 2.  Stokes I
-// with 0/1 antenna weights only.  One lane per output sample t' of channel
-// f; a lane reads its ts consecutive samples of every column (64 lanes read
-// 64 ts 2 contiguous bytes), sums re^2 + im^2 of the column with
-// v_dot4_i32_i8 and adds the column sum to the beamsets that weight the
-// antenna 1.  As in ib_kernel the integer total equals the oracle's float
-// chain while below 2^24; a lane at or above it recomputes its outputs with
-// the float chain in the oracle's order (time, then antenna ascending).
-constexpr int kTmThreads = 256;
-constexpr int kTmMaxCols = 256;  // 128 antennas
+// c = p A + a of channel f at ring + ((f 2A + c) ld + w0 + t) 2.  0/1 antenna
+// weights only.  A workgroup owns 64 outputs t' of channel f; its four waves
+// take every fourth antenna, a lane reading its output's ts consecutive
+// samples of both polarisations (64 lanes read 64 ts 2 contiguous bytes) and
+// adding the antenna's integer sums to the beamsets that weight it 1; the
+// waves' sums meet in LDS.  HBM-bound (a workgroup per 256 outputs, one lane
+// summing all antennas, left half of the CUs idle at 16 channels x 2048
+// outputs).  As in ib_kernel the integer totals equal the oracle's float
+// chains while Stokes I is below 2^24; a lane at or above it recomputes its
+// outputs with the float chains in the oracle's order (time, then antenna
+// ascending).
+constexpr int kTmOut = 64, kTmWaves = 4;
+constexpr int kTmMaxAnts = 128;
 
-template <int SMAX, bool V16>
-__global__ void __launch_bounds__(kTmThreads)
+template <int S, int SMAX, bool V16>
+__global__ void __launch_bounds__(kTmOut * kTmWaves)
 ib_tm_kernel(const uint8_t* __restrict__ ring, long ld, long w0, float* __restrict__ raw,
              int8_t* __restrict__ out, const float* __restrict__ scale, const float* __restrict__ offset,
              const float* __restrict__ antw, int nchans, int nsamples, int nant, int ts, int nbeamsets)
 {
-    __shared__ uint8_t colw[SMAX][kTmMaxCols];  // weight (0/1) of column c in beamset s
-    const int PA = 2 * nant;
-    for(int i = threadIdx.x; i < nbeamsets * PA; i += kTmThreads) {
-        const int sb = i / PA, c = i % PA;
-        colw[sb][c] = antw[sb * nant + c % nant] != 0.0f ? 1 : 0;
-    }
+    constexpr int NV = nstokes(S);
+    __shared__ uint8_t antb[SMAX][kTmMaxAnts];  // weight (0/1) of antenna a in beamset s
+    __shared__ int red[kTmWaves][4][kTmOut];
+    for(int i = threadIdx.x; i < nbeamsets * nant; i += kTmOut * kTmWaves)
+        antb[i / nant][i % nant] = antw[i] != 0.0f ? 1 : 0;
     __syncthreads();
     const int f = blockIdx.y;
+    const int lane = threadIdx.x % kTmOut, wave = threadIdx.x / kTmOut;
     const int nsamps_out = nsamples / ts;
-    const int tp = blockIdx.x * kTmThreads + threadIdx.x;
-    if(tp >= nsamps_out) return;  // after the only barrier
-    const uint8_t* base = ring + ((size_t)f * PA * ld + w0 + (size_t)tp * ts) * 2;
-    int isum[SMAX];
+    const int tp = blockIdx.x * kTmOut + lane;
+    const bool active = tp < nsamps_out;
+    const uint8_t* base = ring + ((size_t)f * 2 * nant * ld + w0 + (size_t)(active ? tp : 0) * ts) * 2;
+    int si[SMAX], sq[SMAX], su[SMAX], sv[SMAX];
 #pragma unroll
-    for(int s = 0; s < SMAX; ++s) isum[s] = 0;
-#pragma unroll 4
-    for(int c = 0; c < PA; ++c) {
-        const uint8_t* x = base + (size_t)c * ld * 2;
-        int acc = 0;  // sum over the window of re^2 + im^2 of column c
+    for(int s = 0; s < SMAX; ++s) si[s] = sq[s] = su[s] = sv[s] = 0;
+#pragma unroll 2
+    for(int a = wave; a < nant; a += kTmWaves) {
+        const uint8_t* x0 = base + (size_t)a * ld * 2;
+        const uint8_t* x1 = base + (size_t)(nant + a) * ld * 2;
+        IbSums<S> c;
         if constexpr(V16) {  // ts % 8 == 0: 16-byte aligned runs
             for(int k = 0; k < ts * 2; k += 16) {
-                const uint4 v = *reinterpret_cast<const uint4*>(x + k);
-                acc = __builtin_amdgcn_sdot4((int)v.x, (int)v.x, acc, false);
-                acc = __builtin_amdgcn_sdot4((int)v.y, (int)v.y, acc, false);
-                acc = __builtin_amdgcn_sdot4((int)v.z, (int)v.z, acc, false);
-                acc = __builtin_amdgcn_sdot4((int)v.w, (int)v.w, acc, false);
+                const uint4 v = *reinterpret_cast<const uint4*>(x0 + k), w = *reinterpret_cast<const uint4*>(x1 + k);
+                c.add(v.x, w.x, ~0u);
+                c.add(v.y, w.y, ~0u);
+                c.add(v.z, w.z, ~0u);
+                c.add(v.w, w.w, ~0u);
             }
         } else {
-            for(int k = 0; k < ts; ++k) {
-                const int v = (int)*reinterpret_cast<const uint16_t*>(x + 2 * k);
-                acc = __builtin_amdgcn_sdot4(v, v, acc, false);
-            }
+            for(int k = 0; k < ts; ++k)
+                c.add(*reinterpret_cast<const uint16_t*>(x0 + 2 * k), *reinterpret_cast<const uint16_t*>(x1 + 2 * k), ~0u);
         }
 #pragma unroll
         for(int s = 0; s < SMAX; ++s)
-            if(s < nbeamsets && colw[s][c]) isum[s] += acc;
-    }
-    float power[SMAX];
-    bool big = false;
-#pragma unroll
-    for(int s = 0; s < SMAX; ++s) {
-        big = big || isum[s] >= (1 << 24);
-        power[s] = (float)isum[s];
-    }
-    if(big) {  // the oracle's float chain
-#pragma unroll
-        for(int s = 0; s < SMAX; ++s) power[s] = 0.0f;
-        for(int tt = 0; tt < ts; ++tt)
-            for(int a = 0; a < nant; ++a) {
-                const uint16_t d0 = *reinterpret_cast<const uint16_t*>(base + ((size_t)a * ld + tt) * 2);
-                const uint16_t d1 = *reinterpret_cast<const uint16_t*>(base + ((size_t)(nant + a) * ld + tt) * 2);
-                const float st = stokes<SW_STOKES_I>((float)(int8_t)d0, (float)(int8_t)(d0 >> 8),
-                                                     (float)(int8_t)d1, (float)(int8_t)(d1 >> 8));
-#pragma unroll
-                for(int s = 0; s < SMAX; ++s)
-                    if(s < nbeamsets) power[s] += st * antw[s * nant + a];
+            if(s < nbeamsets && antb[s][a]) {
+                si[s] += c.total();  // at most 2^24 each
+                if constexpr(S == SW_STOKES_Q || NV == 4) sq[s] += c.q();
+                if constexpr(S == SW_STOKES_U || NV == 4) su[s] += c.uu();
+                if constexpr(S == SW_STOKES_V || NV == 4) sv[s] += c.vv();
             }
     }
 #pragma unroll
     for(int s = 0; s < SMAX; ++s) {
-        if(s < nbeamsets) {
-            const size_t o = ((size_t)s * nsamps_out + tp) * nchans + f;
-            raw[o] = power[s];
-            out[o] = clamp_i8(rescale<SW_STOKES_I>(power[s], offset[s * nchans + f], scale[s * nchans + f]));
+        if(s < nbeamsets) {  // uniform
+            if(s) __syncthreads();
+            red[wave][0][lane] = min(si[s], kExact);
+            if constexpr(S != SW_STOKES_I) {
+                red[wave][1][lane] = sq[s];
+                red[wave][2][lane] = su[s];
+                red[wave][3][lane] = sv[s];
+            }
+            __syncthreads();
+            if(wave == 0 && active) {
+                int t[4];
+#pragma unroll
+                for(int k = 0; k < (S == SW_STOKES_I ? 1 : 4); ++k)
+                    t[k] = red[0][k][lane] + red[1][k][lane] + red[2][k][lane] + red[3][k][lane];
+                float power[NV];
+                if constexpr(NV == 4) {
+#pragma unroll
+                    for(int k = 0; k < 4; ++k) power[k] = (float)t[k];
+                } else {
+                    power[0] = (float)t[S == SW_STOKES_I ? 0 : S == SW_STOKES_Q ? 1 : S == SW_STOKES_U ? 2 : 3];
+                }
+                if(t[0] >= kExact) {  // the oracle's float chains
+#pragma unroll
+                    for(int k = 0; k < NV; ++k) power[k] = 0.0f;
+                    for(int tt = 0; tt < ts; ++tt)
+                        for(int a = 0; a < nant; ++a) {
+                            const uint16_t d0 = *reinterpret_cast<const uint16_t*>(base + ((size_t)a * ld + tt) * 2);
+                            const uint16_t d1 = *reinterpret_cast<const uint16_t*>(base + ((size_t)(nant + a) * ld + tt) * 2);
+                            const float r0 = (float)(int8_t)d0, i0 = (float)(int8_t)(d0 >> 8);
+                            const float r1 = (float)(int8_t)d1, i1 = (float)(int8_t)(d1 >> 8);
+                            const float w = antw[s * nant + a];
+                            if constexpr(NV == 1) {
+                                power[0] += stokes<S>(r0, i0, r1, i1) * w;
+                            } else {
+                                power[0] += stokes<SW_STOKES_I>(r0, i0, r1, i1) * w;
+                                power[1] += stokes<SW_STOKES_Q>(r0, i0, r1, i1) * w;
+                                power[2] += stokes<SW_STOKES_U>(r0, i0, r1, i1) * w;
+                                power[3] += stokes<SW_STOKES_V>(r0, i0, r1, i1) * w;
+                            }
+                        }
+                }
+                ib_store<S>(raw, out, ((size_t)s * nsamps_out + tp) * nchans + f, power, offset[s * nchans + f],
+                            scale[s * nchans + f]);
+            }
         }
     }
 }
@@ -390,30 +421,37 @@ int launch_ib(const uint8_t* ftpa, float* raw, int8_t* out, const float* scale,
 } // namespace
 
 // Incoherent beam from the dedisperser's time-major ring (see ib_tm_kernel):
-// Stokes I, 0/1 antenna weights, d.nantennas <= 128.
+// Stokes I or IQUV, 0/1 antenna weights, d.nantennas <= 128.
 int ib_beamform_tm(const void* d_ring, long ld, long w0, float* d_raw, void* d_out, const float* d_scale,
                    const float* d_offset, const float* d_ant_weights, const sw_bf_dims& d, hipStream_t st)
 {
     SW_CHECK_ARG(d_ring && d_raw && d_out && d_scale && d_offset && d_ant_weights, "null buffer");
-    SW_CHECK_ARG(d.stokes == SW_STOKES_I && 2 * d.nantennas <= kTmMaxCols, "time-major IB: Stokes I, <= 128 antennas");
+    SW_CHECK_ARG((d.stokes == SW_STOKES_I || d.stokes == SW_STOKES_IQUV) && d.nantennas <= kTmMaxAnts,
+                 "time-major IB: Stokes I or IQUV, <= 128 antennas");
     SW_CHECK_ARG(d.nbeamsets > 0 && d.nbeamsets <= 16 && d.nchans > 0 && d.nchans <= 65535, "bad dimensions");
     SW_CHECK_ARG(d.tscrunch > 0 && d.nsamples % d.tscrunch == 0, "nsamples must be a multiple of tscrunch");
     SW_CHECK_ARG((reinterpret_cast<uintptr_t>(d_ring) & 15) == 0 && ld % 8 == 0 && w0 % 8 == 0,
                  "ring must be 16-byte aligned with 8-sample aligned rows");
     const int nout = d.nsamples / d.tscrunch;
-    const dim3 grid((nout + kTmThreads - 1) / kTmThreads, d.nchans);
+    const dim3 grid((nout + kTmOut - 1) / kTmOut, d.nchans), block(kTmOut * kTmWaves);
     const bool v16 = d.tscrunch % 8 == 0;
     auto* in = static_cast<const uint8_t*>(d_ring);
     auto* out = static_cast<int8_t*>(d_out);
-#define SW_IBT(SM)                                                                                         \
-    if(v16)                                                                                                \
-        hipLaunchKernelGGL((ib_tm_kernel<SM, true>), grid, dim3(kTmThreads), 0, st, in, ld, w0, d_raw, out, \
-                           d_scale, d_offset, d_ant_weights, d.nchans, d.nsamples, d.nantennas, d.tscrunch, \
-                           d.nbeamsets);                                                                   \
-    else                                                                                                   \
-        hipLaunchKernelGGL((ib_tm_kernel<SM, false>), grid, dim3(kTmThreads), 0, st, in, ld, w0, d_raw, out,\
-                           d_scale, d_offset, d_ant_weights, d.nchans, d.nsamples, d.nantennas, d.tscrunch, \
-                           d.nbeamsets);
+#define SW_IBT_L(S, SM, V)                                                                                          \
+    hipLaunchKernelGGL((ib_tm_kernel<S, SM, V>), grid, block, 0, st, in, ld, w0, d_raw, out, d_scale, d_offset,     \
+                       d_ant_weights, d.nchans, d.nsamples, d.nantennas, d.tscrunch, d.nbeamsets)
+#define SW_IBT(SM)                                                  \
+    if(d.stokes == SW_STOKES_I) {                                   \
+        if(v16)                                                     \
+            SW_IBT_L(SW_STOKES_I, SM, true);                        \
+        else                                                        \
+            SW_IBT_L(SW_STOKES_I, SM, false);                       \
+    } else {                                                        \
+        if(v16)                                                     \
+            SW_IBT_L(SW_STOKES_IQUV, SM, true);                     \
+        else                                                        \
+            SW_IBT_L(SW_STOKES_IQUV, SM, false);                    \
+    }
     if(d.nbeamsets <= 1) {
         SW_IBT(1)
     } else if(d.nbeamsets <= 4) {
@@ -422,6 +460,7 @@ int ib_beamform_tm(const void* d_ring, long ld, long w0, float* d_raw, void* d_o
         SW_IBT(16)
     }
 #undef SW_IBT
+#undef SW_IBT_L
     SW_LAUNCH_CHECK();
     return SW_OK;
 }

@@ -656,11 +656,9 @@ def test_pipeline_table_fft_lengths_must_fit_the_band(sw, dev, tmp_path):
     assert t["fft_len"][0] > 1024
 
 
-@pytest.mark.parametrize("A,ts,S", [(64, 4, 1), (64, 4, 3), (64, 32, 2), (128, 4, 2), (16, 16, 1), (32, 8, 4)])
-def test_pipeline_fused_ib_outputs(sw, orc, dev, A, ts, S):
-    """The incoherent beam inside the beamformer, one to eight outputs a wave, one beamset over all
-    antennas and several over some; full-scale samples push outputs to 2^24 and past it where the
-    shape allows, to the float chain."""
+def _check_beams_at_dm0(sw, orc, A, ts, S, stokes):
+    """One gulp at DM 0 against the oracle, bit for bit, with full-scale samples that push outputs
+    to 2^24 and past it where the shape allows, to the float chain."""
     F, B, H = 3, 40, 8
     taftp = sw.synth_voltages((H, A, F, 256, 2, 2), seed=77 + A + ts, sigma=30.0)
     taftp[0, :, 0, :64] = -128
@@ -669,7 +667,8 @@ def test_pipeline_fused_ib_outputs(sw, orc, dev, A, ts, S):
     for s in range(1, S):
         antw[s, s::s + 1] = 0
     bmap = (np.arange(B) % S).astype(np.int32)
-    p = sw.BeamformerPipeline(A, F, B, H * 256, ts, [0.0], 1284e6, 13.375e6 * F / 64, fft_len=[1024])
+    p = sw.BeamformerPipeline(A, F, B, H * 256, ts, [0.0], 1284e6, 13.375e6 * F / 64, stokes=stokes,
+                              fft_len=[1024])
     p.set_weights(weights)
     p.set_beamsets(bmap, antw)
     p.init(A)
@@ -685,8 +684,24 @@ def test_pipeline_fused_ib_outputs(sw, orc, dev, A, ts, S):
     ftpa = orc.transpose(taftp, A)
     stats = got["stats"].view(np.float32).reshape(F, 2, A, 4)
     scal = orc.update_scalings(stats[..., 1], antw, S, ts, ts, 24.0)
-    raw, ib = orc.ib_beamform(ftpa, ts, scal["ib_scaling"], scal["ib_offsets"], antw, S, "I")
+    raw, ib = orc.ib_beamform(ftpa, ts, scal["ib_scaling"], scal["ib_offsets"], antw, S, stokes)
     assert (raw >= 2 ** 24).any() == (A * ts >= 256)
-    cb = orc.cb_beamform(ftpa, weights, ts, scal["cb_scaling"], scal["cb_offsets"], antw, bmap, S, "I", True)
+    cb = orc.cb_beamform(ftpa, weights, ts, scal["cb_scaling"], scal["cb_offsets"], antw, bmap, S, stokes, True)
     np.testing.assert_array_equal(got["ib"].view(np.int8).reshape(ib.shape), ib)
     np.testing.assert_array_equal(got["cb"].view(np.int8).reshape(cb.shape), cb)
+
+
+@pytest.mark.parametrize("A,ts,S", [(64, 4, 1), (64, 4, 3), (64, 32, 2), (128, 4, 2), (16, 16, 1), (32, 8, 4)])
+def test_pipeline_fused_ib_outputs(sw, orc, dev, A, ts, S):
+    """The incoherent beam inside the beamformer: one to eight outputs a wave, one beamset over all
+    antennas and several over some."""
+    _check_beams_at_dm0(sw, orc, A, ts, S, "I")
+
+
+@pytest.mark.parametrize("stokes,A,ts,S", [("IQUV", 64, 16, 2), ("IQUV", 16, 4, 1), ("IQUV", 112, 32, 5),
+                                           ("IQUV", 128, 1, 1), ("IQUV", 48, 2, 3), ("IQUV", 32, 8, 4),
+                                           ("I", 48, 8, 3), ("I", 112, 2, 1), ("I", 80, 32, 5)])
+def test_pipeline_ring_beams(sw, orc, dev, stokes, A, ts, S):
+    """Beams from the ring with the incoherent beam in its own kernel: full Stokes, and Stokes I
+    at antenna counts that the beamformer does not fuse."""
+    _check_beams_at_dm0(sw, orc, A, ts, S, stokes)
