@@ -819,7 +819,7 @@ int sw::idisp_launch(sw_idisp* p, const void* d_tfb, size_t nsamples, int nbeams
             const int chunk0 = half ? nfull : 0, nchunks128 = half ? (last > 0 && last <= 64 && !big) : nfull;
             const long nwork = (ntiles + sw::kIdTileGroup - 1) / sw::kIdTileGroup * sw::kIdTileGroup * nchunks128 *
                                (((long)ntb + sw::kIdTbGroup - 1) / sw::kIdTbGroup * sw::kIdTbGroup);
-            const long max_launch = 4L << 20;  // work items per launch (grid x threads < 2^32)
+            const long max_launch = 2L << 20;  // work items per launch (grid x 1024 threads < 2^32)
             for(long w0 = 0; w0 < nwork; w0 += max_launch) {
                 const sw::IdArgs a{static_cast<const int8_t*>(d_tfb), static_cast<int8_t*>(d_tdb), p->d_rel,
                                    p->d_span, p->d_tiles, (int)ntiles, chunk0, nchunks128, ntb, w0,

@@ -128,6 +128,21 @@ def test_matrix_core_rows_past_32_bits(sw, orc, dev):
     np.testing.assert_array_equal(out[:, :, -16:], want[:, :, :16])
 
 
+def test_more_work_than_one_launch(sw, orc, dev):
+    # 4 tiles' work per time block (padded) of 32 samples: two million work items and a few more
+    F, B = 4, 4
+    idd = sw.IncoherentDedisperser(F, 1284e6, 13.375e6, 16, [0.0, 300.0])
+    D = idd.max_delay
+    assert D > 0
+    nout = 32 * (2 << 20) // 4 + 1000
+    x = _rand((65521, F, B), 12, sigma=40.0)
+    tfb = np.tile(x, ((nout + D) // len(x) + 1, 1, 1))[:nout + D]
+    out = _run(sw, idd, tfb, 1)
+    for t in (0, nout // 2, nout - 1200, nout - 200):
+        want = orc.incoherent_dedisperse(np.ascontiguousarray(tfb[t:t + D + 200]), idd.delays, D, 1)
+        np.testing.assert_array_equal(out[t:t + 200], want, err_msg=str(t))
+
+
 def test_saturating_sums(sw, orc, dev):
     # every input at the extremes: the quantised output clamps at -128 / 127
     F, B = 64, 32
