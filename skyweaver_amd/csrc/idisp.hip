@@ -324,7 +324,7 @@ __device__ __forceinline__ void idisp_tile(const IdArgs& p)
     // for every row load before any read)
     __shared__ __attribute__((aligned(16))) int8_t stage0[QB];
     __shared__ __attribute__((aligned(16))) int8_t stage1[QB];
-    __shared__ __attribute__((aligned(16))) int4 tab[kMfTabCh];  // offset of the first row (64 bits), bytes, rows
+    __shared__ __attribute__((aligned(16))) int4 tab[kMfTabCh];  // offset of the first row (64 bits), bytes (BIG: see below), rows
     __shared__ __attribute__((aligned(16))) uint8_t tab_rel[kMfTabCh * NW];  // [channel][wave]: rows to the DM's first
 
     const long per = (p.nwork + 7) / 8;
@@ -373,10 +373,11 @@ __device__ __forceinline__ void idisp_tile(const IdArgs& p)
         const int nr = __builtin_amdgcn_readfirstlane(e.w);
         const int8_t* src = p.in + ((unsigned long)hi << 32 | lo);
         if constexpr(BIG) {
+            const bool last = __builtin_amdgcn_readfirstlane(e.z) != 0;  // the last row ends the input
 #pragma unroll
             for(int k = 0; k < 4; ++k) {
                 const int rs = stored_row(k), b = piece(rs), r = rs % RP * TS + rs / RP;
-                const bool end = ragged && f0 + 4 * q + sc == p.nchans - 1 && r == nr - 1;
+                const bool end = last && r == nr - 1;
                 if(rs < RP * TS && r < nr && (end ? b + 16 <= p.W : b < p.W))
                     __builtin_amdgcn_global_load_lds(
                         src + (unsigned long)r * p.stride_t + b,
@@ -461,8 +462,9 @@ __device__ __forceinline__ void idisp_tile(const IdArgs& p)
             const int nr = (int)min((long)(TT * TS + sp.y - sp.x), p.nsamples - lo);
             // the input's very last piece, where it is no whole one, is finish()'s
             const bool end = ragged && f0 + i == p.nchans - 1 && lo + nr == p.nsamples;
+            // BIG has no use for the bytes: whether finish() loads that piece stands there
             const long bytes = (nr - 1) * p.stride_t + (end ? p.W & ~15 : p.W);
-            tab[i] = make_int4((int)at, (int)(at >> 32), (int)bytes, nr);
+            tab[i] = make_int4((int)at, (int)(at >> 32), BIG ? (int)end : (int)bytes, nr);
             using R = typename std::conditional<NW == 16, uint4, uint2>::type;
             reinterpret_cast<R*>(tab_rel)[i] =
                 reinterpret_cast<const R*>(p.rel)[(size_t)tile * p.nchans + f0 + i];

@@ -128,6 +128,27 @@ def test_matrix_core_rows_past_32_bits(sw, orc, dev):
     np.testing.assert_array_equal(out[:, :, -16:], want[:, :, :16])
 
 
+@pytest.mark.parametrize("ts,nout", [(1, 40), (2, 33), (4, 17)])
+def test_matrix_core_rows_past_32_bits_ragged(sw, orc, dev, ts, nout):
+    """As above with rows that end in a piece of 4 bytes, and a full time block before the last:
+    only the input's very last piece is loaded word by word."""
+    F, B = 1024, 32788
+    idd = sw.IncoherentDedisperser(F, 1284e6, 214e6, 16, np.arange(0, 0.6, 0.2, dtype=np.float32), tscrunch=ts)
+    T = idd.max_delay + ts * nout
+    x = _rand((T, F, 64), 9, sigma=40.0)
+    tfb = np.empty((T, F, B), np.int8)
+    for t in range(T):  # the beams repeat with period 64
+        tfb[t] = np.concatenate([np.tile(x[t], B // 64), x[t, :, :B % 64]], 1)
+    end = x[:, :, :B % 64].copy()
+    end[-1, -1, -4:] = tfb[-1, -1, -4:] = (-128, 127, -77, 101)
+    out = _run(sw, idd, tfb, 1)
+    want = orc.incoherent_dedisperse(x, idd.delays, idd.max_delay, ts)
+    body = out[:, :, :B // 64 * 64]
+    np.testing.assert_array_equal(body, np.tile(want, B // 64))
+    np.testing.assert_array_equal(out[:, :, B // 64 * 64:],
+                                  orc.incoherent_dedisperse(end, idd.delays, idd.max_delay, ts))
+
+
 def test_more_work_than_one_launch(sw, orc, dev):
     # 4 tiles' work per time block (padded) of 32 samples: two million work items and a few more
     F, B = 4, 4
