@@ -557,10 +557,14 @@ __global__ void __launch_bounds__(512) codedisp_reg_kernel(CdParams p, int d, in
 // chirp, inverse transform and stores run in turn, so a unit costs one
 // forward and p.ndm inverse transforms instead of p.ndm of each.  The next
 // unit's input is fetched during the last DM, once X is no longer needed,
-// and packed two to a register at once: one round trip per unit.  (Held one
-// to a register, in flight behind the last inverse or the forward
-// transform, it spilled 50-110 registers: eight DMs of 64 channels took 9.7
-// ms instead of 7.7.)
+// and packed two to a register at once: one round trip per unit, two at R1 =
+// 16, where 32 raw values beside X would spill 17 registers (64 channels x
+// 128 columns x 65536 samples, two DMs at N = 8192: 2.80 ms, 2.70 in halves;
+// seven: 7.43 and 7.22).  At R1 = 4 and 8 one round trip wins although it
+// spills 5 (N = 4096, two DMs: 2.44 ms, 2.68 in quarters; R1 = 4 spills none
+// so, R1 = 8 the same 5).  (Held one to a register, in flight behind the last
+// inverse or the forward transform, it spilled 50-110 registers: eight DMs of
+// 64 channels took 9.7 ms instead of 7.7.)
 template <int R1>
 __global__ void __launch_bounds__(512) codedisp_regm_kernel(CdParams p, int nunits)
 {
@@ -572,25 +576,26 @@ __global__ void __launch_bounds__(512) codedisp_regm_kernel(CdParams p, int nuni
     const int t = threadIdx.x;
     load_step2_tables<R1>(t1k, p.tw, t);
     const int ngrp = p.PA / C;
-    auto fetch = [&](int u, uint32_t (&nxt)[32]) {
-        const int cg = u % ngrp, fs = u / ngrp;
-        const int f = fs / p.nseg, s = fs % p.nseg;
-        load_unit<R1>(p, f, cg * C, p.in0 + (long)s * p.hop, t, nxt);
-    };
     // the next unit's raw samples, two per register: held beside X and v
     uint32_t pk[16];
-    auto pack = [&](const uint32_t (&nxt)[32]) {
+    constexpr int H = R1 == 16 ? 2 : 1;  // parts of the unit's columns, loaded one after the other
+    auto fetch = [&](int u) {
+        const int cg = u % ngrp, fs = u / ngrp;
+        const int f = fs / p.nseg, s = fs % p.nseg;
 #pragma unroll
-        for(int i = 0; i < 16; ++i) {
-            pk[i] = nxt[2 * i] | (nxt[2 * i + 1] << 16);
-            asm volatile("" : "+v"(pk[i]));  // packed here, not where it is used
+        for(int h = 0; h < H; ++h) {
+            uint32_t nxt[32 / H];
+            load_unit<R1>(p, f, cg * C + h * (C / H), p.in0 + (long)s * p.hop, t, nxt);
+#pragma unroll
+            for(int i = 0; i < 16 / H; ++i) {
+                uint32_t& x = pk[h * (16 / H) + i];
+                x = nxt[2 * i] | (nxt[2 * i + 1] << 16);
+                asm volatile("" : "+v"(x));  // packed here, not where it is used
+            }
+            if(h + 1 < H) __builtin_amdgcn_sched_barrier(0);
         }
     };
-    if(blockIdx.x < nunits) {
-        uint32_t nxt[32];
-        fetch(blockIdx.x, nxt);
-        pack(nxt);
-    }
+    if(blockIdx.x < nunits) fetch(blockIdx.x);
     __syncthreads();  // twiddle tables
     // step-1 twiddles W_N^(t k1), the same for every unit; from R1 = 16
     // they are rebuilt at each use (held beside X they would spill)
@@ -610,11 +615,7 @@ __global__ void __launch_bounds__(512) codedisp_regm_kernel(CdParams p, int nuni
         const int j0 = (int)(p.y0 + (long)s * p.hop) - p.O / 2;  // ring index of position 0
         for(int d = 0; d < p.ndm; ++d) {
             if(d > 0) __syncthreads();  // the previous DM's step-1' readers of every row
-            if(d == p.ndm - 1 && u + (int)gridDim.x < nunits) {
-                uint32_t nxt[32];
-                fetch(u + gridDim.x, nxt);
-                pack(nxt);
-            }
+            if(d == p.ndm - 1 && u + (int)gridDim.x < nunits) fetch(u + gridDim.x);
             float2 v[32];
             reg_chirp_inverse<R1, HELD>(X, v, lds, tw, t1k, t, p.chirp[d] + (size_t)f * N, wk, hk0);
             store_unit<R1>(p, d, (size_t)f * p.PA + cg * C, j0, t, v);  // v already / N (chirp)

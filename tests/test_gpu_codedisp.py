@@ -379,3 +379,37 @@ def test_codedisp_history_blocks(sw, dev, T, N, O):
         plan.run(buf, [out])
         plan.push_history(buf)
         assert np.array_equal(out.download(), stream[:, g * T:(g + 1) * T]), g
+
+
+@pytest.mark.parametrize("dms,N", [([350.0], 32768), ([100.0, 180.0], 8192), ([20.0, 50.0], 4096)])
+def test_codedisp_workgroups_loop(sw, orc, dev, dms, N):
+    """More than twice as many units as workgroups and a partial last round: what a workgroup
+    carries from one unit to the next, over two gulps, against the oracle; int8 outputs
+    identical with and without the float ring."""
+    from skyweaver_amd import DeviceBuffer as DB
+    F, A, T = 5, 48, 81920
+    nd = len(dms)
+    kw = dict(fft_len=[N] * nd, share_forward=True)
+    plan_f = sw.CoherentDedisperser(F, A, T, F_LOW, CHAN_BW, TSAMP, dms, **kw)
+    plan_i = sw.CoherentDedisperser(F, A, T, F_LOW, CHAN_BW, TSAMP, dms, **kw)
+    _, O = plan_f.info(0)
+    lat = plan_f.latency(0)
+    gulps = [sw.synth_voltages((F, T, 2, A, 2), seed=0x5EED0050 + g, sigma=16.0) for g in range(2)]
+    for g, x in enumerate(gulps):
+        d_g = DB.from_host(x)
+        of = [DB.empty(x.shape, np.int8, fill=0x55) for _ in dms]
+        off = [DB.empty(x.shape, np.float32) for _ in dms]
+        oi = [DB.empty(x.shape, np.int8, fill=0x33) for _ in dms]
+        plan_f.run(d_g, of, off)
+        plan_i.run(d_g, oi)
+        plan_f.push_history(d_g)
+        plan_i.push_history(d_g)
+        for d in range(nd):
+            np.testing.assert_array_equal(oi[d].download(), of[d].download(), err_msg=f"gulp {g} DM {dms[d]}")
+    pick = [0, F - 1]
+    x = np.concatenate([v[pick] for v in gulps], 1)
+    for d in range(nd):
+        chirp = orc.dm_chirp(dms[d], F_LOW, CHAN_BW, F, N)[pick]
+        ei, ef = _oracle_stream(orc, np.zeros((2, O, 2, A, 2), np.int8), x, chirp, N, O)
+        ei, ef = _window(ei, ef, T - lat, T)
+        _check(of[d].download()[pick], off[d].download()[pick], ei, ef, f"gulp 2 DM {dms[d]} N {N}")
