@@ -109,7 +109,7 @@ ib_kernel(const uint8_t* __restrict__ ftpa, float* __restrict__ raw, int8_t* __r
 {
     constexpr int NV = nstokes(S);
     using P = typename std::conditional<W == 4, uint4, uint2>::type;
-    extern __shared__ uint4 rows[];           // float chain: [ob batches][rowq + 1]
+    extern __shared__ uint4 rows[];  // float chain: [ob batches][rowq + 1], then the weights
     const int f    = blockIdx.y;
     const int tid  = threadIdx.x;
     const int nsamps_out = nsamples / tscrunch;
@@ -202,18 +202,30 @@ ib_kernel(const uint8_t* __restrict__ ftpa, float* __restrict__ raw, int8_t* __r
     }
 
     // ---- float chain: the rows t' ts + tt (one per output) staged in LDS with
-    // coalesced 16-byte loads; each output's lane then sums its own row,
-    // antennas ascending, for every beamset
-    const int nout = ob * batches;  // at most 64
-    const int rowq = nant / 4;      // 16-byte pieces per row: 4 nant bytes
+    // coalesced 16-byte loads, beside the weights.  Bound by its serial adds
+    // (each waits for the one before), so the beamsets are dealt to the threads
+    // beside the outputs: thread tid sums output tid mod nout of the beamsets
+    // tid / nout + G k, antennas ascending.  (One thread per output summing
+    // every beamset left most of the workgroup idle and spilled scalar
+    // registers on the weights: 64 channels x 16384 samples x 64 antennas at
+    // tscrunch 16, five beamsets of weights other than 0 and 1, took 1.10 ms,
+    // now 0.24; with 144 antennas 9.4 ms, now 0.45.)
+    const int nout = ob * batches;      // at most 64, a power of two
+    const int G    = kIbThreads / nout;  // threads per output: at least 4
+    constexpr int KS = (SMAX + 3) / 4;  // beamsets per thread
+    const int o = tid % nout, s0 = tid / nout;
+    const int rowq = nant / 4;  // 16-byte pieces per row: 4 nant bytes
     const int ldsq = rowq + 1;
     const int nrows = min(nout, nsamps_out - tp0);
     const uint4* chan16 = reinterpret_cast<const uint4*>(chan);
-    float power[SMAX][NV];
+    float* wl = reinterpret_cast<float*>(rows + nout * ldsq);  // [beamset][antenna]
+    for(int i = tid; i < nbeamsets * nant; i += kIbThreads) wl[i] = antw[i];
+    const bool active = o < nrows && s0 < nbeamsets;
+    float power[KS][NV];
 #pragma unroll
-    for(int s = 0; s < SMAX; ++s)
+    for(int k = 0; k < KS; ++k)
 #pragma unroll
-        for(int k = 0; k < NV; ++k) power[s][k] = 0.0f;
+        for(int v = 0; v < NV; ++v) power[k][v] = 0.0f;
     for(int tt = 0; tt < tscrunch; ++tt) {
         __syncthreads();
         for(int i = tid; i < nrows * rowq; i += kIbThreads) {
@@ -221,45 +233,48 @@ ib_kernel(const uint8_t* __restrict__ ftpa, float* __restrict__ raw, int8_t* __r
             rows[r * ldsq + q] = chan16[((size_t)(tp0 + r) * tscrunch + tt) * rowq + q];
         }
         __syncthreads();
-        if(tid < nrows) {
-            const uint8_t* rb = reinterpret_cast<const uint8_t*>(rows + tid * ldsq);
+        if(active) {
+            const uint8_t* rb = reinterpret_cast<const uint8_t*>(rows + o * ldsq);
             for(int a4 = 0; a4 < nant; a4 += 4) {
                 // 4 antennas of pol 0 and of pol 1 (8 bytes each, 8-byte aligned)
                 const uint2 q0 = *reinterpret_cast<const uint2*>(rb + a4 * 2);
                 const uint2 q1 = *reinterpret_cast<const uint2*>(rb + (nant + a4) * 2);
                 const uint32_t w0[2] = {q0.x, q0.y};
                 const uint32_t w1[2] = {q1.x, q1.y};
+                float st[4][NV];
 #pragma unroll
                 for(int j = 0; j < 4; ++j) {
                     const uint32_t d0 = w0[j >> 1] >> (16 * (j & 1));
                     const uint32_t d1 = w1[j >> 1] >> (16 * (j & 1));
                     const float r0 = (float)(int8_t)(d0), i0 = (float)(int8_t)(d0 >> 8);
                     const float r1 = (float)(int8_t)(d1), i1 = (float)(int8_t)(d1 >> 8);
-                    float st[NV];
                     if constexpr(NV == 1) {
-                        st[0] = stokes<S>(r0, i0, r1, i1);
+                        st[j][0] = stokes<S>(r0, i0, r1, i1);
                     } else {
-                        st[0] = stokes<SW_STOKES_I>(r0, i0, r1, i1);
-                        st[1] = stokes<SW_STOKES_Q>(r0, i0, r1, i1);
-                        st[2] = stokes<SW_STOKES_U>(r0, i0, r1, i1);
-                        st[3] = stokes<SW_STOKES_V>(r0, i0, r1, i1);
-                    }
-#pragma unroll
-                    for(int s = 0; s < SMAX; ++s) {
-                        if(s < nbeamsets) {
-                            const float w = antw[s * nant + a4 + j];
-#pragma unroll
-                            for(int k = 0; k < NV; ++k) power[s][k] += st[k] * w;
-                        }
+                        st[j][0] = stokes<SW_STOKES_I>(r0, i0, r1, i1);
+                        st[j][1] = stokes<SW_STOKES_Q>(r0, i0, r1, i1);
+                        st[j][2] = stokes<SW_STOKES_U>(r0, i0, r1, i1);
+                        st[j][3] = stokes<SW_STOKES_V>(r0, i0, r1, i1);
                     }
                 }
+#pragma unroll
+                for(int k = 0; k < KS; ++k)
+                    if(k == 0 || G * k < nbeamsets) {  // uniform; a thread past the beamsets takes any weights
+                        const float4 w =
+                            *reinterpret_cast<const float4*>(wl + min(s0 + G * k, nbeamsets - 1) * nant + a4);
+#pragma unroll
+                        for(int j = 0; j < 4; ++j)
+#pragma unroll
+                            for(int v = 0; v < NV; ++v)
+                                power[k][v] += st[j][v] * (j == 0 ? w.x : j == 1 ? w.y : j == 2 ? w.z : w.w);
+                    }
             }
         }
     }
-    if(tid >= nrows) return;
+    if(!active) return;
 #pragma unroll
-    for(int s = 0; s < SMAX; ++s)
-        if(s < nbeamsets) store(s, tp0 + tid, power[s]);
+    for(int k = 0; k < KS; ++k)
+        if(s0 + G * k < nbeamsets) store(s0 + G * k, tp0 + o, power[k]);
 }
 
 // Time-major input (the coherent dedisperser's ring): sample t of column
@@ -389,12 +404,25 @@ int launch_ib(const uint8_t* ftpa, float* raw, int8_t* out, const float* scale,
     while(lanes < 64 && lanes < chunks) lanes *= 2;
     auto groups = [&](int ob) { return (long)((nout + ob - 1) / ob) * d.nchans; };
     while(lanes < 64 && groups(kIbThreads / lanes) < 1024 && (long)d.tscrunch * chunks >= 8L * lanes) lanes *= 2;
-    const int ob = kIbThreads / lanes;
     // 64 outputs per workgroup where enough workgroups are left: the float
-    // chain then fills its wave
-    const int batches = groups(64) >= 2048 ? 64 / ob : 1;
+    // chain then fills its waves
+    int batches = groups(64) >= 2048 ? 64 * lanes / kIbThreads : 1;
+    // LDS of the float chain for n outputs per workgroup: rows and weights
+    auto chain_lds = [&](int n) {
+        return (size_t)n * (d.nantennas / 4 + 1) * 16 + (size_t)d.nbeamsets * d.nantennas * 4;
+    };
+    if(d.nantennas > 2 * kMaskWords) {
+        // the float chain only: 64 outputs per workgroup, fewer (a thread then
+        // takes fewer beamsets) while there is not a workgroup per CU or two
+        // workgroups do not fit a CU's LDS
+        int n = 64;
+        while(n > 8 && (groups(n) < 256 || chain_lds(n) > (size_t)72 << 10)) n /= 2;
+        lanes   = kIbThreads / n;
+        batches = 1;
+    }
+    const int ob = kIbThreads / lanes;
     const dim3 grid((unsigned)((nout + ob * batches - 1) / (ob * batches)), d.nchans);
-    const size_t lds = (size_t)ob * batches * (d.nantennas / 4 + 1) * 16;
+    const size_t lds = chain_lds(ob * batches);
 #define SW_IB_LAUNCH(SM)                                                                                    \
     if(w4)                                                                                                  \
         hipLaunchKernelGGL((ib_kernel<S, SM, 4>), grid, dim3(kIbThreads), lds, st, ftpa, raw, out, scale,   \

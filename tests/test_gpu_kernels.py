@@ -224,6 +224,52 @@ def test_ib_exact_path_splits(sw, orc, dev, stokes, F, T, A, ts, S):
     np.testing.assert_array_equal(out, eout)
 
 
+@pytest.mark.parametrize("stokes", ["I", "V", "IQUV"])
+@pytest.mark.parametrize("F,T,A,ts,S", [(2, 333, 4, 1, 16),       # one 8-byte piece per row
+                                        (64, 2112, 16, 1, 5),     # 64 outputs per workgroup, a partial last one
+                                        (2, 2048, 64, 64, 9),     # 4 outputs per workgroup
+                                        (1, 1200, 128, 8, 13),
+                                        (3, 690, 132, 5, 3),      # past the integer path's antennas
+                                        (40, 1288, 144, 1, 8),
+                                        (2, 1036, 256, 4, 16),
+                                        (1, 68, 512, 4, 7)])
+def test_ib_float_chain_splits(sw, orc, dev, stokes, F, T, A, ts, S):
+    """The ways outputs and beamsets share a workgroup's threads in the float chain: weights other
+    than 0 and 1, one of them huge, still bit for bit."""
+    v = _rand_c8((F, T, 2, A), 23 + A + S, sigma=40.0)
+    w = (_rng(S + A).random((S, A)) * 2.3 - 0.5).astype(np.float32)
+    w[-1, 0] = 3e7
+    scale, offset = _ib_scales(F, S, A, ts)
+    raw, out = _run_ib(sw, dev, v, w, scale, offset, ts, stokes)
+    if F > 8:  # the oracle on a few channels
+        pick = [0, F // 2, F - 1]
+        v, raw, out = v[pick], raw[:, :, pick], out[:, :, pick]
+        scale, offset = (x.reshape(S, F)[:, pick].reshape(-1).copy() for x in (scale, offset))
+    eraw, eout = orc.ib_beamform(np.ascontiguousarray(v), ts, scale, offset, w, S, stokes)
+    np.testing.assert_array_equal(raw, eraw)
+    np.testing.assert_array_equal(out, eout)
+
+
+@pytest.mark.parametrize("stokes,S", [("I", 1), ("I", 6), ("IQUV", 2)])
+def test_ib_exact_path_overflow_in_some_batches(sw, orc, dev, stokes, S):
+    """64 outputs per workgroup in several batches, some of which pass 2^24 in some workgroups."""
+    F, T, A, ts = 64, 8192, 64, 4
+    v = _rand_c8((F, T, 2, A), 31, sigma=8.0)
+    v[0, 70 * ts:75 * ts] = -128    # one batch of the second workgroup
+    v[31, 40 * ts] = 127            # not enough
+    v[63, (T // ts - 1) * ts:] = 127
+    w = np.ones((S, A), np.float32)
+    w[1:] = _rng(3).random((S - 1, A)) > 0.2
+    scale, offset = _ib_scales(F, S, A, ts)
+    raw, out = _run_ib(sw, dev, v, w, scale, offset, ts, stokes)
+    pick = [0, 31, 63]
+    scale, offset = (x.reshape(S, F)[:, pick].reshape(-1).copy() for x in (scale, offset))
+    eraw, eout = orc.ib_beamform(np.ascontiguousarray(v[pick]), ts, scale, offset, w, S, stokes)
+    assert (eraw >= 2 ** 24).any() and (eraw < 2 ** 24).any()
+    np.testing.assert_array_equal(raw[:, :, pick], eraw)
+    np.testing.assert_array_equal(out[:, :, pick], eout)
+
+
 # --------------------------------------------------------- coherent beamformer
 def _cb_scales(F, S, A, ts, level=32.0):
     # CoherentBeamformerTester.cu:224-242
