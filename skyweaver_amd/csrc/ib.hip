@@ -46,16 +46,17 @@ struct IbSums {
     int p0 = 0, p1 = 0, u = 0, v0 = 0, v1 = 0;
     __device__ __forceinline__ void add(uint32_t x0, uint32_t x1, uint32_t m)
     {
-        const uint32_t a0 = x0 & m;
-        p0 = __builtin_amdgcn_sdot4((int)a0, (int)x0, p0, true);
-        p1 = __builtin_amdgcn_sdot4((int)(x1 & m), (int)x1, p1, true);
-        if constexpr(kU) u = __builtin_amdgcn_sdot4((int)a0, (int)x1, u, false);
+        const int a1 = (int)(x1 & m);
+        p0 = __builtin_amdgcn_sdot4((int)(x0 & m), (int)x0, p0, true);
+        p1 = __builtin_amdgcn_sdot4(a1, (int)x1, p1, true);
+        if constexpr(kU) u = __builtin_amdgcn_sdot4((int)x0, a1, u, false);
         if constexpr(kV) {
-            // [i, 0] and [0, r] of each antenna against x1's [r, i]
-            const uint32_t im = __builtin_amdgcn_perm(a0, a0, 0x0C030C01u);
-            const uint32_t re = __builtin_amdgcn_perm(a0, a0, 0x020C000Cu);
-            v0 = __builtin_amdgcn_sdot4((int)im, (int)x1, v0, false);
-            v1 = __builtin_amdgcn_sdot4((int)re, (int)x1, v1, false);
+            // [i, 0] and [0, r] of each antenna (the same for every mask)
+            // against x1's [r, i]
+            const uint32_t im = __builtin_amdgcn_perm(x0, x0, 0x0C030C01u);
+            const uint32_t re = __builtin_amdgcn_perm(x0, x0, 0x020C000Cu);
+            v0 = __builtin_amdgcn_sdot4((int)im, a1, v0, false);
+            v1 = __builtin_amdgcn_sdot4((int)re, a1, v1, false);
         }
     }
     // Stokes I, at most 2^24 (64 of these sum without overflow)
@@ -84,12 +85,56 @@ __device__ __forceinline__ void ib_store(float* raw, int8_t* out, size_t o, cons
     }
 }
 
-// the sum over `lanes` (a power of two) neighbouring lanes
-__device__ __forceinline__ int lanes_sum(int v, int lanes)
+// lane l's partner in a group of eight: l ^ 7, l ^ 2 or l ^ 1
+template <int M>
+__device__ __forceinline__ int lane_xor(int v)
 {
-    for(int m = 1; m < lanes; m <<= 1) v += __shfl_xor(v, m, 64);
-    return v;
+    static_assert(M == 7 || M == 2 || M == 1, "row_half_mirror, quad_perm");
+    return __builtin_amdgcn_mov_dpp(v, M == 7 ? 0x141 : M == 2 ? 0x4E : 0xB1, 0xF, 0xF, true);
 }
+
+// One step of LanesSum: with two or more values left a lane gives its
+// partner half of them and keeps the half that its bit B selects, else both
+// add the one.
+template <int M, int B, int N>
+__device__ __forceinline__ void lanes_step(int* v, int l)
+{
+    if constexpr(N == 1) {
+        v[0] += lane_xor<M>(v[0]);
+    } else {
+#pragma unroll
+        for(int i = 0; i < N / 2; ++i) {
+            const int keep = l & B ? v[N / 2 + i] : v[i], give = l & B ? v[i] : v[N / 2 + i];
+            v[i] = keep + lane_xor<M>(give);
+        }
+    }
+}
+
+// The sums of N values (a power of two) over groups of `lanes` (8 ... 64)
+// lanes, dealt out: lane l ends with the sums first(l) ... first(l) + N' - 1,
+// N' = max(N / 8, 1), in v.  (A tree per value over all lanes, one lane
+// storing every value, was a latency of its own each: 64 channels x 65536
+// samples x 16 antennas at tscrunch 4, five beamsets, took 226 us, now 141;
+// 16 of full Stokes 2.38 ms, now 0.60.)
+template <int N>
+struct LanesSum {
+    static constexpr int kLeft = N < 8 ? 1 : N / 8;
+    __device__ static __forceinline__ int first(int l) { return (l & 7) * N / 8; }
+    // the lanes that hold sums nobody before them holds
+    __device__ static __forceinline__ bool owner(int l) { return l < 8 && (l * N) % 8 < (N < 8 ? N : 8); }
+    __device__ static __forceinline__ void run(int* v, int l, int lanes)
+    {
+        lanes_step<7, 4, N>(v, l);
+        lanes_step<2, 2, (N < 2 ? 1 : N / 2)>(v, l);
+        lanes_step<1, 1, (N < 4 ? 1 : N / 4)>(v, l);
+#pragma unroll
+        for(int i = 0; i < kLeft; ++i) {
+            if(lanes > 8) v[i] += __builtin_amdgcn_mov_dpp(v[i], 0x128, 0xF, 0xF, true);  // row_ror:8
+            if(lanes > 16) v[i] += __builtin_amdgcn_ds_swizzle(v[i], 0x401F);             // lane ^ 16
+            if(lanes > 32) v[i] += __shfl_xor(v[i], 32, 64);
+        }
+    }
+};
 
 // A workgroup owns `batches` runs of ob = 256 / lanes consecutive outputs of
 // one channel.  HBM-bound: `lanes` neighbouring lanes share an output, each
@@ -178,22 +223,31 @@ ib_kernel(const uint8_t* __restrict__ ftpa, float* __restrict__ raw, int8_t* __r
                     }
                 }
             }
+            // the lanes' sums meet, and a lane finishes its share of the beamsets
+            using L = LanesSum<SMAX>;
+            int v[NV + (S == SW_STOKES_I || NV == 4 ? 0 : 1)][SMAX];  // I, then the others wanted
 #pragma unroll
             for(int s = 0; s < SMAX; ++s) {
-                if(s < nbeamsets) {  // uniform
+                v[0][s] = sum[s].total();
+                if constexpr(S == SW_STOKES_Q || NV == 4) v[1][s] = sum[s].q();
+                if constexpr(S == SW_STOKES_U) v[1][s] = sum[s].uu();
+                if constexpr(S == SW_STOKES_V) v[1][s] = sum[s].vv();
+                if constexpr(NV == 4) {
+                    v[2][s] = sum[s].uu();
+                    v[3][s] = sum[s].vv();
+                }
+            }
+            constexpr int NVI = sizeof(v) / sizeof(v[0]);
+#pragma unroll
+            for(int k = 0; k < NVI; ++k) L::run(v[k], l, lanes);
+#pragma unroll
+            for(int i = 0; i < L::kLeft; ++i) {
+                big = big || v[0][i] >= kExact;
+                if(L::owner(l) && L::first(l) + i < nbeamsets && tp < nsamps_out) {
                     float power[NV];
-                    const int tot = lanes_sum(sum[s].total(), lanes);
-                    if constexpr(S == SW_STOKES_I || NV == 4) power[0] = (float)tot;
-                    if constexpr(S == SW_STOKES_Q) power[0] = (float)lanes_sum(sum[s].q(), lanes);
-                    if constexpr(S == SW_STOKES_U) power[0] = (float)lanes_sum(sum[s].uu(), lanes);
-                    if constexpr(S == SW_STOKES_V) power[0] = (float)lanes_sum(sum[s].vv(), lanes);
-                    if constexpr(NV == 4) {
-                        power[1] = (float)lanes_sum(sum[s].q(), lanes);
-                        power[2] = (float)lanes_sum(sum[s].uu(), lanes);
-                        power[3] = (float)lanes_sum(sum[s].vv(), lanes);
-                    }
-                    big = big || tot >= kExact;
-                    if(l == 0 && tp < nsamps_out) store(s, tp, power);
+#pragma unroll
+                    for(int k = 0; k < NV; ++k) power[k] = (float)v[NVI - NV + k][i];
+                    store(L::first(l) + i, tp, power);
                 }
             }
         }
@@ -438,6 +492,8 @@ int launch_ib(const uint8_t* ftpa, float* raw, int8_t* out, const float* scale,
         SW_IB_LAUNCH(2)
     } else if(d.nbeamsets <= 4) {
         SW_IB_LAUNCH(4)
+    } else if(d.nbeamsets <= 8) {
+        SW_IB_LAUNCH(8)
     } else {
         SW_IB_LAUNCH(16)
     }

@@ -224,6 +224,25 @@ def test_ib_exact_path_splits(sw, orc, dev, stokes, F, T, A, ts, S):
     np.testing.assert_array_equal(out, eout)
 
 
+@pytest.mark.parametrize("stokes", ["I", "Q", "U", "IQUV"])
+@pytest.mark.parametrize("F,T,A,ts,S", [(64, 8192, 16, 4, 16),   # 8 lanes per output
+                                        (64, 8192, 20, 4, 6),
+                                        (2, 4096, 64, 8, 8),     # 16 and 32 lanes
+                                        (3, 2048, 32, 16, 9),
+                                        (1, 1024, 128, 64, 16)])  # 64 lanes
+def test_ib_exact_path_many_beamsets(sw, orc, dev, stokes, F, T, A, ts, S):
+    """The beamsets dealt to an output's lanes, each antenna in about half of them."""
+    v = _rand_c8((F, T, 2, A), 41 + S, sigma=20.0)
+    w = (_rng(A).random((S, A)) > 0.5).astype(np.float32)
+    scale, offset = _ib_scales(F, S, A, ts)
+    raw, out = _run_ib(sw, dev, v, w, scale, offset, ts, stokes)
+    pick = sorted({0, F // 2, F - 1})
+    scale, offset = (x.reshape(S, F)[:, pick].reshape(-1).copy() for x in (scale, offset))
+    eraw, eout = orc.ib_beamform(np.ascontiguousarray(v[pick]), ts, scale, offset, w, S, stokes)
+    np.testing.assert_array_equal(raw[:, :, pick], eraw)
+    np.testing.assert_array_equal(out[:, :, pick], eout)
+
+
 @pytest.mark.parametrize("stokes", ["I", "V", "IQUV"])
 @pytest.mark.parametrize("F,T,A,ts,S", [(2, 333, 4, 1, 16),       # one 8-byte piece per row
                                         (64, 2112, 16, 1, 5),     # 64 outputs per workgroup, a partial last one
