@@ -25,12 +25,14 @@
 // of 2^24 or more recomputes its outputs with the float chain.
 #include "sw_common.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace sw {
 namespace {
 
-constexpr int kIbThreads = 256;
+constexpr int kIbThreads = 256;  // 2^8
+constexpr int kSmall = 32;      // antennas x tscrunch of ib_small_kernel's outputs
 constexpr int kMaskWords = 64;  // 0/1 weight masks for up to 128 antennas
 
 // 2^24: integers below it are exact in FP32
@@ -85,6 +87,32 @@ __device__ __forceinline__ void ib_store(float* raw, int8_t* out, size_t o, cons
     }
 }
 
+// Stokes parameters of antennas a4 ... a4 + 3 of the staged row rb
+template <int S>
+__device__ __forceinline__ void stokes4(const uint8_t* rb, int nant, int a4, float (&st)[4][nstokes(S)])
+{
+    // 4 antennas of pol 0 and of pol 1 (8 bytes each, 8-byte aligned)
+    const uint2 q0 = *reinterpret_cast<const uint2*>(rb + a4 * 2);
+    const uint2 q1 = *reinterpret_cast<const uint2*>(rb + (nant + a4) * 2);
+    const uint32_t w0[2] = {q0.x, q0.y};
+    const uint32_t w1[2] = {q1.x, q1.y};
+#pragma unroll
+    for(int j = 0; j < 4; ++j) {
+        const uint32_t d0 = w0[j >> 1] >> (16 * (j & 1));
+        const uint32_t d1 = w1[j >> 1] >> (16 * (j & 1));
+        const float r0 = (float)(int8_t)(d0), i0 = (float)(int8_t)(d0 >> 8);
+        const float r1 = (float)(int8_t)(d1), i1 = (float)(int8_t)(d1 >> 8);
+        if constexpr(nstokes(S) == 1) {
+            st[j][0] = stokes<S>(r0, i0, r1, i1);
+        } else {
+            st[j][0] = stokes<SW_STOKES_I>(r0, i0, r1, i1);
+            st[j][1] = stokes<SW_STOKES_Q>(r0, i0, r1, i1);
+            st[j][2] = stokes<SW_STOKES_U>(r0, i0, r1, i1);
+            st[j][3] = stokes<SW_STOKES_V>(r0, i0, r1, i1);
+        }
+    }
+}
+
 // lane l's partner in a group of eight: l ^ 7, l ^ 2 or l ^ 1
 template <int M>
 __device__ __forceinline__ int lane_xor(int v)
@@ -136,12 +164,12 @@ struct LanesSum {
     }
 };
 
-// A workgroup owns `batches` runs of ob = 256 / lanes consecutive outputs of
-// one channel.  HBM-bound: `lanes` neighbouring lanes share an output, each
-// reading 4 W bytes (2 W antennas) of both polarisations of every (lanes /
-// chunks)-th row of its scrunch window, up to four rows' loads in flight, so
-// that a wave reads whole rows and nothing goes through LDS; the lanes' sums
-// meet in a shuffle tree.  (Staged through LDS by one wave per 64 outputs,
+// A workgroup owns batches = 2^bsh runs of ob = 256 / lanes consecutive outputs
+// of one channel, lanes = 2^lsh.  HBM-bound: `lanes` neighbouring lanes share
+// an output, each reading 4 W bytes (2 W antennas) of both polarisations of
+// every (lanes / chunks)-th row of its scrunch window, up to four rows' loads
+// in flight, so that a wave reads whole rows and nothing goes through LDS; the
+// lanes' sums meet in LanesSum.  (Staged through LDS by one wave per 64 outputs,
 // each lane then summing a whole window, the loads of a row were waited for
 // before the sums of it: 64 channels x 16384 samples x 64 antennas, two
 // beamsets, took 150 us, IQUV of 16 channels x 32768 samples 206 us.)
@@ -149,20 +177,19 @@ template <int S, int SMAX, int W>
 __global__ void __launch_bounds__(kIbThreads)
 ib_kernel(const uint8_t* __restrict__ ftpa, float* __restrict__ raw, int8_t* __restrict__ out,
           const float* __restrict__ scale, const float* __restrict__ offset,
-          const float* __restrict__ antw, int nchans, int nsamples, int nant, int tscrunch,
-          int nbeamsets, int lanes, int batches)
+          const float* __restrict__ antw, int nchans, int nsamps_out, int nant, int tscrunch,
+          int nbeamsets, int lsh, int bsh, int csh)
 {
     constexpr int NV = nstokes(S);
     using P = typename std::conditional<W == 4, uint4, uint2>::type;
     extern __shared__ uint4 rows[];  // float chain: [ob batches][rowq + 1], then the weights
     const int f    = blockIdx.y;
     const int tid  = threadIdx.x;
-    const int nsamps_out = nsamples / tscrunch;
-    const int ob   = kIbThreads / lanes;
+    const int lanes = 1 << lsh, batches = 1 << bsh, ob = kIbThreads >> lsh;
     const int tp0  = blockIdx.x * ob * batches;
-    const uint8_t* chan = ftpa + (size_t)f * nsamples * 4 * nant;
+    const uint8_t* chan = ftpa + (size_t)f * nsamps_out * tscrunch * 4 * nant;
 
-    auto store = [&](int s, int tp, const float* power) {
+    auto store = [&](int f, int s, int tp, const float* power) {
         ib_store<S>(raw, out, ((size_t)s * nsamps_out + tp) * nchans + f, power, offset[s * nchans + f],
                     scale[s * nchans + f]);
     };
@@ -183,10 +210,10 @@ ib_kernel(const uint8_t* __restrict__ ftpa, float* __restrict__ raw, int8_t* __r
     if(exact) {
         const int chunks = nant / (2 * W);        // loads per polarisation of a row
         const int krow   = max(1, lanes / chunks);  // rows an output's lanes read together
-        const int l = tid % lanes;
+        const int l = tid & (lanes - 1);
         bool big = false;
         for(int b = 0; b < batches; ++b) {
-            const int tp = tp0 + b * ob + tid / lanes;
+            const int tp = tp0 + b * ob + (tid >> lsh);
             IbSums<S> sum[SMAX];
             if(l < krow * chunks && tp < nsamps_out) {
                 for(int q = l % chunks; q < chunks; q += lanes) {  // once unless lanes < chunks
@@ -247,73 +274,68 @@ ib_kernel(const uint8_t* __restrict__ ftpa, float* __restrict__ raw, int8_t* __r
                     float power[NV];
 #pragma unroll
                     for(int k = 0; k < NV; ++k) power[k] = (float)v[NVI - NV + k][i];
-                    store(L::first(l) + i, tp, power);
+                    store(f, L::first(l) + i, tp, power);
                 }
             }
         }
-        exact = !__syncthreads_or(big);
-        if(exact) return;
+        if(!__syncthreads_or(big)) return;
     }
 
     // ---- float chain: the rows t' ts + tt (one per output) staged in LDS with
     // coalesced 16-byte loads, beside the weights.  Bound by its serial adds
-    // (each waits for the one before), so the beamsets are dealt to the threads
-    // beside the outputs: thread tid sums output tid mod nout of the beamsets
-    // tid / nout + G k, antennas ascending.  (One thread per output summing
-    // every beamset left most of the workgroup idle and spilled scalar
-    // registers on the weights: 64 channels x 16384 samples x 64 antennas at
-    // tscrunch 16, five beamsets of weights other than 0 and 1, took 1.10 ms,
-    // now 0.24; with 144 antennas 9.4 ms, now 0.45.)
-    const int nout = ob * batches;      // at most 64, a power of two
-    const int G    = kIbThreads / nout;  // threads per output: at least 4
-    constexpr int KS = (SMAX + 3) / 4;  // beamsets per thread
-    const int o = tid % nout, s0 = tid / nout;
+    // (each waits for the one before), so it wants many outputs in flight and
+    // no thread idle: the beamsets are dealt to the threads beside the
+    // outputs, thread tid summing output tid mod run of the beamsets
+    // tid / run + G k, antennas ascending.  Weights other than 0 and 1 are the
+    // same for every workgroup: then the first of them take 2^csh outputs
+    // each, counted over all channels, and the others have none.
+    // (One thread per output summing every beamset, 4 to 64 outputs a
+    // workgroup, left most of it idle and spilled scalar registers on the
+    // weights: 64 channels x 16384 samples x 64 antennas at tscrunch 16, five
+    // beamsets of weights other than 0 and 1, took 1.10 ms, now 0.15; with 144
+    // antennas 9.4 ms, now 0.49; 65536 samples x 16 antennas at tscrunch 4,
+    // full Stokes, five beamsets, with at most 64 outputs a workgroup 327 us,
+    // now 204.)
+    const int rsh = exact ? 8 - lsh + bsh : csh, run = 1 << rsh;
+    int fc = f, t0 = tp0;
+    if(!exact) {
+        const unsigned per = ((unsigned)nsamps_out + run - 1) >> csh;
+        const unsigned w = blockIdx.y * gridDim.x + blockIdx.x;
+        if(w >= per * nchans) return;  // whole workgroup, before any barrier
+        fc = w / per;
+        t0 = (int)(w % per) << csh;
+    }
+    const int nrows = min(run, nsamps_out - t0);
+    const int G = kIbThreads >> rsh;  // threads per output
+    const int o = tid & (run - 1), s0 = tid >> rsh;
+    const bool active = o < nrows && s0 < nbeamsets;
+    // beamsets of the wave's first thread: no thread of it has more
+    const int kn = __builtin_amdgcn_readfirstlane((nbeamsets - s0 + G - 1) >> (8 - rsh));
     const int rowq = nant / 4;  // 16-byte pieces per row: 4 nant bytes
     const int ldsq = rowq + 1;
-    const int nrows = min(nout, nsamps_out - tp0);
-    const uint4* chan16 = reinterpret_cast<const uint4*>(chan);
-    float* wl = reinterpret_cast<float*>(rows + nout * ldsq);  // [beamset][antenna]
+    const uint4* chan16 = reinterpret_cast<const uint4*>(ftpa + (size_t)fc * nsamps_out * tscrunch * 4 * nant);
+    float* wl = reinterpret_cast<float*>(rows + run * ldsq);  // [beamset][antenna]
     for(int i = tid; i < nbeamsets * nant; i += kIbThreads) wl[i] = antw[i];
-    const bool active = o < nrows && s0 < nbeamsets;
-    float power[KS][NV];
+    float power[SMAX][NV];
 #pragma unroll
-    for(int k = 0; k < KS; ++k)
+    for(int k = 0; k < SMAX; ++k)
 #pragma unroll
         for(int v = 0; v < NV; ++v) power[k][v] = 0.0f;
     for(int tt = 0; tt < tscrunch; ++tt) {
         __syncthreads();
         for(int i = tid; i < nrows * rowq; i += kIbThreads) {
             const int r = i / rowq, q = i % rowq;
-            rows[r * ldsq + q] = chan16[((size_t)(tp0 + r) * tscrunch + tt) * rowq + q];
+            rows[r * ldsq + q] = chan16[((size_t)(t0 + r) * tscrunch + tt) * rowq + q];
         }
         __syncthreads();
         if(active) {
             const uint8_t* rb = reinterpret_cast<const uint8_t*>(rows + o * ldsq);
             for(int a4 = 0; a4 < nant; a4 += 4) {
-                // 4 antennas of pol 0 and of pol 1 (8 bytes each, 8-byte aligned)
-                const uint2 q0 = *reinterpret_cast<const uint2*>(rb + a4 * 2);
-                const uint2 q1 = *reinterpret_cast<const uint2*>(rb + (nant + a4) * 2);
-                const uint32_t w0[2] = {q0.x, q0.y};
-                const uint32_t w1[2] = {q1.x, q1.y};
                 float st[4][NV];
+                stokes4<S>(rb, nant, a4, st);
 #pragma unroll
-                for(int j = 0; j < 4; ++j) {
-                    const uint32_t d0 = w0[j >> 1] >> (16 * (j & 1));
-                    const uint32_t d1 = w1[j >> 1] >> (16 * (j & 1));
-                    const float r0 = (float)(int8_t)(d0), i0 = (float)(int8_t)(d0 >> 8);
-                    const float r1 = (float)(int8_t)(d1), i1 = (float)(int8_t)(d1 >> 8);
-                    if constexpr(NV == 1) {
-                        st[j][0] = stokes<S>(r0, i0, r1, i1);
-                    } else {
-                        st[j][0] = stokes<SW_STOKES_I>(r0, i0, r1, i1);
-                        st[j][1] = stokes<SW_STOKES_Q>(r0, i0, r1, i1);
-                        st[j][2] = stokes<SW_STOKES_U>(r0, i0, r1, i1);
-                        st[j][3] = stokes<SW_STOKES_V>(r0, i0, r1, i1);
-                    }
-                }
-#pragma unroll
-                for(int k = 0; k < KS; ++k)
-                    if(k == 0 || G * k < nbeamsets) {  // uniform; a thread past the beamsets takes any weights
+                for(int k = 0; k < SMAX; ++k)
+                    if(k == 0 || k < kn) {  // uniform; a thread past the beamsets takes any weights
                         const float4 w =
                             *reinterpret_cast<const float4*>(wl + min(s0 + G * k, nbeamsets - 1) * nant + a4);
 #pragma unroll
@@ -327,8 +349,97 @@ ib_kernel(const uint8_t* __restrict__ ftpa, float* __restrict__ raw, int8_t* __r
     }
     if(!active) return;
 #pragma unroll
-    for(int k = 0; k < KS; ++k)
-        if(s0 + G * k < nbeamsets) store(s0 + G * k, tp0 + o, power[k]);
+    for(int k = 0; k < SMAX; ++k)
+        if(s0 + G * k < nbeamsets) store(fc, s0 + G * k, t0 + o, power[k]);
+}
+
+// Outputs of few rows and antennas (see launch_ib): one wave per 64 outputs of
+// one channel, a lane per output, the rows staged as for the float chain.  Sums
+// are few and dealing them to neighbouring lanes costs more than it saves: 64
+// channels x 65536 samples x 16 antennas at tscrunch 1 take 91 us so and 183
+// in ib_kernel.  Stokes I with weights of 0 and 1 in integers (the
+// totals are at most 2^21), the rest as the float chain.
+template <int S, int SMAX>
+__global__ void __launch_bounds__(64)
+ib_small_kernel(const uint8_t* __restrict__ ftpa, float* __restrict__ raw, int8_t* __restrict__ out,
+                const float* __restrict__ scale, const float* __restrict__ offset,
+                const float* __restrict__ antw, int nchans, int nsamples, int nant, int tscrunch,
+                int nbeamsets)
+{
+    constexpr int NV = nstokes(S);
+    extern __shared__ uint4 rows[];  // [64][rowq + 1]
+    __shared__ uint32_t wmask[SMAX][kSmall / 2];  // per word: 0xFFFF per antenna of weight 1
+    const int f    = blockIdx.y;
+    const int lane = threadIdx.x;
+    const int nsamps_out = nsamples / tscrunch;
+    const int tp0  = blockIdx.x * 64;
+    const int rowq = nant / 4;  // 16-byte pieces per row: 4 nant bytes
+    const int ldsq = rowq + 1;
+    const int nrows = min(64, nsamps_out - tp0);
+    const uint4* chan = reinterpret_cast<const uint4*>(ftpa + (size_t)f * nsamples * 4 * nant);
+    bool exact = false;
+    if constexpr(S == SW_STOKES_I) {
+        bool binary = true;
+        for(int i = lane; i < nbeamsets * nant / 2; i += 64) {
+            const int sb = i / (nant / 2), j = i % (nant / 2);
+            const float w0 = antw[sb * nant + 2 * j], w1 = antw[sb * nant + 2 * j + 1];
+            binary = binary && (w0 == 0.0f || w0 == 1.0f) && (w1 == 0.0f || w1 == 1.0f);
+            wmask[sb][j] = (w0 != 0.0f ? 0x0000FFFFu : 0u) | (w1 != 0.0f ? 0xFFFF0000u : 0u);
+        }
+        exact = __syncthreads_and(binary);
+    }
+    float power[SMAX][NV];
+    int isum[SMAX];
+#pragma unroll
+    for(int s = 0; s < SMAX; ++s) {
+        isum[s] = 0;
+#pragma unroll
+        for(int k = 0; k < NV; ++k) power[s][k] = 0.0f;
+    }
+    for(int tt = 0; tt < tscrunch; ++tt) {
+        __syncthreads();
+        for(int i = lane; i < nrows * rowq; i += 64) {
+            const int r = i / rowq, q = i % rowq;
+            rows[r * ldsq + q] = chan[((size_t)(tp0 + r) * tscrunch + tt) * rowq + q];
+        }
+        __syncthreads();
+        if(lane >= nrows) continue;
+        if(exact) {
+            const int hw = nant / 2;  // words per polarisation
+            const uint32_t* rw = reinterpret_cast<const uint32_t*>(rows + lane * ldsq);
+#pragma unroll
+            for(int s = 0; s < SMAX; ++s)
+                if(s < nbeamsets)
+                    for(int j = 0; j < hw; ++j) {
+                        const int m = (int)wmask[s][j];
+                        const int x0 = (int)rw[j], x1 = (int)rw[hw + j];
+                        isum[s] = __builtin_amdgcn_sdot4(x0 & m, x0, isum[s], false);
+                        isum[s] = __builtin_amdgcn_sdot4(x1 & m, x1, isum[s], false);
+                    }
+        } else {
+            for(int a4 = 0; a4 < nant; a4 += 4) {
+                float st[4][NV];
+                stokes4<S>(reinterpret_cast<const uint8_t*>(rows + lane * ldsq), nant, a4, st);
+#pragma unroll
+                for(int j = 0; j < 4; ++j)
+#pragma unroll
+                    for(int s = 0; s < SMAX; ++s)
+                        if(s < nbeamsets) {
+                            const float w = antw[s * nant + a4 + j];
+#pragma unroll
+                            for(int k = 0; k < NV; ++k) power[s][k] += st[j][k] * w;
+                        }
+            }
+        }
+    }
+    if(lane >= nrows) return;
+#pragma unroll
+    for(int s = 0; s < SMAX; ++s)
+        if(s < nbeamsets) {
+            if(exact) power[s][0] = (float)isum[s];
+            ib_store<S>(raw, out, ((size_t)s * nsamps_out + tp0 + lane) * nchans + f, power[s],
+                        offset[s * nchans + f], scale[s * nchans + f]);
+        }
 }
 
 // Time-major input (the coherent dedisperser's ring): sample t of column
@@ -448,6 +559,34 @@ int launch_ib(const uint8_t* ftpa, float* raw, int8_t* out, const float* scale,
               const float* offset, const float* antw, const sw_bf_dims& d, hipStream_t st)
 {
     const int nout = d.nsamples / d.tscrunch;
+    // where ib_small_kernel is the faster, one beamset over all 64 channels:
+    // 16384 samples x 4 antennas at tscrunch 1 14.1 us and 37.8, 16 antennas
+    // 18.7 and 41.8; 8192 samples x 16 antennas at tscrunch 2 8.5 and 13.6, x
+    // 32 at 1 17.1 and 23.3.  Not with more rows a window (65536 samples x 8
+    // antennas at tscrunch 4: 77 and 43) or few outputs, for which ib_kernel
+    // finds more lanes (8 channels x 4096 samples x 16 antennas at tscrunch 2,
+    // sixteen beamsets: 11.5 and 7.6)
+    const int window = d.nantennas * d.tscrunch;
+    const long waves = (long)((nout + 63) / 64) * d.nchans;
+    if((window <= kSmall / 2 && waves >= 512) || (window <= kSmall && d.tscrunch <= 2 && waves >= 2048)) {
+        const dim3 grid((unsigned)((nout + 63) / 64), d.nchans);
+        const size_t lds = (size_t)64 * (d.nantennas / 4 + 1) * 16;
+#define SW_IB_LAUNCH(SM)                                                                                           \
+    hipLaunchKernelGGL((ib_small_kernel<S, SM>), grid, dim3(64), lds, st, ftpa, raw, out, scale, offset, antw,     \
+                       d.nchans, d.nsamples, d.nantennas, d.tscrunch, d.nbeamsets);
+        if(d.nbeamsets <= 1) {
+            SW_IB_LAUNCH(1)
+        } else if(d.nbeamsets <= 4) {
+            SW_IB_LAUNCH(4)
+        } else if(d.nbeamsets <= 8) {
+            SW_IB_LAUNCH(8)
+        } else {
+            SW_IB_LAUNCH(16)
+        }
+#undef SW_IB_LAUNCH
+        SW_LAUNCH_CHECK();
+        return SW_OK;
+    }
     const bool w4 = d.nantennas % 8 == 0;  // 16-byte loads, else 8-byte
     const int chunks = d.nantennas / (w4 ? 8 : 4);
     // 8 lanes per output (a row of 64 antennas' polarisation at 16 bytes a
@@ -458,34 +597,35 @@ int launch_ib(const uint8_t* ftpa, float* raw, int8_t* out, const float* scale,
     while(lanes < 64 && lanes < chunks) lanes *= 2;
     auto groups = [&](int ob) { return (long)((nout + ob - 1) / ob) * d.nchans; };
     while(lanes < 64 && groups(kIbThreads / lanes) < 1024 && (long)d.tscrunch * chunks >= 8L * lanes) lanes *= 2;
-    // 64 outputs per workgroup where enough workgroups are left: the float
-    // chain then fills its waves
+    // 64 outputs per workgroup where enough workgroups are left
     int batches = groups(64) >= 2048 ? 64 * lanes / kIbThreads : 1;
-    // LDS of the float chain for n outputs per workgroup: rows and weights
+    // LDS of the float chain for n outputs at a time: rows and weights
     auto chain_lds = [&](int n) {
         return (size_t)n * (d.nantennas / 4 + 1) * 16 + (size_t)d.nbeamsets * d.nantennas * 4;
     };
-    if(d.nantennas > 2 * kMaskWords) {
-        // the float chain only: 64 outputs per workgroup, fewer (a thread then
-        // takes fewer beamsets) while there is not a workgroup per CU or two
-        // workgroups do not fit a CU's LDS
-        int n = 64;
-        while(n > 8 && (groups(n) < 256 || chain_lds(n) > (size_t)72 << 10)) n /= 2;
-        lanes   = kIbThreads / n;
+    // the float chain's outputs per workgroup where it runs alone: a thread
+    // per output, fewer outputs (and a thread for some of the beamsets) while
+    // few workgroups fit a CU's LDS or the chip is not filled four times over
+    int nchain = 256;
+    while(nchain > 4 && (groups(nchain) < 1024 || chain_lds(nchain) > (size_t)(nchain > 64 ? 25 : 72) << 10)) nchain /= 2;
+    if(d.nantennas > 2 * kMaskWords) {  // it does
+        lanes   = kIbThreads / nchain;
         batches = 1;
     }
     const int ob = kIbThreads / lanes;
+    nchain = std::max(nchain, ob * batches);  // the workgroups suffice
     const dim3 grid((unsigned)((nout + ob * batches - 1) / (ob * batches)), d.nchans);
-    const size_t lds = chain_lds(ob * batches);
-#define SW_IB_LAUNCH(SM)                                                                                    \
-    if(w4)                                                                                                  \
-        hipLaunchKernelGGL((ib_kernel<S, SM, 4>), grid, dim3(kIbThreads), lds, st, ftpa, raw, out, scale,   \
-                           offset, antw, d.nchans, d.nsamples, d.nantennas, d.tscrunch, d.nbeamsets, lanes, \
-                           batches);                                                                        \
-    else                                                                                                    \
-        hipLaunchKernelGGL((ib_kernel<S, SM, 2>), grid, dim3(kIbThreads), lds, st, ftpa, raw, out, scale,   \
-                           offset, antw, d.nchans, d.nsamples, d.nantennas, d.tscrunch, d.nbeamsets, lanes, \
-                           batches);
+    const size_t lds = chain_lds(nchain);
+    auto log2i = [](int v) { return __builtin_ctz((unsigned)v); };  // of a power of two
+#define SW_IB_LAUNCH_W(SM, W)                                                                                      \
+    hipLaunchKernelGGL((ib_kernel<S, SM, W>), grid, dim3(kIbThreads), lds, st, ftpa, raw, out, scale, offset, antw, \
+                       d.nchans, nout, d.nantennas, d.tscrunch, d.nbeamsets, log2i(lanes), log2i(batches),         \
+                       log2i(nchain))
+#define SW_IB_LAUNCH(SM)       \
+    if(w4)                     \
+        SW_IB_LAUNCH_W(SM, 4); \
+    else                       \
+        SW_IB_LAUNCH_W(SM, 2);
     if(d.nbeamsets <= 1) {
         SW_IB_LAUNCH(1)
     } else if(d.nbeamsets <= 2) {
@@ -498,6 +638,7 @@ int launch_ib(const uint8_t* ftpa, float* raw, int8_t* out, const float* scale,
         SW_IB_LAUNCH(16)
     }
 #undef SW_IB_LAUNCH
+#undef SW_IB_LAUNCH_W
     SW_LAUNCH_CHECK();
     return SW_OK;
 }

@@ -269,6 +269,31 @@ def test_ib_float_chain_splits(sw, orc, dev, stokes, F, T, A, ts, S):
     np.testing.assert_array_equal(out, eout)
 
 
+@pytest.mark.parametrize("binary", [True, False])
+@pytest.mark.parametrize("stokes", ["I", "U", "IQUV"])
+@pytest.mark.parametrize("F,T,A,ts,S", [(8, 4099, 4, 1, 1),      # the small windows' kernel, a partial last wave
+                                        (64, 8200, 4, 4, 5),     # its largest windows
+                                        (64, 4098, 16, 2, 16),
+                                        (64, 2049, 32, 1, 2),
+                                        (64, 2052, 36, 1, 3),    # just past it
+                                        (64, 16388, 8, 4, 2),    # 256 outputs per workgroup of the float chain
+                                        (64, 9216, 32, 3, 2)])   # 128
+def test_ib_small_windows(sw, orc, dev, stokes, F, T, A, ts, S, binary):
+    """Outputs of few rows and antennas at full scale, weights of 0 and 1 and others."""
+    v = _rand_c8((F, T, 2, A), 51 + A + ts, sigma=60.0)
+    v[0, :8 * ts] = -128
+    w = (_rng(A + S).random((S, A)) > 0.3).astype(np.float32)
+    if not binary:
+        w[-1, -1] = 0.37
+    scale, offset = _ib_scales(F, S, A, ts)
+    raw, out = _run_ib(sw, dev, v, w, scale, offset, ts, stokes)
+    pick = [0, F // 2, F - 1]
+    scale, offset = (x.reshape(S, F)[:, pick].reshape(-1).copy() for x in (scale, offset))
+    eraw, eout = orc.ib_beamform(np.ascontiguousarray(v[pick]), ts, scale, offset, w, S, stokes)
+    np.testing.assert_array_equal(raw[:, :, pick], eraw)
+    np.testing.assert_array_equal(out[:, :, pick], eout)
+
+
 @pytest.mark.parametrize("stokes,S", [("I", 1), ("I", 6), ("IQUV", 2)])
 def test_ib_exact_path_overflow_in_some_batches(sw, orc, dev, stokes, S):
     """64 outputs per workgroup in several batches, some of which pass 2^24 in some workgroups."""
