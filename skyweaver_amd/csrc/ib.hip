@@ -444,42 +444,42 @@ ib_small_kernel(const uint8_t* __restrict__ ftpa, float* __restrict__ raw, int8_
 
 // Time-major input (the coherent dedisperser's ring): sample t of column
 // c = p A + a of channel f at ring + ((f 2A + c) ld + w0 + t) 2.  0/1 antenna
-// weights only.  A workgroup owns 64 outputs t' of channel f; its four waves
-// take every fourth antenna, a lane reading its output's ts consecutive
-// samples of both polarisations (64 lanes read 64 ts 2 contiguous bytes) and
-// adding the antenna's integer sums to the beamsets that weight it 1; the
-// waves' sums meet in LDS.  HBM-bound (a workgroup per 256 outputs, one lane
-// summing all antennas, left half of the CUs idle at 16 channels x 2048
-// outputs).  As in ib_kernel the integer totals equal the oracle's float
-// chains while Stokes I is below 2^24; a lane at or above it recomputes its
-// outputs with the float chains in the oracle's order (time, then antenna
-// ascending).
-constexpr int kTmOut = 64, kTmWaves = 4;
+// weights only.  A workgroup owns 256 / WA outputs t' of channel f; with WA = 4
+// its four waves take every fourth antenna, a lane reading its output's ts
+// consecutive samples of both polarisations (64 lanes read 64 ts 2 contiguous
+// bytes) and adding the antenna's integer sums to the beamsets that weight it
+// 1; the waves' sums meet in LDS.  HBM-bound (a workgroup per 256 outputs, one
+// lane summing all antennas, left half of the CUs idle at 16 channels x 2048
+// outputs; ib_beamform_tm has the rule).  As in ib_kernel the integer totals
+// equal the oracle's float chains while Stokes I is below 2^24; a lane at or
+// above it recomputes its outputs with the float chains in the oracle's order
+// (time, then antenna ascending).
 constexpr int kTmMaxAnts = 128;
 
-template <int S, int SMAX, bool V16>
-__global__ void __launch_bounds__(kTmOut * kTmWaves)
+template <int S, int SMAX, bool V16, int WA>
+__global__ void __launch_bounds__(kIbThreads)
 ib_tm_kernel(const uint8_t* __restrict__ ring, long ld, long w0, float* __restrict__ raw,
              int8_t* __restrict__ out, const float* __restrict__ scale, const float* __restrict__ offset,
              const float* __restrict__ antw, int nchans, int nsamples, int nant, int ts, int nbeamsets)
 {
-    constexpr int NV = nstokes(S);
+    constexpr int NV = nstokes(S), OUT = kIbThreads / WA;
     __shared__ uint8_t antb[SMAX][kTmMaxAnts];  // weight (0/1) of antenna a in beamset s
-    __shared__ int red[kTmWaves][4][kTmOut];
-    for(int i = threadIdx.x; i < nbeamsets * nant; i += kTmOut * kTmWaves)
+    __shared__ int red[WA > 1 ? WA : 1][4][OUT];
+    for(int i = threadIdx.x; i < nbeamsets * nant; i += kIbThreads)
         antb[i / nant][i % nant] = antw[i] != 0.0f ? 1 : 0;
     __syncthreads();
     const int f = blockIdx.y;
-    const int lane = threadIdx.x % kTmOut, wave = threadIdx.x / kTmOut;
+    const int lane = threadIdx.x % OUT, wave = threadIdx.x / OUT;
     const int nsamps_out = nsamples / ts;
-    const int tp = blockIdx.x * kTmOut + lane;
+    const int tp = blockIdx.x * OUT + lane;
     const bool active = tp < nsamps_out;
     const uint8_t* base = ring + ((size_t)f * 2 * nant * ld + w0 + (size_t)(active ? tp : 0) * ts) * 2;
     int si[SMAX], sq[SMAX], su[SMAX], sv[SMAX];
 #pragma unroll
     for(int s = 0; s < SMAX; ++s) si[s] = sq[s] = su[s] = sv[s] = 0;
-#pragma unroll 2
-    for(int a = wave; a < nant; a += kTmWaves) {
+    constexpr int U = WA > 1 ? 2 : 4;
+#pragma unroll U
+    for(int a = wave; a < nant; a += WA) {
         const uint8_t* x0 = base + (size_t)a * ld * 2;
         const uint8_t* x1 = base + (size_t)(nant + a) * ld * 2;
         IbSums<S> c;
@@ -498,7 +498,7 @@ ib_tm_kernel(const uint8_t* __restrict__ ring, long ld, long w0, float* __restri
 #pragma unroll
         for(int s = 0; s < SMAX; ++s)
             if(s < nbeamsets && antb[s][a]) {
-                si[s] += c.total();  // at most 2^24 each
+                si[s] += WA > 1 ? c.total() : c.p0 + c.p1;  // at most 32 of 2^24, or 2^30 in all (the rule)
                 if constexpr(S == SW_STOKES_Q || NV == 4) sq[s] += c.q();
                 if constexpr(S == SW_STOKES_U || NV == 4) su[s] += c.uu();
                 if constexpr(S == SW_STOKES_V || NV == 4) sv[s] += c.vv();
@@ -507,19 +507,26 @@ ib_tm_kernel(const uint8_t* __restrict__ ring, long ld, long w0, float* __restri
 #pragma unroll
     for(int s = 0; s < SMAX; ++s) {
         if(s < nbeamsets) {  // uniform
-            if(s) __syncthreads();
-            red[wave][0][lane] = min(si[s], kExact);
-            if constexpr(S != SW_STOKES_I) {
-                red[wave][1][lane] = sq[s];
-                red[wave][2][lane] = su[s];
-                red[wave][3][lane] = sv[s];
+            int t[4] = {si[s], sq[s], su[s], sv[s]};
+            if constexpr(WA > 1) {
+                if(s) __syncthreads();
+                red[wave][0][lane] = min(si[s], kExact);
+                if constexpr(S != SW_STOKES_I) {
+                    red[wave][1][lane] = sq[s];
+                    red[wave][2][lane] = su[s];
+                    red[wave][3][lane] = sv[s];
+                }
+                __syncthreads();
             }
-            __syncthreads();
             if(wave == 0 && active) {
-                int t[4];
+                if constexpr(WA > 1) {
 #pragma unroll
-                for(int k = 0; k < (S == SW_STOKES_I ? 1 : 4); ++k)
-                    t[k] = red[0][k][lane] + red[1][k][lane] + red[2][k][lane] + red[3][k][lane];
+                    for(int k = 0; k < (S == SW_STOKES_I ? 1 : 4); ++k) {
+                        t[k] = 0;
+#pragma unroll
+                        for(int w = 0; w < WA; ++w) t[k] += red[w][k][lane];
+                    }
+                }
                 float power[NV];
                 if constexpr(NV == 4) {
 #pragma unroll
@@ -658,24 +665,41 @@ int ib_beamform_tm(const void* d_ring, long ld, long w0, float* d_raw, void* d_o
     SW_CHECK_ARG((reinterpret_cast<uintptr_t>(d_ring) & 15) == 0 && ld % 8 == 0 && w0 % 8 == 0,
                  "ring must be 16-byte aligned with 8-sample aligned rows");
     const int nout = d.nsamples / d.tscrunch;
-    const dim3 grid((nout + kTmOut - 1) / kTmOut, d.nchans), block(kTmOut * kTmWaves);
     const bool v16 = d.tscrunch % 8 == 0;
+    // 256 outputs per workgroup, no shared antennas, where the rows come from
+    // HBM (more than the 256 MB behind L2 hold) and a workgroup's run of a
+    // column is long: the four waves then read one run of 512 tscrunch bytes
+    // instead of four of 128.  48 antennas x 32 channels x 65536 samples at
+    // tscrunch 32 156 us shared, 93 so; 112 x 64 x 32768 304 and 211; at
+    // tscrunch 8 99 and 85, 199 and 188.  Shared where that leaves fewer
+    // workgroups than CUs or the samples stay on the chip (64 antennas x 64
+    // channels x 16384 samples at tscrunch 16, full Stokes: 60 us shared, 74
+    // not; 48 x 16 x 65536 at 8 40 and 47), and at other tscrunches (48 x 64 x
+    // 40960 at 4: 182 and 241)
+    const long groups = (long)((nout + kIbThreads - 1) / kIbThreads) * d.nchans;
+    const long bytes = 4L * d.nantennas * d.nchans * d.nsamples;
+    const bool share = !(v16 && groups >= 256 && groups <= 2048 && bytes >= 256L << 20 &&
+                         (d.nsamples >= 32768 || bytes > 384L << 20) &&
+                         d.tscrunch <= 16384 / d.nantennas);  // totals of at most 2^30
     auto* in = static_cast<const uint8_t*>(d_ring);
     auto* out = static_cast<int8_t*>(d_out);
-#define SW_IBT_L(S, SM, V)                                                                                          \
-    hipLaunchKernelGGL((ib_tm_kernel<S, SM, V>), grid, block, 0, st, in, ld, w0, d_raw, out, d_scale, d_offset,     \
-                       d_ant_weights, d.nchans, d.nsamples, d.nantennas, d.tscrunch, d.nbeamsets)
-#define SW_IBT(SM)                                                  \
-    if(d.stokes == SW_STOKES_I) {                                   \
-        if(v16)                                                     \
-            SW_IBT_L(SW_STOKES_I, SM, true);                        \
-        else                                                        \
-            SW_IBT_L(SW_STOKES_I, SM, false);                       \
-    } else {                                                        \
-        if(v16)                                                     \
-            SW_IBT_L(SW_STOKES_IQUV, SM, true);                     \
-        else                                                        \
-            SW_IBT_L(SW_STOKES_IQUV, SM, false);                    \
+    const int ob = share ? kIbThreads / 4 : kIbThreads;
+    const dim3 grid((unsigned)((nout + ob - 1) / ob), d.nchans);
+#define SW_IBT_L(S, SM, V, WA)                                                                                       \
+    hipLaunchKernelGGL((ib_tm_kernel<S, SM, V, WA>), grid, dim3(kIbThreads), 0, st, in, ld, w0, d_raw, out, d_scale, \
+                       d_offset, d_ant_weights, d.nchans, d.nsamples, d.nantennas, d.tscrunch, d.nbeamsets)
+#define SW_IBT_V(S, SM)            \
+    if(!share)                     \
+        SW_IBT_L(S, SM, true, 1);  \
+    else if(v16)                   \
+        SW_IBT_L(S, SM, true, 4);  \
+    else                           \
+        SW_IBT_L(S, SM, false, 4);
+#define SW_IBT(SM)                   \
+    if(d.stokes == SW_STOKES_I) {    \
+        SW_IBT_V(SW_STOKES_I, SM)    \
+    } else {                         \
+        SW_IBT_V(SW_STOKES_IQUV, SM) \
     }
     if(d.nbeamsets <= 1) {
         SW_IBT(1)
@@ -685,6 +709,7 @@ int ib_beamform_tm(const void* d_ring, long ld, long w0, float* d_raw, void* d_o
         SW_IBT(16)
     }
 #undef SW_IBT
+#undef SW_IBT_V
 #undef SW_IBT_L
     SW_LAUNCH_CHECK();
     return SW_OK;

@@ -705,3 +705,37 @@ def test_pipeline_ring_beams(sw, orc, dev, stokes, A, ts, S):
     """Beams from the ring with the incoherent beam in its own kernel: full Stokes, and Stokes I
     at antenna counts that the beamformer does not fuse."""
     _check_beams_at_dm0(sw, orc, A, ts, S, stokes)
+
+
+@pytest.mark.parametrize("stokes,F,A,ts,S", [("I", 48, 48, 8, 3), ("IQUV", 64, 48, 32, 2)])
+def test_pipeline_ring_incoherent_beam_large_gulp(sw, orc, dev, stokes, F, A, ts, S):
+    """A gulp past the on-chip cache, whose incoherent beam takes 256 outputs per workgroup, with
+    outputs past 2^24: a few channels against the oracle."""
+    B, H = 16, 128
+    taftp = sw.synth_voltages((H, A, F, 256, 2, 2), seed=91 + ts, sigma=20.0)
+    taftp[1, :, 0, :3 * ts] = -128
+    taftp[-1, :, F - 1, -ts:] = 127
+    antw = np.ones((S, A), np.float32)
+    antw[1:, 5::7] = 0
+    p = sw.BeamformerPipeline(A, F, B, H * 256, ts, [0.0], 1284e6, 13.375e6 * F / 64, stokes=stokes, fft_len=[1024])
+    p.set_weights(sw.synth_weights((F, B, A, 2), seed=5))
+    p.set_beamsets((np.arange(B) % S).astype(np.int32), antw)
+    p.init(A)
+    got = {}
+
+    def grab(key):
+        def f(blk):
+            got[key] = sw.download_block(blk)
+        return f
+    p.set_sinks(ib=grab("ib"), stats=grab("stats"))
+    p(sw.DeviceBuffer.from_host(taftp))
+    p.close()
+    stats = got["stats"].view(np.float32).reshape(F, 2, A, 4)
+    scal = orc.update_scalings(stats[..., 1], antw, S, ts, ts, 24.0)
+    pick = [0, F // 2, F - 1]
+    sc, of = (scal[k].reshape(S, F)[:, pick].reshape(-1).copy() for k in ("ib_scaling", "ib_offsets"))
+    raw, ib = orc.ib_beamform(orc.transpose(np.ascontiguousarray(taftp[:, :, pick]), A), ts, sc, of, antw, S, stokes)
+    assert (raw >= 2 ** 24).any() and (raw < 2 ** 24).any()
+    nv = 4 if stokes == "IQUV" else 1
+    out = got["ib"].view(np.int8).reshape(S, H * 256 // ts, F, nv)[:, :, pick]
+    np.testing.assert_array_equal(out, ib.reshape(out.shape))
