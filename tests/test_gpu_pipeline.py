@@ -739,3 +739,56 @@ def test_pipeline_ring_incoherent_beam_large_gulp(sw, orc, dev, stokes, F, A, ts
     nv = 4 if stokes == "IQUV" else 1
     out = got["ib"].view(np.int8).reshape(S, H * 256 // ts, F, nv)[:, :, pick]
     np.testing.assert_array_equal(out, ib.reshape(out.shape))
+
+
+@pytest.mark.parametrize("stokes,A,ts,S,N,O,graph", [("IQUV", 64, 16, 2, 1024, 0, False),   # no latency
+                                                     ("IQUV", 48, 8, 3, 1024, 62, False),   # windows that wrap
+                                                     ("IQUV", 112, 4, 1, 512, 20, False),
+                                                     ("I", 64, 16, 2, 1024, 62, False),     # beams fused
+                                                     ("I", 16, 8, 1, 2048, 6, True),
+                                                     ("I", 80, 2, 5, 1024, 62, False),
+                                                     ("Q", 32, 8, 2, 1024, 62, False)])     # through FTPA
+def test_pipeline_beams_behind_the_transforms(sw, orc, dev, stokes, A, ts, S, N, O, graph):
+    """A DM so small that its transforms return their int8 input, beside DM 0, which is not
+    transformed: both give the beams of the stream delayed by the latency and half the overlap,
+    over gulps whose output windows go round the ring, against the oracle bit for bit."""
+    F, B, H, G = 3, 40, 8, 5
+    T = H * 256
+    gulps = [sw.synth_voltages((H, A, F, 256, 2, 2), seed=300 + A + g, sigma=28.0) for g in range(G)]
+    weights = sw.synth_weights((F, B, A, 2), seed=5)
+    antw = np.ones((S, A), np.float32)
+    for s in range(1, S):
+        antw[s, s::s + 1] = 0
+    bmap = (np.arange(B) % S).astype(np.int32)
+    dms = [1e-9, 0.0]
+    p = sw.BeamformerPipeline(A, F, B, T, ts, dms, 1284e6, 13.375e6 * F / 64, stokes=stokes, fft_len=[N, N],
+                              overlap=[O, O], async_sinks=graph, graph=graph)
+    p.set_weights(weights)
+    p.set_beamsets(bmap, antw)
+    p.init(A)
+    got = {"cb": [], "ib": [], "stats": []}
+
+    def grab(key):
+        def f(blk):
+            got[key].append((blk.dm_idx, sw.download_block(blk)))
+        return f
+    p.set_sinks(cb=grab("cb"), ib=grab("ib"), stats=grab("stats"))
+    bufs = [sw.DeviceBuffer.from_host(x) for x in gulps]
+    for b in bufs:
+        p(b)
+    p.synchronize()
+    p.close()
+    stats = got["stats"][0][1].view(np.float32).reshape(F, 2, A, 4)
+    scal = orc.update_scalings(stats[..., 1], antw, S, ts, ts, 24.0)
+    delay = O // 2 + (0 if T % (N - O) == 0 else N - O)
+    stream = np.concatenate([np.zeros((F, delay, 2, A, 2), np.int8)] + [orc.transpose(x, A) for x in gulps], 1)
+    for g in range(G):
+        ftpa = np.ascontiguousarray(stream[:, g * T:(g + 1) * T])
+        raw, ib = orc.ib_beamform(ftpa, ts, scal["ib_scaling"], scal["ib_offsets"], antw, S, stokes)
+        cb = orc.cb_beamform(ftpa, weights, ts, scal["cb_scaling"], scal["cb_offsets"], antw, bmap, S, stokes, True)
+        for d in range(2):
+            for key, want in (("ib", ib), ("cb", cb)):
+                idx, blk = got[key][2 * g + d]
+                assert idx == d
+                np.testing.assert_array_equal(blk.view(np.int8).reshape(want.shape), want,
+                                              err_msg=f"{key} gulp {g} DM {dms[d]}")
