@@ -606,6 +606,7 @@ int launch_ib(const uint8_t* ftpa, float* raw, int8_t* out, const float* scale,
     while(lanes < 64 && groups(kIbThreads / lanes) < 1024 && (long)d.tscrunch * chunks >= 8L * lanes) lanes *= 2;
     // 64 outputs per workgroup where enough workgroups are left
     int batches = groups(64) >= 2048 ? 64 * lanes / kIbThreads : 1;
+    if(nout > 1 << 29) batches = lanes;  // 256: the grid's threads stay below 2^32
     // LDS of the float chain for n outputs at a time: rows and weights
     auto chain_lds = [&](int n) {
         return (size_t)n * (d.nantennas / 4 + 1) * 16 + (size_t)d.nbeamsets * d.nantennas * 4;

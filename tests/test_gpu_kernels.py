@@ -314,6 +314,30 @@ def test_ib_exact_path_overflow_in_some_batches(sw, orc, dev, stokes, S):
     np.testing.assert_array_equal(out[:, :, pick], eout)
 
 
+def test_ib_more_outputs_than_2_to_30(sw, dev):
+    """Every output is written where a thread per output and lane would pass the 2^32 threads of a
+    launch; weights of 0 and 1 and others."""
+    A, n, m = 36, (1 << 30) + 197, 600
+    if sw.mem_info()[0] < 170 << 30:
+        pytest.skip("needs 170 GB of device memory")
+    DB = sw.DeviceBuffer
+    v = DB(n * 4 * A)
+    v.fill_bytes(3)
+    raw, out = DB(n * 4), DB(n)
+    scale, offset = DB.from_host(np.float32([100.0])), DB.from_host(np.float32([1000.0]))
+    for w0 in (1.0, 0.5):
+        w = np.ones((1, A), np.float32)
+        w[0, 0] = w0
+        raw.fill_bytes(0)
+        sw.ib_beamform(v, raw, out, scale, offset, DB.from_host(w), sw.dims(1, n, A, 1, 1, "I", 1))
+        sw.synchronize()
+        for o in (0, n // 2, n - m):
+            got = np.empty(m, np.float32)
+            sw.check(sw.lib().sw_memcpy_dtoh(got.ctypes.data, raw.ptr + 4 * o, got.nbytes, 0))
+            sw.synchronize()
+            assert (got == (A - 1 + w0) * 36.0).all(), (w0, o)
+
+
 # --------------------------------------------------------- coherent beamformer
 def _cb_scales(F, S, A, ts, level=32.0):
     # CoherentBeamformerTester.cu:224-242
