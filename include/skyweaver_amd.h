@@ -609,7 +609,8 @@ int sw_pipeline_tile(const sw_pipeline* pipeline, int* cb_waves, int* fft_len, i
  * are fixed, cpp/skyweaver/src/CoherentBeamformer.cu:241-267, and its FFT
  * length is the gulp).  For the workload of cfg on min(tune_chans, nchans)
  * channels of synthetic device input, times the coherent and incoherent
- * beams with 2, 4 and 8 waves per workgroup and, when cfg->fft_len is NULL,
+ * beams with 2, 4 and 8 waves per workgroup (with the corner turn of their
+ * input where only some of the three need one) and, when cfg->fft_len is NULL,
  * runs sw_codedisp_autotune; writes the result as one JSON object (an
  * "entries" item of the tuning table, with the measured times) into json
  * (json_len bytes, NUL-terminated). */

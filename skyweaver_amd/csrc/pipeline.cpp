@@ -1183,8 +1183,8 @@ extern "C" int sw_pipeline_autotune(const sw_pipeline_config* cfg, int tune_chan
     std::vector<int8_t> w((size_t)Fs * c.nbeams * c.nantennas * 2);
     sw_synth_phase_weights(w.data(), w.size() / 2, 0x5EED1000);
     static const int kWaves[] = {2, 4, 8};
-    float ms[3] = {-1, -1, -1};
-    int best = -1;
+    float ms[3] = {-1, -1, -1}, dd[3] = {0, 0, 0};  // beams; dedispersion
+    bool ring[3] = {false, false, false};
     int rc = SW_OK;
     for(int k = 0; k < 3 && rc == SW_OK; ++k) {
         sub.cb_waves = kWaves[k];
@@ -1198,9 +1198,13 @@ extern "C" int sw_pipeline_autotune(const sw_pipeline_config* cfg, int tune_chan
         rc = sw_pipeline_set_weights(p, w.data());
         if(!rc) rc = sw_pipeline_init(p, &h);
         float acc = 0.0f;
+        ring[k] = !rc && beams_on_ring(p);
         for(int it = 0; it < 5 && rc == SW_OK; ++it) {  // two warm-up gulps, three timed
             rc = sw_pipeline_process(p, d_in, gulp, 1);
-            if(rc == SW_OK && it >= 2) acc += p->stage_ms[3] + p->stage_ms[4];
+            if(rc == SW_OK && it >= 2) {
+                acc += p->stage_ms[3] + p->stage_ms[4];
+                dd[k] += p->stage_ms[2] / 3.0f;
+            }
         }
         sw_pipeline_destroy(p);
         if(rc == SW_ERR_UNSUPPORTED) {  // this shape does not fit the workload (LDS): not a candidate
@@ -1208,11 +1212,24 @@ extern "C" int sw_pipeline_autotune(const sw_pipeline_config* cfg, int tune_chan
             continue;
         }
         if(rc) break;
-        ms[k] = acc / 3.0f * (float)c.nchans / (float)Fs;
-        if(best < 0 || ms[k] < ms[best]) best = k;
+        ms[k] = acc / 3.0f;
     }
     (void)hipFree(d_in);
     if(rc) return rc;
+    // where some shapes read the dedisperser's ring and others do not (full
+    // Stokes), those are charged the corner turn to FTPA that the dedispersion
+    // stage then holds (64 antennas x 8 channels x 65536 samples, 16 beams: 50 us
+    // beside 76 to 91 of beams)
+    float on_ring = -1.0f;
+    for(int k = 0; k < 3; ++k)
+        if(ms[k] >= 0 && ring[k] && (on_ring < 0 || dd[k] < on_ring)) on_ring = dd[k];
+    int best = -1;
+    for(int k = 0; k < 3; ++k) {
+        if(ms[k] < 0) continue;
+        if(on_ring >= 0 && !ring[k]) ms[k] += std::max(0.0f, dd[k] - on_ring);
+        ms[k] *= (float)c.nchans / (float)Fs;
+        if(best < 0 || ms[k] < ms[best]) best = k;
+    }
     SW_CHECK_ARG(best >= 0, "autotune: no beamformer workgroup shape runs this workload");
     static const char* stokes[] = {"I", "Q", "U", "V", "IQUV"};
     std::vector<float> dms(c.coherent_dms, c.coherent_dms + c.ndms), fls(fl.begin(), fl.end());

@@ -53,7 +53,8 @@ def main():
              "generated": datetime.datetime.utcnow().strftime("%Y-%m-%d %H:%M UTC"),
              "tool": "python -m skyweaver_amd.tune --chans %d" % args.chans,
              "note": "beams_ms_per_gulp: coherent + incoherent beam device time per gulp for 2, 4 and 8 waves "
-                     "per workgroup (-1: the shape does not fit), scaled from the tuned channels to the workload",
+                     "per workgroup (-1: the shape does not fit), with the corner turn of their input where only "
+                     "some shapes need one, scaled from the tuned channels to the workload",
              "entries": entries}
     os.makedirs(os.path.dirname(os.path.abspath(args.out)), exist_ok=True)
     with open(args.out, "w") as f:

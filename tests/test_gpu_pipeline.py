@@ -792,3 +792,31 @@ def test_pipeline_beams_behind_the_transforms(sw, orc, dev, stokes, A, ts, S, N,
                 assert idx == d
                 np.testing.assert_array_equal(blk.view(np.int8).reshape(want.shape), want,
                                               err_msg=f"{key} gulp {g} DM {dms[d]}")
+
+
+def test_autotune_charges_the_corner_turn(sw, dev):
+    """Full Stokes reads the dedisperser's ring with 4 waves and FTPA, turned in the dedispersion
+    stage, with 2: the tuner's time of the 2-wave shape holds that turn."""
+    A, F, B, T, ts, dms = 64, 8, 16, 65536, 16, [50.0]
+    x = sw.DeviceBuffer.from_host(sw.synth_voltages((T // 256, A, F, 256, 2, 2), seed=7, sigma=16.0))
+    dedisp, beams = {}, {}
+    for waves in (2, 4):
+        p = sw.BeamformerPipeline(A, F, B, T, ts, dms, 1284e6, 13.375e6 * F / 64, stokes="IQUV", fft_len=[1024],
+                                  cb_waves=waves, tuning_file="")
+        p.set_weights(sw.synth_weights((F, B, A, 2), seed=1))
+        p.init(A)
+        t = []
+        for _ in range(7):
+            p(x)
+            t.append(p.stage_times())
+        p.close()
+        dedisp[waves] = np.median([v["dedispersion"] for v in t[2:]])
+        beams[waves] = np.median([v["incoherent_beam"] + v["coherent_beam"] for v in t[2:]])
+    turn = dedisp[2] - dedisp[4]
+    e = sw.pipeline_autotune(A, F, B, T, ts, dms, 1284e6, 13.375e6 * F / 64, stokes="IQUV", fft_len=[1024],
+                             tune_chans=F)
+    times = e["beams_ms_per_gulp"]
+    print(f"dedispersion {dedisp} beams {beams} tuner {times}", flush=True)
+    assert turn > 0.2 * beams[2]
+    assert times["2"] > beams[2] + 0.5 * turn
+    assert times[str(e["cb_waves"])] == min(v for v in times.values() if v >= 0)
