@@ -706,6 +706,8 @@ int ib_beamform_tm(const void* d_ring, long ld, long w0, float* d_raw, void* d_o
         SW_IBT(1)
     } else if(d.nbeamsets <= 4) {
         SW_IBT(4)
+    } else if(d.nbeamsets <= 8) {
+        SW_IBT(8)
     } else {
         SW_IBT(16)
     }

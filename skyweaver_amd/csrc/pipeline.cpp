@@ -658,13 +658,19 @@ int run_gulp(sw_pipeline* p, const void* in, hipEvent_t consumed);
 // Stokes I, or IQUV in 4-wave workgroups, with 0/1 antenna weights (what delay
 // models give): the MFMA beamformer (and the incoherent beam, inside it where
 // supported, else its own kernel) reads the dedisperser's time-major output
-// ring directly, with no corner turn to FTPA (IQUV of 16 channels x 32768
-// samples, 240 beams: 473 us a gulp through FTPA, 441 us from the ring)
+// ring directly, with no corner turn to FTPA.  IQUV, a whole gulp through FTPA
+// and from the ring: 16 channels x 32768 samples x 64 antennas, 240 beams, 473
+// us and 441 at tscrunch 16, 407 and 386 at 4, 806 and 751 at 1; over 16 to 80
+// antennas, tscrunch 1 to 32 and 1 to 16 beamsets the ring is up to 1.7 times
+// as fast and at most 5 % slower, but for 16 channels x 131072 samples x 16
+// antennas at 32 (251 and 288) and for more than eight beamsets at tscrunch 1
+// and 2, whose incoherent beam FTPA does faster (8 channels x 16384 samples x
+// 64 antennas, sixteen: 195 and 215)
 bool beams_on_ring(const sw_pipeline* p)
 {
     const auto& c = p->cfg;
-    bool r = p->use_mfma && (c.stokes == SW_STOKES_I || (c.stokes == SW_STOKES_IQUV && p->cb_waves == 4)) &&
-             2 * c.nantennas <= 256 && c.nsamples % 8 == 0;
+    const bool iquv = c.stokes == SW_STOKES_IQUV && p->cb_waves == 4 && (p->nbeamsets <= 8 || c.tscrunch > 2);
+    bool r = p->use_mfma && (c.stokes == SW_STOKES_I || iquv) && 2 * c.nantennas <= 256 && c.nsamples % 8 == 0;
     for(float w : p->h_antw) r = r && (w == 0.0f || w == 1.0f);
     return r;
 }

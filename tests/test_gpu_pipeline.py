@@ -707,6 +707,13 @@ def test_pipeline_ring_beams(sw, orc, dev, stokes, A, ts, S):
     _check_beams_at_dm0(sw, orc, A, ts, S, stokes)
 
 
+@pytest.mark.parametrize("stokes,A,ts,S", [("IQUV", 32, 4, 7), ("IQUV", 48, 1, 8), ("IQUV", 64, 4, 9),
+                                           ("IQUV", 64, 2, 9), ("IQUV", 16, 1, 16),  # through FTPA
+                                           ("I", 48, 8, 8), ("I", 80, 4, 16)])
+def test_pipeline_ring_many_beamsets(sw, orc, dev, stokes, A, ts, S):
+    _check_beams_at_dm0(sw, orc, A, ts, S, stokes)
+
+
 @pytest.mark.parametrize("stokes,F,A,ts,S", [("I", 48, 48, 8, 3), ("IQUV", 64, 48, 32, 2)])
 def test_pipeline_ring_incoherent_beam_large_gulp(sw, orc, dev, stokes, F, A, ts, S):
     """A gulp past the on-chip cache, whose incoherent beam takes 256 outputs per workgroup, with
