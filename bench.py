@@ -45,7 +45,7 @@ VALU_ADD16_PEAK = 78.6e12   # 16-bit lane adds/s: 256 CUs x 64 lanes x 2 lanes p
 # rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE calibrated on a 1 GiB copy kernel
 # (profiles/hbm_traffic_pipeline_64ant_64ch_65536samp_800beam_dm50.md)
 TRAFFIC_BYTES = {"coherent_beam": 1.314e9, "dedispersion": 2.218e9}
-INT8_LDS_BYTES_PER_CLK = 128   # LDS bytes per clock per CU
+INT8_LDS_BYTES_PER_CLK = 128   # LDS bytes per clock per CU (a rate to compare with: 16-byte reads can run faster)
 NUM_CU, PEAK_CLK_GHZ = 256, 2.4
 
 # incoherent dedispersion workload: 256 channels (4 x 64 over 53.5 MHz at

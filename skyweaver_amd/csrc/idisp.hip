@@ -291,13 +291,17 @@ struct IdArgs {
 // and 16-byte piece c of stored row r' in slot c ^ ((r' / 2) mod 8): any 16
 // consecutive rows then start on distinct banks.  (Rows TS apart put a read
 // on 16 / TS banks: 300 DMs x 404 beams x 64 channels x 3000 samples at
-// tscrunch 4 took 5.4 ms.)
+// tscrunch 4 took 5.4 ms.)  That holds for the rows of one channel: a read
+// takes those of four, each from its own first row, and what these lose to
+// each other is left (24 % of the LDS's active cycles at tscrunch 1, 10 % at
+// 4).
 //
 // What bounds it: the round trip of a quad's row loads, issued after the
-// barrier that frees their buffer, together with the LDS reads of the
-// products, 8 cycles of the CU per 1024 channel sums.  1024 DMs x 512 beams x
-// 256 channels x 4096 samples take 10.2 ms (5.4e13 sums/s), 6.6 ms without the
-// loads, 8.4 ms without the products.  A load therefore costs no address
+// barrier that frees their buffer.  1024 DMs x 512 beams x 256 channels x 4096
+// samples take 9.9 to 10.4 ms by card (5.3e13 to 5.6e13 sums/s), 6.6 ms
+// without the loads, 8.4 ms without the products; of 2.3e7 cycles a CU's LDS
+// is active for 52 %, 5.75 cycles per read of a product (1.4 of them the
+// conflicts above), the matrix cores for 37 %.  A load therefore costs no address
 // arithmetic: per channel a table in LDS, filled once per kMfTabCh channels,
 // holds where its rows begin and end, a buffer resource over them takes the
 // lane's fixed offset and its range check stands for the row tests, and a
