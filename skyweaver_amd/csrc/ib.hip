@@ -138,6 +138,16 @@ __device__ __forceinline__ void lanes_step(int* v, int l)
     }
 }
 
+// The sums of N = 2 or 4 values over groups of N lanes: value l % N in lane l
+template <int N>
+__device__ __forceinline__ int lanes_deal(int (&v)[N], int l)
+{
+    static_assert(N == 2 || N == 4, "neighbours of a quad");
+    if constexpr(N == 4) lanes_step<2, 2, 4>(v, l);
+    lanes_step<1, 1, 2>(v, l);
+    return v[0];
+}
+
 // The sums of N values (a power of two) over groups of `lanes` (8 ... 64)
 // lanes, dealt out: lane l ends with the sums first(l) ... first(l) + N' - 1,
 // N' = max(N / 8, 1), in v.  (A tree per value over all lanes, one lane
@@ -454,9 +464,21 @@ ib_small_kernel(const uint8_t* __restrict__ ftpa, float* __restrict__ raw, int8_
 // equal the oracle's float chains while Stokes I is below 2^24; a lane at or
 // above it recomputes its outputs with the float chains in the oracle's order
 // (time, then antenna ascending).
+//
+// L: 16-byte loads of L neighbouring lanes make up an output's window (ts = 8 L;
+// with L = 1 a lane takes all of a window of 8 n samples); 0: 2-byte loads.
+// With L > 1 a load of the wave covers whole lines, the windows of 64 / L
+// outputs; the L lanes' sums of L such loads are dealt out, so that each lane
+// ends with one output's, and the next antenna's loads are in flight meanwhile.
+// (A lane that took a window of 32 samples by itself left 64 lines half used by
+// each load, and where the columns' pitch is a large power of two these did not
+// stay in the cache: full Stokes of 16 antennas x 16 channels x 131072 samples
+// took 107 us, now 30; 64 x 8 x 16384 22.4, now 13.8; at tscrunch 16 43 and 30,
+// 16.0 and 12.7.  Without the loads ahead the last is 14.4, and with each load
+// summed where it was issued 30.8 at tscrunch 32.)
 constexpr int kTmMaxAnts = 128;
 
-template <int S, int SMAX, bool V16, int WA>
+template <int S, int SMAX, int L, int WA>
 __global__ void __launch_bounds__(kIbThreads)
 ib_tm_kernel(const uint8_t* __restrict__ ring, long ld, long w0, float* __restrict__ raw,
              int8_t* __restrict__ out, const float* __restrict__ scale, const float* __restrict__ offset,
@@ -471,19 +493,58 @@ ib_tm_kernel(const uint8_t* __restrict__ ring, long ld, long w0, float* __restri
     const int f = blockIdx.y;
     const int lane = threadIdx.x % OUT, wave = threadIdx.x / OUT;
     const int nsamps_out = nsamples / ts;
-    const int tp = blockIdx.x * OUT + lane;
+    // the lane's output, and with L > 1 the outputs first + j 64 / L whose
+    // piece l % L it loads
+    constexpr int LL = L > 1 ? L : 1, G = 64 / LL;
+    const int l = threadIdx.x % 64, first = blockIdx.x * OUT + lane - l + l / LL;
+    const int tp = first + l % LL * G;
     const bool active = tp < nsamps_out;
+    const uint8_t* chan = ring + ((size_t)f * 2 * nant * ld + w0) * 2 + l % LL * 16;
     const uint8_t* base = ring + ((size_t)f * 2 * nant * ld + w0 + (size_t)(active ? tp : 0) * ts) * 2;
     int si[SMAX], sq[SMAX], su[SMAX], sv[SMAX];
 #pragma unroll
     for(int s = 0; s < SMAX; ++s) si[s] = sq[s] = su[s] = sv[s] = 0;
-    constexpr int U = WA > 1 ? 2 : 4;
+    uint4 ny[LL], nz[LL];
+    auto fetch = [&](int a) {
+#pragma unroll
+        for(int j = 0; j < L; ++j) {
+            const int o = first + j * G < nsamps_out ? first + j * G : 0;
+            const uint8_t* x = chan + ((size_t)a * ld + (size_t)o * (8 * L)) * 2;
+            ny[j] = *reinterpret_cast<const uint4*>(x);
+            nz[j] = *reinterpret_cast<const uint4*>(x + (size_t)nant * ld * 2);
+        }
+    };
+    if constexpr(L > 1)
+        if(wave < nant) fetch(wave);
+    constexpr int U = L > 1 ? 1 : WA > 1 ? 2 : 4;
 #pragma unroll U
     for(int a = wave; a < nant; a += WA) {
         const uint8_t* x0 = base + (size_t)a * ld * 2;
         const uint8_t* x1 = base + (size_t)(nant + a) * ld * 2;
         IbSums<S> c;
-        if constexpr(V16) {  // ts % 8 == 0: 16-byte aligned runs
+        int i = 0, q = 0, u = 0, v = 0;  // the antenna's sums of the lane's output
+        if constexpr(L > 1) {
+            uint4 y[L], z[L];
+#pragma unroll
+            for(int j = 0; j < L; ++j) y[j] = ny[j], z[j] = nz[j];
+            fetch(a + WA < nant ? a + WA : a);
+            __builtin_amdgcn_sched_barrier(0);
+            int vi[L], vq[L], vu[L], vv[L];
+#pragma unroll
+            for(int j = 0; j < L; ++j) {
+                IbSums<S> b;
+                b.add(y[j].x, z[j].x, ~0u);
+                b.add(y[j].y, z[j].y, ~0u);
+                b.add(y[j].z, z[j].z, ~0u);
+                b.add(y[j].w, z[j].w, ~0u);
+                vi[j] = b.p0 + b.p1;  // at most 2^19
+                vq[j] = b.q(), vu[j] = b.uu(), vv[j] = b.vv();
+            }
+            i = lanes_deal<L>(vi, l);
+            if constexpr(S == SW_STOKES_Q || NV == 4) q = lanes_deal<L>(vq, l);
+            if constexpr(S == SW_STOKES_U || NV == 4) u = lanes_deal<L>(vu, l);
+            if constexpr(S == SW_STOKES_V || NV == 4) v = lanes_deal<L>(vv, l);
+        } else if constexpr(L == 1) {  // ts % 8 == 0: 16-byte aligned runs
             for(int k = 0; k < ts * 2; k += 16) {
                 const uint4 v = *reinterpret_cast<const uint4*>(x0 + k), w = *reinterpret_cast<const uint4*>(x1 + k);
                 c.add(v.x, w.x, ~0u);
@@ -495,13 +556,17 @@ ib_tm_kernel(const uint8_t* __restrict__ ring, long ld, long w0, float* __restri
             for(int k = 0; k < ts; ++k)
                 c.add(*reinterpret_cast<const uint16_t*>(x0 + 2 * k), *reinterpret_cast<const uint16_t*>(x1 + 2 * k), ~0u);
         }
+        if constexpr(L <= 1) {
+            i = WA > 1 ? c.total() : c.p0 + c.p1;
+            q = c.q(), u = c.uu(), v = c.vv();
+        }
 #pragma unroll
         for(int s = 0; s < SMAX; ++s)
             if(s < nbeamsets && antb[s][a]) {
-                si[s] += WA > 1 ? c.total() : c.p0 + c.p1;  // at most 32 of 2^24, or 2^30 in all (the rule)
-                if constexpr(S == SW_STOKES_Q || NV == 4) sq[s] += c.q();
-                if constexpr(S == SW_STOKES_U || NV == 4) su[s] += c.uu();
-                if constexpr(S == SW_STOKES_V || NV == 4) sv[s] += c.vv();
+                si[s] += i;  // at most 32 of 2^24, or 2^30 in all (the rule)
+                if constexpr(S == SW_STOKES_Q || NV == 4) sq[s] += q;
+                if constexpr(S == SW_STOKES_U || NV == 4) su[s] += u;
+                if constexpr(S == SW_STOKES_V || NV == 4) sv[s] += v;
             }
     }
 #pragma unroll
@@ -671,16 +736,20 @@ int ib_beamform_tm(const void* d_ring, long ld, long w0, float* d_raw, void* d_o
     // HBM (more than the 256 MB behind L2 hold) and a workgroup's run of a
     // column is long: the four waves then read one run of 512 tscrunch bytes
     // instead of four of 128.  48 antennas x 32 channels x 65536 samples at
-    // tscrunch 32 156 us shared, 93 so; 112 x 64 x 32768 304 and 211; at
-    // tscrunch 8 99 and 85, 199 and 188.  Shared where that leaves fewer
-    // workgroups than CUs or the samples stay on the chip (64 antennas x 64
-    // channels x 16384 samples at tscrunch 16, full Stokes: 60 us shared, 74
-    // not; 48 x 16 x 65536 at 8 40 and 47), and at other tscrunches (48 x 64 x
-    // 40960 at 4: 182 and 241)
+    // tscrunch 8 99 us shared, 85 so, at 16 97 and 82, at 32 96 and 83; 32 x 32 x
+    // 65536, full Stokes, 67 and 53 at 16, 71 and 50 at 32.  Shared where that
+    // leaves fewer workgroups than CUs or the samples stay on the chip (48 x 16
+    // x 65536 at 8 40 and 47), at other tscrunches (48 x 64 x 40960 at 4: 182
+    // and 241), and for more than four beamsets where lanes share an output and
+    // the columns lie at no large power of two (16 x 64 x 73728, full Stokes,
+    // eight: 113 and 142 at 16, 102 and 121 at 32; 48 x 64 x 40960 136 and 150,
+    // 132 and 146)
     const long groups = (long)((nout + kIbThreads - 1) / kIbThreads) * d.nchans;
     const long bytes = 4L * d.nantennas * d.nchans * d.nsamples;
+    const int dealt = d.tscrunch == 16 ? 2 : d.tscrunch == 32 ? 4 : 1;  // lanes per output
     const bool share = !(v16 && groups >= 256 && groups <= 2048 && bytes >= 256L << 20 &&
                          (d.nsamples >= 32768 || bytes > 384L << 20) &&
+                         (dealt == 1 || d.nbeamsets <= 4 || d.nsamples % 16384 == 0) &&
                          d.tscrunch <= 16384 / d.nantennas);  // totals of at most 2^30
     auto* in = static_cast<const uint8_t*>(d_ring);
     auto* out = static_cast<int8_t*>(d_out);
@@ -689,13 +758,21 @@ int ib_beamform_tm(const void* d_ring, long ld, long w0, float* d_raw, void* d_o
 #define SW_IBT_L(S, SM, V, WA)                                                                                       \
     hipLaunchKernelGGL((ib_tm_kernel<S, SM, V, WA>), grid, dim3(kIbThreads), 0, st, in, ld, w0, d_raw, out, d_scale, \
                        d_offset, d_ant_weights, d.nchans, d.nsamples, d.nantennas, d.tscrunch, d.nbeamsets)
-#define SW_IBT_V(S, SM)            \
-    if(!share)                     \
-        SW_IBT_L(S, SM, true, 1);  \
-    else if(v16)                   \
-        SW_IBT_L(S, SM, true, 4);  \
-    else                           \
-        SW_IBT_L(S, SM, false, 4);
+#define SW_IBT_V(S, SM)              \
+    if(!v16)                         \
+        SW_IBT_L(S, SM, 0, 4);       \
+    else if(dealt == 2 && !share)    \
+        SW_IBT_L(S, SM, 2, 1);       \
+    else if(dealt == 4 && !share)    \
+        SW_IBT_L(S, SM, 4, 1);       \
+    else if(!share)                  \
+        SW_IBT_L(S, SM, 1, 1);       \
+    else if(dealt == 2)              \
+        SW_IBT_L(S, SM, 2, 4);       \
+    else if(dealt == 4)              \
+        SW_IBT_L(S, SM, 4, 4);       \
+    else                             \
+        SW_IBT_L(S, SM, 1, 4);
 #define SW_IBT(SM)                   \
     if(d.stokes == SW_STOKES_I) {    \
         SW_IBT_V(SW_STOKES_I, SM)    \

@@ -662,8 +662,7 @@ int run_gulp(sw_pipeline* p, const void* in, hipEvent_t consumed);
 // and from the ring: 16 channels x 32768 samples x 64 antennas, 240 beams, 473
 // us and 441 at tscrunch 16, 407 and 386 at 4, 806 and 751 at 1; over 16 to 80
 // antennas, tscrunch 1 to 32 and 1 to 16 beamsets the ring is up to 1.7 times
-// as fast and at most 6 % slower, but for 16 channels x 131072 samples x 16
-// antennas at 32 (251 and 288) and for more than eight beamsets at tscrunch 1
+// as fast and at most 5 % slower, but for more than eight beamsets at tscrunch 1
 // and 2, whose incoherent beam FTPA does faster (8 channels x 16384 samples x
 // 64 antennas, sixteen: 195 and 215)
 bool beams_on_ring(const sw_pipeline* p)

@@ -748,6 +748,44 @@ def test_pipeline_ring_incoherent_beam_large_gulp(sw, orc, dev, stokes, F, A, ts
     np.testing.assert_array_equal(out, ib.reshape(out.shape))
 
 
+@pytest.mark.parametrize("stokes,F,A,ts,S,H", [("IQUV", 3, 16, 16, 1, 5), ("IQUV", 3, 48, 32, 3, 3),
+                                              ("IQUV", 2, 80, 32, 6, 9), ("IQUV", 2, 112, 16, 9, 1),
+                                              ("I", 3, 48, 16, 9, 5), ("I", 3, 96, 32, 2, 11), ("I", 3, 16, 8, 1, 7),
+                                              ("IQUV", 64, 32, 16, 5, 136)])
+def test_pipeline_ring_incoherent_beam_dealt_windows(sw, orc, dev, stokes, F, A, ts, S, H):
+    """Windows that two or four lanes share (tscrunch 16 and 32), with a last workgroup that is not
+    full, and one lane's beside them; outputs below 2^24 and past it, against the oracle."""
+    B, T = 16, H * 256
+    taftp = sw.synth_voltages((H, A, F, 256, 2, 2), seed=191 + A + ts, sigma=16.0)
+    taftp[-1, :, 0, -3 * ts - 5:] = -128
+    taftp[0, ::2, F - 1, 1:4 * ts:2, 1] = 127
+    antw = np.ones((S, A), np.float32)
+    for s in range(1, S):
+        antw[s, s::s + 1] = 0
+    p = sw.BeamformerPipeline(A, F, B, T, ts, [0.0], 1284e6, 13.375e6 * F / 64, stokes=stokes, fft_len=[256])
+    p.set_weights(sw.synth_weights((F, B, A, 2), seed=5))
+    p.set_beamsets((np.arange(B) % S).astype(np.int32), antw)
+    p.init(A)
+    got = {}
+
+    def grab(key):
+        def f(blk):
+            got[key] = sw.download_block(blk)
+        return f
+    p.set_sinks(ib=grab("ib"), stats=grab("stats"))
+    p(sw.DeviceBuffer.from_host(taftp))
+    p.close()
+    stats = got["stats"].view(np.float32).reshape(F, 2, A, 4)
+    scal = orc.update_scalings(stats[..., 1], antw, S, ts, ts, 24.0)
+    pick = sorted({0, F // 2, F - 1})
+    sc, of = (scal[k].reshape(S, F)[:, pick].reshape(-1).copy() for k in ("ib_scaling", "ib_offsets"))
+    raw, ib = orc.ib_beamform(orc.transpose(np.ascontiguousarray(taftp[:, :, pick]), A), ts, sc, of, antw, S, stokes)
+    assert (raw >= 2 ** 24).any() == (A * ts >= 256)
+    nv = 4 if stokes == "IQUV" else 1
+    out = got["ib"].view(np.int8).reshape(S, T // ts, F, nv)[:, :, pick]
+    np.testing.assert_array_equal(out, ib.reshape(out.shape))
+
+
 @pytest.mark.parametrize("stokes,A,ts,S,N,O,graph", [("IQUV", 64, 16, 2, 1024, 0, False),   # no latency
                                                      ("IQUV", 48, 8, 3, 1024, 62, False),   # windows that wrap
                                                      ("IQUV", 112, 4, 1, 512, 20, False),
